@@ -299,7 +299,7 @@ def _prepare_decode(case, seed):
     graph = _Graph(ctx, d.step_fused)
     ctx.sync()
     return {"kind": "decode", "ctx": ctx, "decoder": d, "token": token, "position": position, "graph": graph,
-            "out": [out] + _last_caches(s, caches)}
+            "keep": caches, "out": [out] + _last_caches(s, caches)}
 
 
 def _prepare_batch(case, seed):
@@ -320,7 +320,7 @@ def _prepare_batch(case, seed):
     graph = _Graph(ctx, d.step)
     ctx.sync()
     return {"kind": "batch", "ctx": ctx, "decoder": d, "tokens": tokens, "lengths": lengths, "graph": graph,
-            "out": [out] + _last_caches(s, caches)}
+            "keep": caches, "out": [out] + _last_caches(s, caches)}
 
 
 def _batch_table(lens, seed):
@@ -351,7 +351,7 @@ def _prepare_prefill(case, seed):
     setattr(d, "logits" if head else "hidden", _on(ctx, out))
     torch.cuda.synchronize()
     return {"kind": "prefill", "ctx": ctx, "decoder": d, "prompt": _tokens(seed, case["tokens"]),
-            "start": case["start"], "out": out, "caches": _last_caches(s, caches)}
+            "start": case["start"], "keep": caches, "out": out, "caches": _last_caches(s, caches)}
 
 
 def _head_tensors(case, seed):
