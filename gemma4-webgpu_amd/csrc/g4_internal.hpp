@@ -344,6 +344,18 @@ struct OpsSub {
   __host__ __device__ static constexpr uint32_t scale_off(int ntv) { return (uint32_t)ntv * MAIN_T; }
   __host__ __device__ static constexpr uint32_t bytes(int ntv) { return (uint32_t)ntv * (MAIN_T + 512); }
 };
+// Operand blocks of the prefill matmul (k_prefill.hip), one per 64 vectors
+// and super-block of K: main and sums as Ops with 4 vector tiles, but one
+// 2^e per vector and half super-block (equal halves where a whole super-block
+// shares one):
+//   scale [t][half][16] f32: 2^-e of vector 16t + lane%16
+struct PfOps {
+  static constexpr uint32_t MAIN_T = Ops::MAIN_T;
+  static constexpr uint32_t STEP = 4 * 4096;  // 64 k of the four vector tiles
+  static constexpr uint32_t SUMS = 4 * MAIN_T;
+  static constexpr uint32_t SCALE = SUMS + 4 * 1024;
+  static constexpr uint32_t BYTES = SCALE + 4 * 128;
+};
 
 }  // namespace g4d
 

@@ -36,16 +36,11 @@
 //    activations).
 #include <utility>
 
-#include "g4_internal.hpp"
+#include "mm_operand.hpp"
 
 namespace {
 
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x3a __attribute__((ext_vector_type(3), aligned(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));  // native vector: stays in registers
+using namespace g4mm;
 
 constexpr int PNT = 256;   // prep threads
 constexpr int MNT = 256;   // matmul threads (4 waves)
@@ -55,11 +50,6 @@ constexpr int PMAX = 12;   // partials added per pass of the prep loads (24 meas
 using g4d::Ops;
 using g4d::OpsSub;
 using g4d::pad_batch;
-
-__device__ __forceinline__ uint32_t pack_h2(_Float16 a, _Float16 b) {
-  h2 v = {a, b};
-  return __builtin_bit_cast(uint32_t, v);
-}
 
 // ---------------------------------------------------------------------------
 // per-vector prologue: out = x' where x = sum of the nparts partials and
@@ -80,6 +70,7 @@ struct BPrepArgs {
   uint8_t* ops;  // optional: operand blocks [K/256][Ops::bytes(ntv)]
   int ntv;
   const uint16_t* scale;  // mode 2: h = (residual + norm(x)) * f16 scale (NULL: 1)
+  bool prefill;           // ops are the prefill matmul's [B / 64][K/256][PfOps::BYTES]
 };
 
 __device__ __forceinline__ float4 mulw(float4 x, uint2 w, float s) {
@@ -176,12 +167,13 @@ __global__ __launch_bounds__(PNT) void bprep_kernel(BPrepArgs a) {
 #pragma unroll
   for (int p = 0; p < XP; ++p) {
     const int f = 4 * tid + 4 * PNT * p;
-    if (f < K) *(float4*)(a.out + (size_t)v * K + f) = x[p];
+    if (a.out && f < K) *(float4*)(a.out + (size_t)v * K + f) = x[p];
   }
   if (!a.ops) return;
   // operand blocks: wave w of pass p holds super-block 4p + w, lanes 8j .. 8j+7 its sub-block j
-  const uint32_t sblk = Ops::bytes(a.ntv);
-  const uint32_t t = v / 16, c = v % 16;
+  const uint32_t sblk = a.prefill ? g4d::PfOps::BYTES : Ops::bytes(a.ntv);
+  uint8_t* const ops = a.ops + (a.prefill ? (size_t)(v / 64) * BPR * sblk : (size_t)0);
+  const uint32_t t = a.prefill ? v / 16 % 4 : v / 16, c = v % 16;
   const int s = lane >> 3;        // sub-block within the super-block
   const int kk = (lane & 7) * 4;  // first element within the sub-block
   const int q = kk >> 3;          // 8-element group
@@ -207,7 +199,7 @@ __global__ __launch_bounds__(PNT) void bprep_kernel(BPrepArgs a) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) sum += xs[e];
     sum = g4d::sum8(sum) * 0.015625f;  // * 2^-6
-    uint8_t* base = a.ops + (size_t)sb * sblk;
+    uint8_t* base = ops + (size_t)sb * sblk;
     uint8_t* mp = base + t * Ops::MAIN_T + s * 2048 + (c + 16u * q) * 16 + (kk & 7) * 2;
     *(uint2*)mp = make_uint2(pack_h2(hi[0], hi[1]), pack_h2(hi[2], hi[3]));
     *(uint2*)(mp + 1024) = make_uint2(pack_h2(lo[0], lo[1]), pack_h2(lo[2], lo[3]));
@@ -219,7 +211,11 @@ __global__ __launch_bounds__(PNT) void bprep_kernel(BPrepArgs a) {
       *(uint2*)(base + Ops::sums_off(a.ntv) + t * 1024 + (c + 16u * (uint32_t)(s >> 1)) * 16 + (s & 1) * 8) =
           make_uint2(pack_h2(p0, p1), pack_h2(p2, (_Float16)0.f));
     }
-    if (lane == 0) *(float*)(base + Ops::scale_off(a.ntv) + t * 64 + c * 4) = ldexpf(1.0f, -k);
+    if (a.prefill) {  // (both halves of the super-block share the scale)
+      if (lane < 2) *(float*)(base + g4d::PfOps::SCALE + t * 128 + lane * 64 + c * 4) = ldexpf(1.0f, -k);
+    } else if (lane == 0) {
+      *(float*)(base + Ops::scale_off(a.ntv) + t * 64 + c * 4) = ldexpf(1.0f, -k);
+    }
   }
 }
 
@@ -238,11 +234,6 @@ __global__ __launch_bounds__(PNT) void reduce_kernel(const float* part, float* Y
 // matmul
 // ---------------------------------------------------------------------------
 
-template <int QT>
-struct Blk;
-template <> struct Blk<0> { static constexpr int BYTES = 144; };
-template <> struct Blk<1> { static constexpr int BYTES = 210; };
-
 struct MmSeg {
   const uint8_t* W;
   float* Y;  // ksplit == 1: [B][M]; else the partials [ksplit][B][M]
@@ -260,176 +251,6 @@ struct MmArgs {
   uint32_t ksplit, kc;  // K in ksplit chunks of kc super-blocks
   uint8_t* ops_out;     // MODE 1: the product's sub-block-scaled operand blocks (or null)
 };
-
-// Weight registers of one 16-row tile and super-block. A side (row lane%16,
-// k-group q = lane/16): codes and sub-block scales; D side (rows 4q + i): d
-// (Q4_K: d | dmin << 16).
-template <int QT>
-struct WRegs;
-template <> struct WRegs<0> {
-  uint2 qs[4];
-  uint4 hdr;
-  uint32_t dd[4];
-};
-template <> struct WRegs<1> {
-  uint2 ql[4], qh[2];
-  uint4 sc;
-  uint32_t dd[4];
-};
-
-// What load_w leaves in registers: the weights as loaded. Q4_K blocks are
-// 16-byte aligned and load straight into WRegs; a Q6_K block (210 bytes) may
-// sit 2 bytes off a dword, so its pieces are loaded as the aligned dwords
-// around them and shifted into place by w_decode where they are used (a
-// shift at the load would wait for the load there, also for the weights of
-// a block that is only prefetched).
-template <int QT>
-struct WLoad;
-template <> struct WLoad<0> {
-  WRegs<0> r;
-};
-template <> struct WLoad<1> {
-  u32x3a ql[4], qh[2];
-  uint32_t s0, s1, s2, s3, s4;  // the dwords around the 16 scale bytes
-  uint32_t dd[4];
-  uint32_t sh;                  // the block's byte offset within its dword (0 or 2)
-};
-
-template <int BPR>
-__device__ __forceinline__ void load_w(WLoad<0>& ld, const uint8_t* W, uint32_t M, uint32_t rbase, uint32_t kb,
-                                       int l) {
-  WRegs<0>& r = ld.r;
-  constexpr int BY = 144;
-  const int q = l >> 4;
-  const uint32_t ra = min(rbase + (uint32_t)(l & 15), M - 1);
-  const uint8_t* blk = W + ((size_t)ra * BPR + kb) * BY;
-  r.hdr = *(const uint4*)blk;
-#pragma unroll
-  for (int g = 0; g < 4; ++g) r.qs[g] = *(const uint2*)(blk + 16 + 32 * g + 8 * q);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t rd = min(rbase + 4u * q + i, M - 1);
-    r.dd[i] = *(const uint32_t*)(W + ((size_t)rd * BPR + kb) * BY);
-  }
-}
-
-template <int BPR>
-__device__ __forceinline__ void load_w(WLoad<1>& r, const uint8_t* W, uint32_t M, uint32_t rbase, uint32_t kb,
-                                       int l) {
-  constexpr int BY = 210;
-  const int q = l >> 4;
-  const uint32_t ra = min(rbase + (uint32_t)(l & 15), M - 1);
-  const uint8_t* blk = W + ((size_t)ra * BPR + kb) * BY;
-  // every piece sits at a multiple of 8 bytes into the block: one shift for all
-  r.sh = (uint32_t)((uintptr_t)blk & 3);
-  const uint8_t* b4 = blk - r.sh;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    r.ql[2 * h] = *(const u32x3a*)(b4 + 64 * h + 8 * q);
-    r.ql[2 * h + 1] = *(const u32x3a*)(b4 + 64 * h + 32 + 8 * q);
-    r.qh[h] = *(const u32x3a*)(b4 + 128 + 32 * h + 8 * q);
-  }
-  // sc[16] at bytes 192..207: four dwords from the one holding byte 192 and
-  // a fifth (bytes 206..209) that only a block at 2 mod 4 needs
-  const uint32_t* p4 = (const uint32_t*)(b4 + 192);
-  r.s0 = p4[0];
-  r.s1 = p4[1];
-  r.s2 = p4[2];
-  r.s3 = p4[3];
-  r.s4 = *(const uint32_t*)((const uint8_t*)p4 + 12 + 2 * r.sh);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t rd = min(rbase + 4u * q + i, M - 1);
-    r.dd[i] = *(const uint16_t*)(W + ((size_t)rd * BPR + kb) * BY + 208);
-  }
-}
-
-__device__ __forceinline__ const WRegs<0>& w_decode(const WLoad<0>& ld) { return ld.r; }
-__device__ __forceinline__ WRegs<1> w_decode(const WLoad<1>& ld) {
-  WRegs<1> r;
-  const uint32_t sh = ld.sh;
-  auto piece = [&](const u32x3a& w) {
-    return make_uint2(__builtin_amdgcn_alignbyte(w.y, w.x, sh), __builtin_amdgcn_alignbyte(w.z, w.y, sh));
-  };
-#pragma unroll
-  for (int i = 0; i < 4; ++i) r.ql[i] = piece(ld.ql[i]);
-#pragma unroll
-  for (int h = 0; h < 2; ++h) r.qh[h] = piece(ld.qh[h]);
-  r.sc = make_uint4(__builtin_amdgcn_alignbyte(ld.s1, ld.s0, sh), __builtin_amdgcn_alignbyte(ld.s2, ld.s1, sh),
-                    __builtin_amdgcn_alignbyte(ld.s3, ld.s2, sh), __builtin_amdgcn_alignbyte(ld.s4, ld.s3, sh));
-#pragma unroll
-  for (int i = 0; i < 4; ++i) r.dd[i] = ld.dd[i];
-  return r;
-}
-
-// f16 pairs (1024 + b_i, 1024 + b_j) from two bytes of `codes`: v_perm_b32
-// takes selector bytes 0-3 from its second operand and 4-7 from its first.
-__device__ __forceinline__ h2 biased_pair(uint32_t codes, uint32_t sel) {
-  return __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, codes, sel));
-}
-constexpr uint32_t kSel01 = 0x04010400u, kSel23 = 0x04030402u;
-
-__device__ __forceinline__ h8 cat(h2 a, h2 b, h2 c, h2 d) { return h8{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y}; }
-
-// Q4_K 6-bit scale and min of sub-block j (src/gguf.ts:175-182).
-__device__ __forceinline__ void q4k_sc_mn(const uint4& hdr, int j, uint32_t& sc, uint32_t& mn) {
-  const int sh = 8 * (j & 3);
-  if (j < 4) {
-    sc = (hdr.y >> sh) & 63u;
-    mn = (hdr.z >> sh) & 63u;
-  } else {
-    sc = ((hdr.w >> sh) & 15u) | (((hdr.y >> sh) >> 6 & 3u) << 4);
-    mn = ((hdr.w >> sh) >> 4 & 15u) | (((hdr.z >> sh) >> 6 & 3u) << 4);
-  }
-}
-
-// Weight operand of sub-block s: 8 f16 values sc * q of row lane%16, k = 8q .. 8q+7.
-__device__ __forceinline__ h8 a_operand(const WRegs<0>& r, int s, int) {
-  const uint2 raw = r.qs[s >> 1];
-  const uint32_t c0 = (s & 1) ? (raw.x >> 4) & 0x0f0f0f0fu : raw.x & 0x0f0f0f0fu;
-  const uint32_t c1 = (s & 1) ? (raw.y >> 4) & 0x0f0f0f0fu : raw.y & 0x0f0f0f0fu;
-  uint32_t sc, mn;
-  q4k_sc_mn(r.hdr, s, sc, mn);
-  const _Float16 f = (_Float16)(float)sc;
-  const _Float16 fb = (_Float16)(-1024.0f * (float)sc);  // exact: sc <= 63
-  const h2 mul = {f, f}, bias = {fb, fb};
-  // (1024 + c) * sc - 1024 * sc = c * sc, one rounding of an exact value
-  return cat(__builtin_elementwise_fma(biased_pair(c0, kSel01), mul, bias),
-             __builtin_elementwise_fma(biased_pair(c0, kSel23), mul, bias),
-             __builtin_elementwise_fma(biased_pair(c1, kSel01), mul, bias),
-             __builtin_elementwise_fma(biased_pair(c1, kSel23), mul, bias));
-}
-
-// Q6_K sub-block s: half h = s/4, run pair k' = s%4 (src/gguf.ts:344-361);
-// this lane's 8 codes lie in run q/2 of the sub-block.
-__device__ __forceinline__ h8 a_operand(const WRegs<1>& r, int s, int q) {
-  const int h = s >> 2, kp = s & 3;
-  const uint2 ql = r.ql[2 * h + (kp & 1)];
-  const uint2 qh = r.qh[h];
-  const uint32_t lo0 = kp < 2 ? (ql.x & 0x0f0f0f0fu) : ((ql.x >> 4) & 0x0f0f0f0fu);
-  const uint32_t lo1 = kp < 2 ? (ql.y & 0x0f0f0f0fu) : ((ql.y >> 4) & 0x0f0f0f0fu);
-  const uint32_t c0 = lo0 | (((qh.x >> (2 * kp)) & 0x03030303u) << 4);
-  const uint32_t c1 = lo1 | (((qh.y >> (2 * kp)) & 0x03030303u) << 4);
-  const int is = 8 * h + 2 * kp + (q >> 1);
-  const uint32_t wd = (is < 4) ? r.sc.x : (is < 8) ? r.sc.y : (is < 12) ? r.sc.z : r.sc.w;
-  const int scv = (int)(int8_t)((wd >> (8 * (is & 3))) & 0xffu);
-  const _Float16 f = (_Float16)(float)scv;
-  const h2 mul = {f, f};
-  const h2 off = {(_Float16)-1056.0f, (_Float16)-1056.0f};
-  // (1024 + c) - 1056 = c - 32 exactly, then one rounding of (c - 32) * sc
-  return cat((biased_pair(c0, kSel01) + off) * mul, (biased_pair(c0, kSel23) + off) * mul,
-             (biased_pair(c1, kSel01) + off) * mul, (biased_pair(c1, kSel23) + off) * mul);
-}
-
-// Min operand of a Q4_K super-block: slots 8q .. 8q+3 hold the min of
-// sub-block 2q, slots 8q+4 .. +7 that of sub-block 2q+1.
-__device__ __forceinline__ h8 min_operand(const WRegs<0>& r, int q) {
-  uint32_t sc0, m0, sc1, m1;
-  q4k_sc_mn(r.hdr, 2 * q, sc0, m0);
-  q4k_sc_mn(r.hdr, 2 * q + 1, sc1, m1);
-  const _Float16 a = (_Float16)(float)m0, b = (_Float16)(float)m1;
-  return h8{a, a, a, a, b, b, b, b};
-}
 
 // Activations of one super-block: item (v, s) = vector v, sub-block s,
 // item = tid + MNT * u, v = item / 8, s = item % 8; 8 float4 per item.
@@ -832,14 +653,14 @@ __attribute__((amdgpu_waves_per_eu(OPK == 1 && KG == 1 && NKB == 0 ? (NTV <= 2 ?
   if constexpr (NKB > 0) {
     WLoad<QT> wr[NKB];
     src.load(a, kb0, tid);
-    load_w<BPR>(wr[0], rw.W, rw.M, rw.rbase, kb0, l);
-    if constexpr (NKB > 1) load_w<BPR>(wr[1], rw.W, rw.M, rw.rbase, kb0 + KG, l);
+    load_w(wr[0], rw.W, rw.M, (uint32_t)BPR, rw.rbase, kb0, l);
+    if constexpr (NKB > 1) load_w(wr[1], rw.W, rw.M, (uint32_t)BPR, rw.rbase, kb0 + KG, l);
     src.store(lds, a, tid);
     __syncthreads();
     static_for<NKB>([&](auto jc) {
       constexpr int j = decltype(jc)::value;
       if constexpr (j + 1 < NKB) src.load(a, kb0 + KG * (j + 1), tid);  // the next block's operands
-      if constexpr (j + 2 < NKB) load_w<BPR>(wr[j + 2], rw.W, rw.M, rw.rbase, kb0 + KG * (j + 2), l);
+      if constexpr (j + 2 < NKB) load_w(wr[j + 2], rw.W, rw.M, (uint32_t)BPR, rw.rbase, kb0 + KG * (j + 2), l);
       mm_block<QT, NTV, OPK>(w_decode(wr[j]), lds, acc, l, q);
       __syncthreads();  // every wave is done with this block's operands
       if constexpr (j + 1 < NKB) {
@@ -853,14 +674,14 @@ __attribute__((amdgpu_waves_per_eu(OPK == 1 && KG == 1 && NKB == 0 ? (NTV <= 2 ?
     const uint32_t nkb = a.kc / KG;
     WLoad<QT> wa, wb;
     src.load(a, kb0, tid);
-    load_w<BPR>(wa, rw.W, rw.M, rw.rbase, kb0, l);
+    load_w(wa, rw.W, rw.M, (uint32_t)BPR, rw.rbase, kb0, l);
     src.store(lds, a, tid);
     __syncthreads();
     auto step = [&](const WLoad<QT>& cur, WLoad<QT>& nxt, uint32_t j) {
       const bool more = j + 1 < nkb;  // (uniform)
       if (more) {  // the next block is in flight during this one
         src.load(a, kb0 + KG * (j + 1), tid);
-        load_w<BPR>(nxt, rw.W, rw.M, rw.rbase, kb0 + KG * (j + 1), l);
+        load_w(nxt, rw.W, rw.M, (uint32_t)BPR, rw.rbase, kb0 + KG * (j + 1), l);
       }
       mm_block<QT, NTV, OPK>(w_decode(cur), lds, acc, l, q);
       __syncthreads();  // every wave is done with this block's operands
@@ -883,7 +704,7 @@ __attribute__((amdgpu_waves_per_eu(OPK == 1 && KG == 1 && NKB == 0 ? (NTV <= 2 ?
         const bool more = j + 1 < nkb;  // (uniform)
         if (more) {
           src.load(a, kb0 + KG * (j + 1), tid);
-          load_w<BPR>(wb, rw.W, rw.M, rw.rbase, kb0 + KG * (j + 1), l);
+          load_w(wb, rw.W, rw.M, (uint32_t)BPR, rw.rbase, kb0 + KG * (j + 1), l);
         }
         mm_block<QT, NTV, OPK>(wr, lds, acc, l, q);
         __syncthreads();  // every wave is done with this block's operands
@@ -913,7 +734,7 @@ __global__ __launch_bounds__(64) void operand_check_kernel(const uint8_t* W, uin
   const int l = threadIdx.x, q = l >> 4;
   const uint32_t rbase = blockIdx.x * 16u;
   WLoad<QT> wl;
-  load_w<1>(wl, W, nblocks, rbase, 0, l);
+  load_w(wl, W, nblocks, 1u, rbase, 0, l);
   const auto& wr = w_decode(wl);
   const uint32_t row = rbase + (uint32_t)(l & 15);
   if (row >= nblocks) return;
@@ -953,6 +774,16 @@ int bprep_launch(g4_ctx* ctx, uint32_t N, int pro, const BPrepArgs& p) {
   switch (N / 256) {
     case 6: return bprep_bpr<6>(ctx, pro, p);
     case 8: return bprep_bpr<8>(ctx, pro, p);
+    case 16:  // (operands of a head-dim-512 layer's attention output)
+      if (pro) return G4_ERR_UNSUPPORTED;
+      hipLaunchKernelGGL((bprep_kernel<16, 0>), dim3(p.B), dim3(PNT), 0, ctx->stream, p);
+      G4_LAUNCHED(ctx, "batch_prep");
+      return G4_OK;
+    case 1:  // (of a per-layer embedding's gated input)
+      if (pro) return G4_ERR_UNSUPPORTED;
+      hipLaunchKernelGGL((bprep_kernel<1, 0>), dim3(p.B), dim3(PNT), 0, ctx->stream, p);
+      G4_LAUNCHED(ctx, "batch_prep");
+      return G4_OK;
     default: return G4_ERR_UNSUPPORTED;
   }
 }
@@ -1303,6 +1134,24 @@ int g4_batchPrepScale(g4_ctx* ctx, const float* x, uint32_t nparts, const uint16
   const int pro = !w1 ? 0 : (residual ? 2 : 1);
   const BPrepArgs p{x, nparts, batch, w1, residual, w2, h_out, out, eps, (uint8_t*)ops,
                     (int)(pad_batch(batch) / 16), out_scale};
+  return bprep_launch(ctx, N, pro, p);
+}
+
+int g4_prefillPrep(g4_ctx* ctx, const float* x, uint32_t nparts, const uint16_t* w1, const float* residual,
+                   const uint16_t* out_scale, const uint16_t* w2, float* h_out, float* out, void* ops, uint32_t N,
+                   uint32_t vectors, float eps) {
+  G4_ENTER(ctx);
+  G4_REQUIRE(x && nparts >= 1 && (out || ops || h_out), "g4_prefillPrep: null buffer or no parts");
+  G4_REQUIRE(vectors >= 1 && vectors <= 65535, "g4_prefillPrep: %u vectors outside 1..65535", vectors);
+  G4_REQUIRE(w1 || (!residual && !w2), "g4_prefillPrep: residual and w2 need w1");
+  G4_REQUIRE(residual || (!out_scale && !w2), "g4_prefillPrep: out_scale and w2 need the residual form");
+  G4_REQUIRE(N == 1536 || N == 2048 || (!w1 && (N == 4096 || N == 256)),
+             "g4_prefillPrep: N=%u (1536, 2048; without a norm also 256 and 4096)", N);
+  G4_REQUIRE((((uintptr_t)x | (uintptr_t)out | (uintptr_t)ops | (uintptr_t)residual | (uintptr_t)h_out) & 15) == 0,
+             "g4_prefillPrep: buffers must be 16-byte aligned");
+  G4_REQUIRE((((uintptr_t)w1 | (uintptr_t)w2) & 7) == 0, "g4_prefillPrep: norm weights must be 8-byte aligned");
+  const int pro = !w1 ? 0 : (residual ? 2 : 1);
+  const BPrepArgs p{x, nparts, vectors, w1, residual, w2, h_out, out, eps, (uint8_t*)ops, 4, out_scale, true};
   return bprep_launch(ctx, N, pro, p);
 }
 

@@ -1,0 +1,510 @@
+// k_prefill.hip — quantized matmuls for a whole prompt (hundreds to
+// thousands of activation vectors) on the gfx950 matrix cores.
+//
+// The reference prefills one token at a time (src/engine.ts:1923-1938); the
+// ragged step's matmul (k_batch.hip) takes 64 vectors a launch and gives each
+// wave one 16-row tile, so every 64 tokens re-read and re-decode every
+// weight, and a wave reads 4 KB of activation operands from LDS for each
+// 1 KB weight operand. Here one pass takes the prompt:
+//  * unpack_kernel decodes a launch's matrices once into matrix-core operand
+//    order in a scratch buffer (f16 sc * q, the values k_batch.hip's waves
+//    form in registers; the f16 row d's and the Q4_K mins beside them). It
+//    costs one write and one read of 2 B per weight: 4-5 % of a 1900-token
+//    pass; decoding in the matmul instead would repeat per 64 tokens and take
+//    about as many VALU cycles as the products take matrix-core cycles.
+//  * pf_gemm_kernel: a workgroup (4 waves) owns 64 RT rows (RT 16-row tiles
+//    per wave) x 64 vectors. The weight operands go from memory (L2) straight
+//    into registers, 1 KB contiguous per wave load; the activation operands
+//    (f16 hi + lo, twice the bytes) are shared by the waves through a double
+//    LDS buffer of 64 k. With RT = 4 a wave issues 64 MFMAs per 16 KB of LDS
+//    reads, half the LDS rate; with all operands in LDS the reads would take
+//    as long as the products.
+// The arithmetic is that of mmf_kernel: x * 2^e as f16 hi + lo, exact f16
+// sc * q (Q6_K rounds once above 2048), f32 accumulation over a super-block,
+// then d and 2^-e in f32.
+#include <algorithm>
+
+#include "mm_operand.hpp"
+
+namespace {
+
+using namespace g4mm;
+using g4d::PfOps;
+
+constexpr int NT = 256;
+constexpr int kMaxSeg = 4;
+
+struct PfSeg {
+  const uint8_t* W;
+  float* Y;       // [ksplit][T][rows]
+  uint32_t rows;
+  uint32_t rt0;   // first row tile
+};
+
+// Unpacked weights of one launch: rtn row tiles of 16 rows (each segment
+// padded to whole tiles, the padding repeating its last row).
+struct PfWeights {
+  uint8_t* A;   // [rtn][K/32][64 lanes] 16 B: f16 sc * q of row lane % 16, k = 32s + 8 (lane / 16) .. +7
+  uint8_t* Mn;  // Q4_K: [rtn][K/256][64 lanes] 16 B: the min operand
+  float* D;     // [K/256][16 rtn]: d
+  float* DM;    // Q4_K: 64 dmin
+};
+
+struct PfArgs {
+  PfSeg s[kMaxSeg];
+  int n;
+  PfWeights w;
+  uint32_t rtn, K, nsb;  // row tiles; width; super-blocks of the width
+  const uint8_t* ops;    // [T / 64][nsb][PfOps::BYTES]
+  uint32_t T, ntt;       // vectors, tiles of 64
+  uint32_t ksplit, kc;
+  uint32_t groups, items;
+  uint8_t* ops_out;  // gate/up: the product's operands [T / 64][rows / 256][PfOps::BYTES]
+};
+
+template <int QT>
+__global__ __launch_bounds__(NT) void unpack_kernel(PfArgs a) {
+  const int l = threadIdx.x & 63, q = l >> 4, c = l & 15;
+  const uint32_t u = blockIdx.x * 4u + (threadIdx.x >> 6);  // (row tile, super-block)
+  if (u >= a.rtn * a.nsb) return;
+  const uint32_t rt = u / a.nsb, sb = u % a.nsb;
+  const uint8_t* W = a.s[0].W;
+  uint32_t M = a.s[0].rows, rt0 = 0;
+#pragma unroll
+  for (int i = 1; i < kMaxSeg; ++i)
+    if (i < a.n && rt >= a.s[i].rt0) {
+      W = a.s[i].W;
+      M = a.s[i].rows;
+      rt0 = a.s[i].rt0;
+    }
+  const uint32_t rbase = (rt - rt0) * 16u;
+  u32x4* out = (u32x4*)a.w.A + ((size_t)rt * (a.K / 32) + sb * 8u) * 64u + l;
+  if constexpr (QT == 2) {  // f16 rows: only the order changes
+    const u32x4* row = (const u32x4*)(W + ((size_t)min(rbase + (uint32_t)c, M - 1) * a.K + sb * 256u + 8u * q) * 2u);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) out[s * 64] = row[s * 4];
+  } else {
+    WLoad<QT> ld;
+    load_w(ld, W, M, a.nsb, rbase, sb, l);
+    const auto& wr = w_decode(ld);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) out[s * 64] = __builtin_bit_cast(u32x4, a_operand(wr, s, q));
+    float4 d, dm = make_float4(0.f, 0.f, 0.f, 0.f);
+    float* dp = (float*)&d;
+    float* dmp = (float*)&dm;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      dp[i] = g4d::f16_bits_to_f32(wr.dd[i] & 0xffffu);
+      if constexpr (QT == 0) dmp[i] = g4d::f16_bits_to_f32(wr.dd[i] >> 16) * 64.0f;
+    }
+    const size_t di = (size_t)sb * a.rtn * 16u + rt * 16u + 4u * q;
+    if (c == 0) *(float4*)(a.w.D + di) = d;
+    if constexpr (QT == 0) {
+      if (c == 0) *(float4*)(a.w.DM + di) = dm;
+      ((u32x4*)a.w.Mn)[((size_t)rt * a.nsb + sb) * 64u + l] = __builtin_bit_cast(u32x4, min_operand(wr, q));
+    }
+  }
+}
+
+// MODE 0: row group g is row tiles 4 RT g .. +4 RT - 1 of the segments in
+// order, RT consecutive tiles per wave. MODE 1 (gate/up, RT 4): segments 0
+// and 1 have the same rows; a row group is 128 rows of both, a wave's tiles
+// 0-1 the gate's and 2-3 the up's same 32 rows, so gelu(gate) * up needs no
+// exchange; the product leaves as the down projection's operands, one
+// 32-row sub-block per wave, one 2^e per vector and 128 rows (the four
+// waves' maxima meet in LDS). SG: scale groups per super-block of the
+// operands read (2 for that product, 1 otherwise: both halves equal).
+template <int QT, int RT, int MODE, int SG>
+__global__ __launch_bounds__(NT, 2) void pf_gemm_kernel(PfArgs a) {
+  static_assert(MODE == 0 || RT == 4, "gate/up: two tiles of each");
+  __shared__ __align__(16) uint8_t lds[2][PfOps::STEP];
+  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, q = l >> 4, c = l & 15;
+  // Workgroups go to the XCDs in turn (linear id mod 8): XCD x takes the
+  // x-th eighth of the items, in which the vector tiles of one row group and
+  // K chunk are neighbours, so the group's operands come from that XCD's L2.
+  const uint32_t per = (a.items + 7u) / 8u;
+  const uint32_t item = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
+  if (item >= a.items) return;  // (uniform)
+  const uint32_t tt = item % a.ntt, gc = item / a.ntt, chunk = gc % a.ksplit, g = gc / a.ksplit;
+  const uint32_t sb0 = chunk * a.kc;
+  const uint32_t nsub = a.K / 32;
+
+  uint32_t rt[RT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+    if constexpr (MODE == 0) rt[r] = min((g * 4u + w) * RT + r, a.rtn - 1);  // (past the last tile: not stored)
+    else rt[r] = (r >= 2 ? a.s[1].rt0 : 0u) + g * 8u + w * 2u + (r & 1);
+  }
+  const u32x4* Ap[RT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r) Ap[r] = (const u32x4*)a.w.A + ((size_t)rt[r] * nsub + sb0 * 8u) * 64u + l;
+  const uint8_t* Bg = a.ops + ((size_t)tt * a.nsb + sb0) * PfOps::BYTES;
+
+  f4 acc[RT][4], C[RT][4];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[r][t] = f4{0.f, 0.f, 0.f, 0.f};
+
+  u32x4 bs[4];
+  auto stage = [&](const uint8_t* sb, int p) {  // 64 k (step p of the super-block) of every vector tile
+#pragma unroll
+    for (int t = 0; t < 4; ++t) bs[t] = *(const u32x4*)(sb + t * PfOps::MAIN_T + p * 4096 + tid * 16);
+  };
+  auto put = [&](int b) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) *(u32x4*)(lds[b] + t * 4096 + tid * 16) = bs[t];
+  };
+  u32x4 A[RT], An[RT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r) A[r] = Ap[r][0];
+  stage(Bg, 0);
+  put(0);
+  __syncthreads();
+
+  for (uint32_t j = 0; j < a.kc; ++j) {
+    const bool last_sb = j + 1 == a.kc;  // (uniform)
+    const uint8_t* Bsb = Bg + (size_t)j * PfOps::BYTES;
+    const size_t drow = (size_t)(sb0 + j) * a.rtn * 16u;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      // the next 64 k of the vectors are in flight during this step (the last
+      // step of the walk reads its own again)
+      stage(p < 3 ? Bsb : (last_sb ? Bsb : Bsb + PfOps::BYTES), (p + 1) & 3);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int s = 2 * p + h;
+        {
+          const uint32_t nx = (s == 7 && last_sb) ? j * 8u + s : j * 8u + s + 1;
+#pragma unroll
+          for (int r = 0; r < RT; ++r) An[r] = Ap[r][(size_t)nx * 64u];
+        }
+        const uint8_t* base = lds[p & 1] + h * 2048 + l * 16;
+        const bool first = SG == 2 ? (s & 3) == 0 : s == 0;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const h8 bh = *(const h8*)(base + t * 4096), bl = *(const h8*)(base + t * 4096 + 1024);
+#pragma unroll
+          for (int r = 0; r < RT; ++r)
+            C[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, A[r]), bh,
+                                                             first ? f4{0.f, 0.f, 0.f, 0.f} : C[r][t], 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < RT; ++r)
+            C[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, A[r]), bl, C[r][t], 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < RT; ++r) A[r] = An[r];
+        // the super-block's (or its half's) d, min term and 2^-e
+        if (s == 7 || (SG == 2 && s == 3)) {
+          const int hf = SG == 2 ? s >> 2 : 0;
+          float fs[4];
+          h8 bm[QT == 0 ? 4 : 1];
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            fs[t] = *(const float*)(Bsb + PfOps::SCALE + t * 128 + hf * 64 + c * 4);
+            if constexpr (QT == 0) bm[t] = *(const h8*)(Bsb + PfOps::SUMS + t * 1024 + l * 16);
+          }
+#pragma unroll
+          for (int r = 0; r < RT; ++r) {
+            if constexpr (QT == 2) {
+#pragma unroll
+              for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[r][t][i] += fs[t] * C[r][t][i];
+            } else {
+              const f4 d = *(const f4*)(a.w.D + drow + rt[r] * 16u + 4u * q);
+              f4 dm = f4{0.f, 0.f, 0.f, 0.f};
+              h8 am = h8{};
+              if constexpr (QT == 0) {
+                dm = *(const f4*)(a.w.DM + drow + rt[r] * 16u + 4u * q);
+                am = *(const h8*)(a.w.Mn + ((size_t)rt[r] * a.nsb + sb0 + j) * 1024u + l * 16);
+                // slots 8q .. 8q + 7 are sub-blocks 2q and 2q + 1: a half is two lane groups
+                if (SG == 2 && (q >> 1) != hf) am = h8{};
+              }
+#pragma unroll
+              for (int t = 0; t < 4; ++t) {
+                f4 cm = f4{0.f, 0.f, 0.f, 0.f};
+                if constexpr (QT == 0) cm = __builtin_amdgcn_mfma_f32_16x16x32_f16(am, bm[t], cm, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                  if constexpr (QT == 0) acc[r][t][i] += fs[t] * (d[i] * C[r][t][i] - dm[i] * cm[i]);
+                  else acc[r][t][i] += fs[t] * d[i] * C[r][t][i];
+                }
+              }
+            }
+          }
+        }
+      }
+      // one barrier a step: the buffer written here was last read in the
+      // step before, which every wave had left at that step's barrier
+      put((p + 1) & 1);
+      __syncthreads();
+    }
+  }
+
+  // ---- outputs: lane (q, c) holds rows 4q + i of a row tile, vector 64 tt + 16t + c ----
+  if constexpr (MODE == 0) {
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      const uint32_t rr = (g * 4u + w) * RT + r;
+      if (rr >= a.rtn) continue;  // (uniform over the wave)
+      float* Y = a.s[0].Y;
+      uint32_t M = a.s[0].rows, rt0 = 0;
+#pragma unroll
+      for (int i = 1; i < kMaxSeg; ++i)
+        if (i < a.n && rr >= a.s[i].rt0) {
+          Y = a.s[i].Y;
+          M = a.s[i].rows;
+          rt0 = a.s[i].rt0;
+        }
+      const uint32_t row = (rr - rt0) * 16u + 4u * q;
+      Y += (size_t)chunk * a.T * M;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const uint32_t v = tt * 64u + 16u * t + c;
+        if (v >= a.T) continue;
+        float* dst = Y + (size_t)v * M + row;
+        if ((M & 3) == 0 && row + 3 < M) {
+          *(f4*)dst = acc[r][t];
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (row + i < M) dst[i] = acc[r][t][i];
+        }
+      }
+    }
+  } else {
+    f4 y[2][4];
+    float* mx = (float*)lds[0];  // [wave][t][16]: the walk's last barrier ended every read of the buffers
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const bool live = tt * 64u + 16u * t + c < a.T;
+      float m = 0.f;
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          y[r][t][i] = live ? g4d::gelu_tanh(acc[r][t][i]) * acc[r + 2][t][i] : 0.f;
+          m = fmaxf(m, fabsf(y[r][t][i]));
+        }
+      m = g4d::xmax32(g4d::xmax16(m));
+      if (q == 0) mx[(w * 4 + t) * 16 + c] = m;
+    }
+    __syncthreads();
+    const uint32_t hf = g & 1u, s = hf * 4u + w;  // this wave's sub-block of super-block g / 2
+    uint8_t* ob = a.ops_out + ((size_t)tt * (a.s[0].rows / 256u) + (g >> 1)) * PfOps::BYTES;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const float am = fmaxf(fmaxf(mx[t * 16 + c], mx[(4 + t) * 16 + c]),
+                             fmaxf(mx[(8 + t) * 16 + c], mx[(12 + t) * 16 + c]));
+      int ex = 0;
+      (void)frexpf(am, &ex);
+      const int k = am > 0.f ? min(max(14 - ex, -120), 120) : 0;
+      const float sc = ldexpf(1.0f, k);
+      float sum = 0.f;
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        _Float16 hi[4], lo[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float xs = y[r][t][i] * sc;
+          sum += xs;
+          hi[i] = (_Float16)xs;
+          lo[i] = (_Float16)(xs - (float)hi[i]);
+        }
+        // rows 16r + 4q + i of the sub-block: 8-element group 2r + q / 2, half q % 2 of it
+        uint8_t* slot = ob + t * PfOps::MAIN_T + s * 2048u + (c + 16u * (2u * r + (q >> 1))) * 16u + (q & 1) * 8u;
+        *(u32x2*)slot = u32x2{pack_h2(hi[0], hi[1]), pack_h2(hi[2], hi[3])};
+        *(u32x2*)(slot + 1024) = u32x2{pack_h2(lo[0], lo[1]), pack_h2(lo[2], lo[3])};
+      }
+      sum = g4d::xsum32(g4d::xsum16(sum)) * 0.015625f;  // the sub-block's sum * 2^-6
+      if (q == 0) {
+        const _Float16 p0 = (_Float16)sum;
+        const float r1 = sum - (float)p0;
+        const _Float16 p1 = (_Float16)r1;
+        const _Float16 p2 = (_Float16)(r1 - (float)p1);
+        *(u32x2*)(ob + PfOps::SUMS + t * 1024 + (c + 16u * (s >> 1)) * 16u + (s & 1u) * 8u) =
+            u32x2{pack_h2(p0, p1), pack_h2(p2, (_Float16)0.f)};
+        if (w == 0) *(float*)(ob + PfOps::SCALE + t * 128 + hf * 64u + c * 4) = ldexpf(1.0f, -k);
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// host
+// ---------------------------------------------------------------------------
+
+size_t up256(size_t n) { return (n + 255) / 256 * 256; }
+
+struct WLayout {
+  size_t a, mn, d, dm, total;
+};
+WLayout w_layout(int wtype, uint32_t rtn, uint32_t K) {
+  WLayout o{};
+  const size_t nsb = K / 256;
+  o.a = 0;
+  size_t at = (size_t)rtn * (K / 32) * 1024;
+  o.mn = at;
+  if (wtype == 0) at += (size_t)rtn * nsb * 1024;
+  o.d = at;
+  if (wtype != 2) at = up256(at + nsb * rtn * 16 * sizeof(float));
+  o.dm = at;
+  if (wtype == 0) at = up256(at + nsb * rtn * 16 * sizeof(float));
+  o.total = at;
+  return o;
+}
+
+int check_pf(const char* fn, int wtype, const void* const* weights, const uint32_t* rows, int nseg, uint32_t N,
+             const void* ops, uint32_t T, const void* wops, size_t wops_bytes, uint32_t& rtn) {
+  G4_REQUIRE(wtype >= 0 && wtype <= 2, "%s: wtype must be 0 (Q4_K), 1 (Q6_K) or 2 (f16)", fn);
+  G4_REQUIRE(nseg >= 1 && nseg <= kMaxSeg && weights && rows, "%s: 1..%d segments", fn, kMaxSeg);
+  G4_REQUIRE(N >= 256 && N % 256 == 0 && N <= 65536, "%s: N=%u must be a multiple of 256", fn, N);
+  G4_REQUIRE(T >= 1 && T <= 65535, "%s: %u vectors outside 1..65535", fn, T);
+  G4_REQUIRE(ops && ((uintptr_t)ops & 15) == 0 && wops && ((uintptr_t)wops & 15) == 0,
+             "%s: operands must be non-null and 16-byte aligned", fn);
+  rtn = 0;
+  for (int i = 0; i < nseg; ++i) {
+    G4_REQUIRE(weights[i] && rows[i] > 0 && rows[i] <= (1u << 20), "%s: segment %d empty or too tall", fn, i);
+    G4_REQUIRE(((uintptr_t)weights[i] & (wtype == 1 ? 3 : 15)) == 0,
+               "%s: weights misaligned (Q4_K and f16 16 B, Q6_K 4 B)", fn);
+    rtn += ceil_div(rows[i], 16);
+  }
+  G4_REQUIRE(wops_bytes >= w_layout(wtype, rtn, N).total, "%s: weight operand buffer of %zu bytes, %zu needed", fn,
+             wops_bytes, w_layout(wtype, rtn, N).total);
+  return G4_OK;
+}
+
+PfArgs pf_args(int wtype, const void* const* weights, float* const* outputs, const uint32_t* rows, int nseg, uint32_t N,
+               const void* ops, uint32_t T, void* wops, uint32_t rtn) {
+  PfArgs a{};
+  uint32_t rt0 = 0;
+  for (int i = 0; i < nseg; ++i) {
+    a.s[i] = PfSeg{(const uint8_t*)weights[i], outputs ? outputs[i] : nullptr, rows[i], rt0};
+    rt0 += ceil_div(rows[i], 16);
+  }
+  a.n = nseg;
+  const WLayout o = w_layout(wtype, rtn, N);
+  uint8_t* b = (uint8_t*)wops;
+  a.w = PfWeights{b + o.a, b + o.mn, (float*)(b + o.d), (float*)(b + o.dm)};
+  a.rtn = rtn;
+  a.K = N;
+  a.nsb = N / 256;
+  a.ops = (const uint8_t*)ops;
+  a.T = T;
+  a.ntt = ceil_div(T, 64);
+  a.ksplit = 1;
+  a.kc = a.nsb;
+  return a;
+}
+
+int unpack(g4_ctx* ctx, int wtype, const PfArgs& a) {
+  const dim3 grid(ceil_div((uint64_t)a.rtn * a.nsb, 4));
+  if (wtype == 0) hipLaunchKernelGGL(unpack_kernel<0>, grid, dim3(NT), 0, ctx->stream, a);
+  else if (wtype == 1) hipLaunchKernelGGL(unpack_kernel<1>, grid, dim3(NT), 0, ctx->stream, a);
+  else hipLaunchKernelGGL(unpack_kernel<2>, grid, dim3(NT), 0, ctx->stream, a);
+  G4_LAUNCHED(ctx, "prefill_unpack");
+  return G4_OK;
+}
+
+template <int RT, int MODE, int SG>
+int gemm_qt(g4_ctx* ctx, int wtype, PfArgs a, uint32_t groups) {
+  a.groups = groups;
+  a.items = groups * a.ksplit * a.ntt;
+  const dim3 grid(ceil_div(a.items, 8) * 8);
+  if (wtype == 0) hipLaunchKernelGGL((pf_gemm_kernel<0, RT, MODE, SG>), grid, dim3(NT), 0, ctx->stream, a);
+  else if (wtype == 1) hipLaunchKernelGGL((pf_gemm_kernel<1, RT, MODE, SG>), grid, dim3(NT), 0, ctx->stream, a);
+  else hipLaunchKernelGGL((pf_gemm_kernel<2, RT, MODE, SG>), grid, dim3(NT), 0, ctx->stream, a);
+  G4_LAUNCHED(ctx, "prefill_gemm");
+  return G4_OK;
+}
+
+// Row tiles per wave (4 or 2) and K split of a launch: the pair with the
+// least estimated time, in units of one super-block of a RT = 4 workgroup
+// (half as much with RT = 2, a fifth more per tile as the operands read from
+// LDS serve half the rows), over rounds of two workgroups per CU, plus the
+// split's partial sums (their write and the next launch's read).
+struct Plan {
+  int rt;
+  uint32_t ks;
+};
+Plan pick_plan(const g4_ctx* ctx, const PfArgs& a, uint32_t max_split) {
+  const uint32_t slots = 2u * (uint32_t)(ctx->num_cus > 0 ? ctx->num_cus : 256);
+  Plan best{4, 1};
+  double bt = 1e30;
+  for (int rt = 4; rt >= 2; rt -= 2)
+    for (uint32_t ks = 1; ks <= a.nsb && ks <= max_split; ++ks) {
+      if (a.nsb % ks) continue;
+      const uint32_t items = ceil_div(a.rtn, 4u * rt) * a.ntt * ks, rounds = ceil_div(items, slots);
+      const double sb = rt == 4 ? 1.0 : 0.6;
+      // a last round that leaves one workgroup per CU runs it about 1.6 times as fast
+      const uint32_t rest = items - (rounds - 1) * slots;
+      const double eff = rounds - 1 + (rest <= slots / 2 ? 0.62 : 1.0);
+      const double t = eff * (a.nsb / ks * sb + 1.0) + (ks > 1 ? ks * (double)a.T * a.rtn * 16.0 * 1e-7 : 0.0);
+      if (t < bt) {
+        bt = t;
+        best = Plan{rt, ks};
+      }
+    }
+  return best;
+}
+
+}  // namespace
+
+extern "C" {
+
+int g4_prefillWeightBytes(int wtype, uint32_t rows, uint32_t N, size_t* bytes) {
+  G4_REQUIRE(bytes && wtype >= 0 && wtype <= 2 && rows > 0 && rows <= (1u << 22) && N >= 256 && N % 256 == 0 &&
+                 N <= 65536,
+             "g4_prefillWeightBytes: bad shape");
+  *bytes = w_layout(wtype, ceil_div(rows, 16), N).total;
+  return G4_OK;
+}
+
+int g4_prefillOperandBytes(uint32_t N, uint32_t vectors, size_t* bytes) {
+  G4_REQUIRE(bytes && N >= 256 && N % 256 == 0 && N <= 65536 && vectors >= 1 && vectors <= 65535,
+             "g4_prefillOperandBytes: bad shape");
+  *bytes = (size_t)ceil_div(vectors, 64) * (N / 256) * PfOps::BYTES;
+  return G4_OK;
+}
+
+int g4_prefillMatmul(g4_ctx* ctx, int wtype, const void* const* weights, float* const* outputs, const uint32_t* rows,
+                     int nseg, uint32_t N, const void* ops, int product_ops, uint32_t vectors, void* wops,
+                     size_t wops_bytes, uint32_t max_ksplit, uint32_t* ksplit) {
+  G4_ENTER(ctx);
+  uint32_t rtn;
+  int rc = check_pf(__func__, wtype, weights, rows, nseg, N, ops, vectors, wops, wops_bytes, rtn);
+  if (rc) return rc;
+  G4_REQUIRE(outputs && ksplit && max_ksplit >= 1, "g4_prefillMatmul: null outputs, null ksplit or max_ksplit 0");
+  for (int i = 0; i < nseg; ++i)
+    G4_REQUIRE(outputs[i] && ((uintptr_t)outputs[i] & 15) == 0, "g4_prefillMatmul: output %d null or misaligned", i);
+  PfArgs a = pf_args(wtype, weights, outputs, rows, nseg, N, ops, vectors, wops, rtn);
+  rc = unpack(ctx, wtype, a);
+  if (rc) return rc;
+  const Plan p = pick_plan(ctx, a, max_ksplit);
+  a.ksplit = p.ks;
+  a.kc = a.nsb / p.ks;
+  *ksplit = p.ks;
+  const uint32_t groups = ceil_div(rtn, 4u * (uint32_t)p.rt);
+  if (product_ops) return p.rt == 4 ? gemm_qt<4, 0, 2>(ctx, wtype, a, groups) : gemm_qt<2, 0, 2>(ctx, wtype, a, groups);
+  return p.rt == 4 ? gemm_qt<4, 0, 1>(ctx, wtype, a, groups) : gemm_qt<2, 0, 1>(ctx, wtype, a, groups);
+}
+
+int g4_prefillGateUp(g4_ctx* ctx, int wtype, const void* w_gate, const void* w_up, const void* ops, void* product_ops,
+                     uint32_t M, uint32_t N, uint32_t vectors, void* wops, size_t wops_bytes) {
+  G4_ENTER(ctx);
+  const void* weights[2] = {w_gate, w_up};
+  const uint32_t rows[2] = {M, M};
+  uint32_t rtn;
+  int rc = check_pf(__func__, wtype, weights, rows, 2, N, ops, vectors, wops, wops_bytes, rtn);
+  if (rc) return rc;
+  G4_REQUIRE(M % 256 == 0, "g4_prefillGateUp: M=%u must be a multiple of 256", M);
+  G4_REQUIRE(product_ops && ((uintptr_t)product_ops & 15) == 0, "g4_prefillGateUp: product operands null or misaligned");
+  PfArgs a = pf_args(wtype, weights, nullptr, rows, 2, N, ops, vectors, wops, rtn);
+  a.ops_out = (uint8_t*)product_ops;
+  rc = unpack(ctx, wtype, a);
+  if (rc) return rc;
+  return gemm_qt<4, 1, 1>(ctx, wtype, a, M / 128);
+}
+
+}  // extern "C"

@@ -212,6 +212,12 @@ SIGNATURES = {
                                            ctypes.POINTER(_U32), _I, _U32, _U32, _U32, _F,
                                            ctypes.POINTER(_U32)]),
     "g4_batchOperandBytes": (_I, [_U32, _U32, ctypes.POINTER(_SZ)]),
+    "g4_prefillWeightBytes": (_I, [_I, _U32, _U32, ctypes.POINTER(_SZ)]),
+    "g4_prefillOperandBytes": (_I, [_U32, _U32, ctypes.POINTER(_SZ)]),
+    "g4_prefillPrep": (_I, [_P, _P, _U32, _P, _P, _P, _P, _P, _P, _P, _U32, _U32, _F]),
+    "g4_prefillMatmul": (_I, [_P, _I, ctypes.POINTER(_P), ctypes.POINTER(_P), ctypes.POINTER(_U32), _I, _U32, _P, _I,
+                              _U32, _P, _SZ, _U32, ctypes.POINTER(_U32)]),
+    "g4_prefillGateUp": (_I, [_P, _I, _P, _P, _P, _P, _U32, _U32, _U32, _P, _SZ]),
     "g4_batchPrep": (_I, [_P, _P, _U32, _P, _P, _P, _P, _P, _P, _U32, _U32, _F]),
     "g4_gateUpGeluBatch": (_I, [_P, _P, _P, _P, _P, _P, MatmulParams, _U32]),
     "g4_batchSubOperandBytes": (_I, [_U32, _U32, ctypes.POINTER(_SZ)]),

@@ -57,6 +57,9 @@ Q6K_BYTES = 210
 BLOCK_BYTES = {"q4k": Q4K_BYTES, "q6k": Q6K_BYTES}
 # the layer matrices and their default formats (Q4_K, the down projection Q6_K)
 MATRICES = ("wq", "wk", "wv", "wo", "wgate", "wup", "wdown")
+# rows of a long prompt's pass through the layers (BatchDecoder.prefill): its
+# buffers take about 0.2 MB a row; past this the matmuls gain nothing
+WIDE_ROWS = 2048
 DEFAULT_TYPES = {"wq": "q4k", "wk": "q4k", "wv": "q4k", "wo": "q4k", "wgate": "q4k", "wup": "q4k", "wdown": "q6k"}
 
 
@@ -926,6 +929,11 @@ class BatchDecoder(_SyntheticModel):
         self.block_ws = ctx.zeros(max(ctx.paged_block_workspace_bytes(p, self.ks_h) for p in self.pro_params),
                                   np.uint8)
         self.rope_cs = self._rope_tables(self.max_seq)
+        # prompts longer than one chunk of B rows go through the layers this
+        # many rows at a time (0: B at a time)
+        self.wide_rows = min(max(B, WIDE_ROWS // B * B), -(-self.max_seq // B) * B) if self._wide_prefill() else 0
+        if self.wide_rows:
+            self._build_wide()
         ctx.fill_normal_f32(self.hidden, B * s.hidden, self._seed(), 0.0, 1.0)
         ctx.sync()
 
@@ -1083,20 +1091,26 @@ class BatchDecoder(_SyntheticModel):
                         H, B, s.eps, ops=self.xops)
         if probe:
             probe("prep", s.n_layers, 0)
-        if self.lm_head is not None:
-            if self.lm_type == "f16":
-                c.matmulF16(self.xn, self.lm_head, self.logits, s.vocab, H, B)
-                c.logitSoftcap(self.logits, B * s.vocab, s.softcap)
-            else:
-                c.matmulSegmentsBatchPartial(self.lm_type, self.xn, [self.lm_head], [self.logits], [s.vocab], H, B,
-                                             1, ops=self.xops, softcap=s.softcap)
-            if sample == "argmax":
-                c.argmaxBatch(self.logits, self.tokens, s.vocab, B)
-            else:
-                c.topk256Batch(self.logits, self.topk, s.vocab, B)
-            if probe:
-                probe("head", s.n_layers, 0)
+        self._head(sample)
+        if probe and self.lm_head is not None:
+            probe("head", s.n_layers, 0)
         self.lens_host = self.lens_host + 1
+
+    def _head(self, sample: str) -> None:
+        """LM head + softcap over the normalised rows in xn / xops, then the sample of every row."""
+        c, s, B, H = self.ctx, self.s, self.B, self.s.hidden
+        if self.lm_head is None:
+            return
+        if self.lm_type == "f16":
+            c.matmulF16(self.xn, self.lm_head, self.logits, s.vocab, H, B)
+            c.logitSoftcap(self.logits, B * s.vocab, s.softcap)
+        else:
+            c.matmulSegmentsBatchPartial(self.lm_type, self.xn, [self.lm_head], [self.logits], [s.vocab], H, B, 1,
+                                         ops=self.xops, softcap=s.softcap)
+        if sample == "argmax":
+            c.argmaxBatch(self.logits, self.tokens, s.vocab, B)
+        else:
+            c.topk256Batch(self.logits, self.topk, s.vocab, B)
 
     def _ffn_handoff(self, il: int) -> bool:
         """Layer il's gate/up launch hands its product to the down projection
@@ -1125,7 +1139,10 @@ class BatchDecoder(_SyntheticModel):
         launch reads them, so the chunk is causal). The reference runs one
         full forward per prompt token instead (src/engine.ts:1923-1938) and
         samples from the last one (src/engine.ts:2014-2017); as there, only
-        the last chunk runs the LM head. A short last
+        the last chunk runs the LM head. A prompt of more than one chunk
+        takes the layers up to `wide_rows` rows at a time instead, through the
+        prefill matmuls (each weight read and unpacked once per pass), and
+        leaves the same rows as its last chunk would. A short last
         chunk repeats its last token and position in the spare rows
         (identical rows, identical writes). Returns the row of the final
         chunk that holds the prompt's last token: its logits and `tokens`
@@ -1140,6 +1157,9 @@ class BatchDecoder(_SyntheticModel):
         nch = -(-T // B)
         n = T - (nch - 1) * B
         pad = nch * B - T
+        if nch > 1 and self.wide_rows and probe is None:
+            self._prefill_wide(toks, start, pad, sample)
+            return n - 1
         # every chunk's tokens and lengths (before the step appends each row)
         # uploaded once; the chunks then run back to back on the stream
         ctok = np.concatenate([toks, np.repeat(toks[-1], pad)]).astype(np.uint32)
@@ -1154,6 +1174,122 @@ class BatchDecoder(_SyntheticModel):
         dtok.free()
         dpos.free()
         return n - 1
+
+    def _wide_prefill(self) -> bool:
+        """Whether prompts may take the layers many rows at a time: one prompt
+        per decoder, longer than a chunk, and widths the prefill kernels take."""
+        s = self.s
+        return (self.shared_pages and self.embedding is not None and self.max_seq > self.B
+                and s.hidden in (1536, 2048) and s.ple_dim in (0, 256)
+                and all(s.q_dim_of(il) in (1536, 2048, 4096) and s.ffn_of(il) % 256 == 0
+                        and L.qt["wgate"] == L.qt["wup"] for il, L in enumerate(self.layers)))
+
+    def _build_wide(self) -> None:
+        c, s, R, f32 = self.ctx, self.s, self.wide_rows, np.float32
+        H = s.hidden
+        ob = c.prefill_operand_bytes
+        w = self.wide = {
+            "hidden": c.empty(R * H, f32), "hidden2": c.empty(R * H, f32), "xops": c.empty(ob(H, R), np.uint8),
+            "q": c.empty(R * s.q_dim, f32), "k": c.empty(R * s.kv_dim, f32), "v": c.empty(R * s.kv_dim, f32),
+            "attn": c.empty(R * s.q_dim, f32), "aops": c.empty(ob(s.q_dim, R), np.uint8),
+            "fops": c.empty(ob(s.max_ffn, R), np.uint8)}
+        # split-K partial sums of o and down: four chunks of a full pass, more of a short one
+        self.wide_parts = 4 * max(R, 512) * H
+        w["parts"] = c.empty(self.wide_parts, f32)
+        need = 0
+        for il, L in enumerate(self.layers):
+            Q, KV, I = s.q_dim_of(il), s.kv_dim_of(il), s.ffn_of(il)
+            qkv = [("wq", Q)] + ([("wk", KV), ("wv", KV)] if s.is_producer(il) else [])
+            for ms, rows, n in [([m for m, _ in qkv], [r for _, r in qkv], H), (["wo"], [H], Q),
+                                (["wgate", "wup"], [I, I], H), (["wdown"], [H], I)]:
+                need = max([need] + [c.prefill_weight_bytes(L.qt[m], rows, n) for m in ms])
+        w["wops"] = c.empty(need, np.uint8)
+        if s.ple_dim:
+            LD = s.n_layers * s.ple_dim
+            w.update(hidden3=c.empty(R * H, f32), ple_projected=c.empty(R * LD, f32), ple_inputs=c.empty(R * LD, f32),
+                     ple_gated=c.empty(R * s.ple_dim, f32), ple_out=c.empty(R * H, f32))
+
+    def _prefill_wide(self, toks, start: int, pad: int, sample: str) -> None:
+        """The prompt (its last token repeated `pad` times to whole chunks of
+        B rows) up to wide_rows rows a pass, then the head over the last B."""
+        c, s, B, H, w = self.ctx, self.s, self.B, self.s.hidden, self.wide
+        T = int(toks.size)
+        ctok = np.concatenate([toks, np.repeat(toks[-1], pad)]).astype(np.uint32)
+        clen = (np.concatenate([np.arange(T), np.repeat(T - 1, pad)]) + start + 1).astype(np.uint32)
+        dtok, dlen = c.from_numpy(ctok), c.from_numpy(clen)
+        n = 0
+        for at in range(0, T + pad, self.wide_rows):
+            n = min(self.wide_rows, T + pad - at)
+            self._wide_pass(dtok.offset(4 * at), dlen.offset(4 * at), n)
+        # the last B rows are what the last chunk of B rows leaves: the residual
+        # stream, its tokens and lengths, then the head and the sample
+        c.copy(self.hidden, w["hidden"].offset(4 * H * (n - B)), 4 * H * B)
+        c.copy(self.tokens, dtok.offset(4 * (T + pad - B)), 4 * B)
+        c.copy(self.seq_lens, dlen.offset(4 * (T + pad - B)), 4 * B)
+        self.lens_host = clen[-B:].copy()
+        c.batchPrep(self.hidden, 1, self.final_norm, None, None, None, self.xn, H, B, s.eps, ops=self.xops)
+        self._head(sample)
+        c.sync()
+        dtok.free()
+        dlen.free()
+
+    def _wide_pass(self, tokens, lens, n: int) -> None:
+        """n rows (a multiple of B) of one prompt through every layer; the
+        residual stream after the last layer is left in wide["hidden"]."""
+        c, s, B, w = self.ctx, self.s, self.B, self.wide
+        H, wops = s.hidden, w["wops"]
+        c.embeddingLookupBatch(self.embedding, s.vocab, w["hidden"], H, tokens, n)
+        if s.ple_dim:
+            LD = s.n_layers * s.ple_dim
+            c.matmulF16(w["hidden"], self.ple_model_proj, w["ple_projected"], LD, H, n)
+            c.pleStage1Fuse(w["ple_projected"], self.ple_proj_norm, self.ple_table, s.vocab, w["ple_inputs"],
+                            s.n_layers, s.ple_dim, s.eps, tokens_dev=tokens, count=n)
+        max_ks = max(1, self.wide_parts // (n * H))
+        nd = 0
+        for il in range(s.n_layers + 1):
+            L = self.layers[il] if il < s.n_layers else None
+            norm, ops = (L.attn_norm, w["xops"]) if L else (None, None)
+            if il == 0:
+                c.prefillPrep(w["hidden"], 1, norm, None, None, None, None, None, H, n, s.eps, ops=ops)
+            elif s.ple_dim:
+                prev = self.layers[il - 1]
+                c.prefillPrep(w["ple_out"], 1, prev.ple_post_norm, w["hidden3"], prev.ple_scale, norm, w["hidden"],
+                              None, H, n, s.eps, ops=ops)
+            else:
+                prev = self.layers[il - 1]
+                c.prefillPrep(w["parts"], nd, prev.post_ffn_norm, w["hidden2"], None, norm, w["hidden"], None, H, n,
+                              s.eps, ops=ops)
+            if L is None:
+                return
+            Q, KV, I = s.q_dim_of(il), s.kv_dim_of(il), s.ffn_of(il)
+            prod = s.is_producer(il)
+            outs = [w["q"], w["k"], w["v"]] if prod else [w["q"]]
+            for qt, ws, go, gr in qkv_groups(L, outs, [Q, KV, KV] if prod else [Q]):
+                c.prefillMatmul(qt, ws, go, gr, H, w["xops"], n, wops)
+            rope = self.rope_cs[s.is_global(il)]
+            for r in range(0, n, B):  # every row of the pass is appended before any is read
+                c.pagedAttnPrologue(w["q"].offset(4 * Q * r), w["k"].offset(4 * KV * r) if prod else None,
+                                    w["v"].offset(4 * KV * r) if prod else None, 1, L.q_norm, L.k_norm,
+                                    self.rope_freqs, w["q"].offset(4 * Q * r), L.k_cache if prod else None,
+                                    L.v_cache if prod else None, self.page_table, lens.offset(4 * r),
+                                    self.pro_params[il], rope, self.rope_rows)
+            for r in range(0, n, B):
+                c.pagedAttnDecode(w["q"].offset(4 * Q * r), L.k_cache, L.v_cache, self.page_table, lens.offset(4 * r),
+                                  w["attn"].offset(4 * Q * r), self.attn_params[il], self.attn_ws)
+            c.prefillPrep(w["attn"], 1, None, None, None, None, None, None, Q, n, s.eps, ops=w["aops"])
+            no = c.prefillMatmul(L.qt["wo"], [L.wo], [w["parts"]], [H], Q, w["aops"], n, wops, max_ks)
+            c.prefillPrep(w["parts"], no, L.post_attn_norm, w["hidden"], None, L.pre_ffn_norm, w["hidden2"], None, H,
+                          n, s.eps, ops=w["xops"])
+            c.prefillGateUp(L.qt["wgate"], L.wgate, L.wup, w["xops"], w["fops"], I, H, n, wops)
+            nd = c.prefillMatmul(L.qt["wdown"], [L.wdown], [w["parts"]], [H], I, w["fops"], n, wops, max_ks,
+                                 product_ops=True)
+            if s.ple_dim:
+                D = s.ple_dim
+                c.prefillPrep(w["parts"], nd, L.post_ffn_norm, w["hidden2"], None, None, w["hidden3"], None, H, n,
+                              s.eps)
+                c.pleGate(w["hidden3"], None, None, None, L.ple_gate, w["ple_inputs"], s.n_layers * D, il * D,
+                          w["ple_gated"], D, H, s.eps, batch=n)
+                c.matmulF16(w["ple_gated"], L.ple_proj, w["ple_out"], H, D, n)
 
     def capture(self, sample: str = "argmax"):
         """The step as a HIP graph; each replay appends one token per sequence."""

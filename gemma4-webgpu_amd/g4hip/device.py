@@ -92,6 +92,9 @@ def _p(b: Ptr) -> ctypes.c_void_p:
     return ctypes.c_void_p(int(b))
 
 
+PREFILL_TYPES = {"q4k": 0, "q6k": 1, "f16": 2}
+
+
 class Context:
     """One HIP device + stream. All kernels enqueue on `stream`."""
 
@@ -322,6 +325,45 @@ class Context:
         """batchPrep with h = (residual + norm(x)*w1) * out_scale[0]; w2 None: out = h."""
         check(lib().g4_batchPrepScale(self.h, _p(x_parts), nparts, _p(w1), _p(residual), _p(out_scale), _p(w2),
                                       _p(h_out), _p(out), _p(ops), N, batch, eps))
+
+    # ---- a whole prompt in one pass ----
+    @staticmethod
+    def prefill_weight_bytes(wtype: str, rows, N: int) -> int:
+        """Scratch for the unpacked weights of matrices of `rows` rows."""
+        n = ctypes.c_size_t()
+        check(lib().g4_prefillWeightBytes(PREFILL_TYPES[wtype], sum(-(-r // 16) * 16 for r in rows), N,
+                                          ctypes.byref(n)))
+        return int(n.value)
+
+    @staticmethod
+    def prefill_operand_bytes(N: int, vectors: int) -> int:
+        n = ctypes.c_size_t()
+        check(lib().g4_prefillOperandBytes(N, vectors, ctypes.byref(n)))
+        return int(n.value)
+
+    def prefillPrep(self, x_parts: Ptr, nparts: int, w1: Ptr, residual: Ptr, out_scale: Ptr, w2: Ptr, h_out: Ptr,
+                    out: Ptr, N: int, vectors: int, eps: float = 1e-6, ops: Ptr = None) -> None:
+        """batchPrepScale over any number of vectors; `ops` receives the prefill matmul's operand blocks."""
+        check(lib().g4_prefillPrep(self.h, _p(x_parts), nparts, _p(w1), _p(residual), _p(out_scale), _p(w2),
+                                   _p(h_out), _p(out), _p(ops), N, vectors, eps))
+
+    def prefillMatmul(self, wtype: str, weights, outputs, rows, N: int, ops: Ptr, vectors: int, wops: Buffer,
+                      max_ksplit: int = 1, product_ops: bool = False) -> int:
+        """outputs[i] [ksplit][vectors][rows[i]] = each weight times the vectors behind `ops`; returns ksplit."""
+        n = len(weights)
+        W = (ctypes.c_void_p * n)(*[_p(w).value for w in weights])
+        Y = (ctypes.c_void_p * n)(*[_p(y).value for y in outputs])
+        R = (ctypes.c_uint32 * n)(*rows)
+        ks = ctypes.c_uint32(0)
+        check(lib().g4_prefillMatmul(self.h, PREFILL_TYPES[wtype], W, Y, R, n, N, _p(ops), int(product_ops), vectors,
+                                     _p(wops), wops.nbytes, max_ksplit, ctypes.byref(ks)))
+        return int(ks.value)
+
+    def prefillGateUp(self, wtype: str, w_gate: Ptr, w_up: Ptr, ops: Ptr, product_ops: Ptr, M: int, N: int,
+                      vectors: int, wops: Buffer) -> None:
+        """gelu(gate) * up of the vectors behind `ops`, as the down projection's operand blocks."""
+        check(lib().g4_prefillGateUp(self.h, PREFILL_TYPES[wtype], _p(w_gate), _p(w_up), _p(ops), _p(product_ops),
+                                     M, N, vectors, _p(wops), wops.nbytes))
 
     # ---- per-layer embeddings (shaders/ple_*.wgsl) ----
     def pleStage1Fuse(self, projected: Ptr, norm_w: Ptr, table: Ptr, table_rows: int, ple_inputs: Ptr,

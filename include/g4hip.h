@@ -696,6 +696,35 @@ int g4_gateUpGeluBatchOps(g4_ctx* ctx, const float* x, const void* ops, const vo
 int g4_matmulSubBatchPartial(g4_ctx* ctx, const void* ops, const void* weight, float* out, uint32_t M,
                              uint32_t K, uint32_t batch, uint32_t max_ksplit, uint32_t* ksplit);
 
+/* A whole prompt in one pass (src/engine.ts:1896-1900, 1923-1938 run one
+ * forward per prompt token): matmuls over up to 65535 activation vectors.
+ * g4_prefillPrep forms each vector's prologue as g4_batchPrepScale does
+ * (w1 NULL: x; residual NULL: x * w1 / rms(x); else h = (residual + norm(x))
+ * * out_scale[0], then * w2 / rms(h) unless w2 is NULL), writing any of
+ * h_out, out [vectors][N] and `ops`, the operand blocks of the matmuls below
+ * (g4_prefillOperandBytes(N, vectors) bytes). N 1536 or 2048; without a norm
+ * also 256 and 4096. */
+int g4_prefillWeightBytes(int wtype, uint32_t rows, uint32_t N, size_t* bytes);
+int g4_prefillOperandBytes(uint32_t N, uint32_t vectors, size_t* bytes);
+int g4_prefillPrep(g4_ctx* ctx, const float* x, uint32_t nparts, const uint16_t* w1,
+                   const float* residual, const uint16_t* out_scale, const uint16_t* w2, float* h_out,
+                   float* out, void* ops, uint32_t N, uint32_t vectors, float eps);
+/* outputs[i] [*ksplit][vectors][rows[i]] = partial sums of up to 4 matrices
+ * (wtype 0 Q4_K, 1 Q6_K, 2 f16 rows) times the vectors behind `ops`, K in
+ * *ksplit <= max_ksplit chunks which the consumer adds in order.
+ * product_ops: `ops` are g4_prefillGateUp's. wops: scratch for the unpacked
+ * weights, g4_prefillWeightBytes(wtype, the rows of all segments, each
+ * rounded up to a multiple of 16, N) bytes, free again once the launch ends. */
+int g4_prefillMatmul(g4_ctx* ctx, int wtype, const void* const* weights, float* const* outputs,
+                     const uint32_t* rows, int nseg, uint32_t N, const void* ops, int product_ops,
+                     uint32_t vectors, void* wops, size_t wops_bytes, uint32_t max_ksplit, uint32_t* ksplit);
+/* gelu(W_gate . x) * (W_up . x), left as operand blocks of the down
+ * projection (product_ops, g4_prefillOperandBytes(M, vectors) bytes); M a
+ * multiple of 256. */
+int g4_prefillGateUp(g4_ctx* ctx, int wtype, const void* w_gate, const void* w_up, const void* ops,
+                     void* product_ops, uint32_t M, uint32_t N, uint32_t vectors, void* wops,
+                     size_t wops_bytes);
+
 /* ------------------------------------------------------------------------ */
 /* Debug / test exports                                                      */
 /* ------------------------------------------------------------------------ */

@@ -1,0 +1,141 @@
+"""GPU parity of the whole-prompt path: the prefill matmuls against a float64
+product of the same dequantized weights, at the edges of their 64-vector and
+256- / 128- / 16-row tiles, and prompts of more than one chunk against the
+chunk-by-chunk path on the same weights (itself held to the oracle's
+sequential forwards in test_gpu_prefill.py).
+
+Tolerances: Q4_K and f16 weights enter the matrix cores exactly and the
+vectors as 22-bit hi + lo pairs, so only f32 accumulation is left (a few
+1e-7): 2e-6. Q6_K weights round sc * (q - 32) once to f16 (2^-12 at most,
+1.4e-4 root mean square): 3e-4. A prompt's layers append f16 K/V rows, whose
+half-ulp differences (2^-12) reach its last token: 1e-3, the paths' bar."""
+import numpy as np
+import pytest
+
+import oracle as O
+import synth
+from g4hip.decoder import BatchDecoder, E2BShape
+from gpu_util import assert_close
+
+pytestmark = pytest.mark.gpu
+
+BAR = {"q4k": 2e-6, "q6k": 3e-4, "f16": 2e-6}
+
+
+def _weights(wtype, seed, M, N):
+    """Blocks as stored and their float64 values [M][N]."""
+    if wtype == "f16":
+        w = O.gen_normal_f16(seed, M * N, 0.0, 0.03)
+        return w, O.np_f16_to_f32(w).astype(np.float64).reshape(M, N)
+    b = (synth.q4k_centered if wtype == "q4k" else synth.q6k_wide)(seed, M * N // 256)
+    deq = O.np_dequant_q4k if wtype == "q4k" else O.np_dequant_q6k
+    return b, deq(b).astype(np.float64).reshape(M, N)
+
+
+def _vectors(seed, T, N):
+    X = O.gen_normal_f32(seed, T * N, 0.0, 1.5).reshape(T, N)
+    X[T // 2] *= 40.0   # one vector of another scale, one with a huge element, one of zeros
+    X[0, 3] = 3e4
+    X[T - 1] = 0.0
+    return X
+
+
+def _ops(ctx, X):
+    T, N = X.shape
+    ops = ctx.alloc(ctx.prefill_operand_bytes(N, T))
+    ctx.prefillPrep(ctx.from_numpy(X), 1, None, None, None, None, None, None, N, T, ops=ops)
+    ctx.sync()
+    return ops
+
+
+@pytest.mark.parametrize("wtype,rows,N,T,split", [
+    ("q4k", [2048, 256, 256], 1536, 65, 1),    # q/k/v, one vector past a tile
+    ("q4k", [16], 1536, 1, 1),                 # the smallest
+    ("q4k", [100, 33], 2048, 130, 1),          # rows that fill no tile, a padded segment
+    ("q4k", [1536], 4096, 127, 16),            # o of a head-dim-512 layer, K split
+    ("q6k", [1536], 2048, 64, 8),
+    ("q6k", [257], 1536, 100, 2),              # one row past a 256-row group
+    ("f16", [256], 1536, 129, 6),
+    ("f16", [1536], 256, 70, 1),               # one super-block
+    ("q4k", [4096, 512, 512], 1536, 700, 1),   # enough row groups and vectors for the wide row tiles
+    ("q6k", [4096], 1536, 1030, 1),
+])
+def test_prefill_matmul(ctx, wtype, rows, N, T, split):
+    WV = [_weights(wtype, 11 + i, M, N) for i, M in enumerate(rows)]
+    X = _vectors(5, T, N)
+    wops = ctx.alloc(ctx.prefill_weight_bytes(wtype, rows, N))
+    Y = [ctx.zeros(split * T * M, np.float32) for M in rows]
+    ks = ctx.prefillMatmul(wtype, [ctx.from_numpy(b) for b, _ in WV], Y, rows, N, _ops(ctx, X), T, wops, split)
+    assert 1 <= ks <= split
+    for (_, w), y, M in zip(WV, Y, rows):
+        got = y.download(np.float32, ks * T * M).reshape(ks, T, M).astype(np.float64).sum(0)
+        want = X.astype(np.float64) @ w.T
+        assert np.all(np.isfinite(got))
+        for v in sorted({0, T // 2, T - 1, min(63, T - 1), min(64, T - 1)}):
+            assert O.rel_l2(got[v], want[v]) <= BAR[wtype], (M, v)
+        assert O.rel_l2(got, want) <= BAR[wtype]
+
+
+@pytest.mark.parametrize("wtype", ["q4k", "q6k", "f16"])
+@pytest.mark.parametrize("down", ["q4k", "q6k", "f16"])
+def test_prefill_ffn(ctx, wtype, down):
+    """gate/up -> GELU product -> down, over 90 vectors (a whole tile and a part of one)."""
+    N, M, T = 1536, 512, 90
+    (gb, g), (ub, u) = (_weights(wtype, s, M, N) for s in (21, 22))
+    db, d = _weights(down, 23, 1536, M)
+    X = O.gen_normal_f32(7, T * N, 0.0, 0.5).reshape(T, N)
+    X[T // 2] *= 20.0
+    X[T - 1] = 0.0
+    wops = ctx.alloc(max(ctx.prefill_weight_bytes(wtype, [M, M], N), ctx.prefill_weight_bytes(down, [1536], M)))
+    prod = ctx.alloc(ctx.prefill_operand_bytes(M, T))
+    Y = ctx.zeros(2 * T * 1536, np.float32)
+    ctx.prefillGateUp(wtype, ctx.from_numpy(gb), ctx.from_numpy(ub), _ops(ctx, X), prod, M, N, T, wops)
+    ks = ctx.prefillMatmul(down, [ctx.from_numpy(db)], [Y], [1536], M, prod, T, wops, 2, product_ops=True)
+    got = Y.download(np.float32, ks * T * 1536).reshape(ks, T, 1536).astype(np.float64).sum(0)
+    x = X.astype(np.float64)
+    a = x @ g.T
+    t = np.clip(0.7978845608028654 * a * (1 + 0.044715 * a * a), -15, 15)
+    want = (0.5 * a * (1 + np.tanh(t)) * (x @ u.T)) @ d.T
+    # (the GELU's own f32 evaluation adds a few 1e-7 relative to the product's size; twice the weights' bar)
+    bar = BAR[down] + 2 * BAR[wtype]
+    assert np.all(np.isfinite(got))
+    assert O.rel_l2(got, want) <= bar
+    for v in (0, 63, 64):
+        assert O.rel_l2(got[v], want[v]) <= bar, v
+
+
+@pytest.mark.parametrize("layout,B,T,start", [
+    ("uniform", 64, 65, 0),      # one row past a chunk
+    ("uniform", 64, 300, 600),   # past the window
+    ("real", 64, 131, 37),
+    ("real", 7, 23, 0),          # odd chunks
+    ("uniform", 1, 3, 5),
+])
+def test_wide_prefill_equals_chunks(ctx, layout, B, T, start):
+    s = (E2BShape(n_layers=2, global_layers=(1,), vocab=4096) if layout == "uniform" else
+         E2BShape.real(n_layers=4, n_unshared=2, global_layers=(1, 3), vocab=4096))
+    d = BatchDecoder(ctx, [0] * B, s, seed=31, reserve=start + T + 2 * B, shared_pages=True, embed=True)
+    assert d.wide_rows >= B
+    toks = np.random.default_rng(3).integers(0, s.vocab, T).astype(np.uint32)
+
+    def go(**kw):
+        d.fill_kv(seed=32)
+        row = d.prefill(toks, start, **kw)
+        ctx.sync()
+        kv = [p.download(np.uint16).view(np.float16).astype(np.float32) for L in d.layers
+              for p in (L.k_cache, L.v_cache)]
+        return (row, d.hidden.download(np.float32).reshape(B, -1), d.logits.download(np.float32).reshape(B, -1),
+                d.tokens.download(np.uint32), d.seq_lens.download(np.uint32), kv)
+
+    want = go(probe=lambda *a: None)  # chunk by chunk
+    for rows in (d.wide_rows, max(B, 128 // B * B)):  # one pass, then several
+        d.wide_rows = rows
+        got = go()
+        assert got[0] == want[0]
+        n = got[0]
+        assert_close(got[1][n], want[1][n], what="hidden")
+        assert_close(got[2][n], want[2][n], what="logits")
+        assert got[3][n] == O.argmax(got[2][n])
+        assert np.array_equal(got[4], want[4])
+        for a, b in zip(got[5], want[5]):
+            assert_close(a, b, what="cache")
