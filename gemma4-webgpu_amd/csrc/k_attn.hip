@@ -1060,6 +1060,7 @@ struct ProArgs {
   const uint32_t* seq_lens;
   uint32_t page_size, max_pages, num_pages, cap;
   const float2* rope_cs;  // [cap][hd/2] (cos, sin) of every position (g4_ropeTable), or null
+  uint32_t table_stride;  // page-table entries from one row's list to the next (0: one list for all)
 };
 
 // Elements i0 and i1 summed over the n partials in chunk order; the loads of
@@ -1137,7 +1138,7 @@ __global__ __launch_bounds__(NT) void attn_prologue_kernel(ProArgs a) {
   }
   // append at pos when the length is in range and the page id is in the pool
   if (L == 0 || L > a.cap) return;
-  const int32_t pg = a.page_table[(size_t)seq * a.max_pages + pos / a.page_size];
+  const int32_t pg = a.page_table[(size_t)seq * a.table_stride + pos / a.page_size];
   if (pg < 0 || pg >= (int32_t)a.num_pages) return;
   const size_t row = ((size_t)pg * a.page_size + pos % a.page_size) * a.nkh + kvh;
   uint16_t* kd = a.kp + row * a.hd;
@@ -1836,30 +1837,31 @@ int g4_pagedAttnDecodeFused(g4_ctx* ctx, const float* q_raw, const float* k_raw,
   return merge(ctx, a, output, sp, p.num_seqs, G, p.head_dim);
 }
 
-int g4_pagedAttnPrologue(g4_ctx* ctx, const float* q_parts, const float* k_parts, const float* v_parts,
-                         uint32_t nparts, const uint16_t* q_norm_w, const uint16_t* k_norm_w,
-                         const uint16_t* rope_freqs, float* q_out, uint16_t* k_pool, uint16_t* v_pool,
-                         const int32_t* page_table, const uint32_t* seq_lens, g4_paged_attn_fused_params p,
-                         const float* rope_cs, uint32_t rope_rows) {
-  G4_ENTER(ctx);
-  G4_REQUIRE(!rope_cs || rope_rows >= p.max_seq_len, "g4_pagedAttnPrologue: RoPE table of %u rows < max_seq_len %u",
+// The attention prologue of the paged forms: one page list per row
+// (table_stride max_pages) or one for every row (0).
+static int paged_prologue(g4_ctx* ctx, const char* fn, const float* q_parts, const float* k_parts,
+                          const float* v_parts, uint32_t nparts, const uint16_t* q_norm_w, const uint16_t* k_norm_w,
+                          const uint16_t* rope_freqs, float* q_out, uint16_t* k_pool, uint16_t* v_pool,
+                          const int32_t* page_table, const uint32_t* seq_lens, g4_paged_attn_fused_params p,
+                          const float* rope_cs, uint32_t rope_rows, uint32_t table_stride) {
+  G4_REQUIRE(!rope_cs || rope_rows >= p.max_seq_len, "%s: RoPE table of %u rows < max_seq_len %u", fn,
              rope_rows, p.max_seq_len);
   G4_REQUIRE(q_parts && q_norm_w && q_out && page_table && seq_lens && nparts >= 1,
-             "g4_pagedAttnPrologue: null buffer or no parts");
+             "%s: null buffer or no parts", fn);
   // k_parts = v_parts = null: q only (a layer reading its producer layer's
   // pool appends no row); the pools and k_norm_w are then not used
   const bool kv = k_parts != nullptr;
   G4_REQUIRE(kv ? (v_parts && k_norm_w && k_pool && v_pool) : !v_parts,
-             "g4_pagedAttnPrologue: k_parts, v_parts, k_norm_w and the pools go together");
-  G4_REQUIRE(((uintptr_t)rope_cs & 7) == 0, "g4_pagedAttnPrologue: rope_cs must be 8-byte aligned");
-  G4_REQUIRE(!p.apply_divisor || rope_freqs, "g4_pagedAttnPrologue: apply_divisor needs rope_freqs");
+             "%s: k_parts, v_parts, k_norm_w and the pools go together", fn);
+  G4_REQUIRE(((uintptr_t)rope_cs & 7) == 0, "%s: rope_cs must be 8-byte aligned", fn);
+  G4_REQUIRE(!p.apply_divisor || rope_freqs, "%s: apply_divisor needs rope_freqs", fn);
   G4_REQUIRE(p.num_seqs > 0 && p.num_seqs <= 65535 && p.num_q_heads > 0 && p.num_kv_heads > 0,
-             "g4_pagedAttnPrologue: empty batch or heads");
+             "%s: empty batch or heads", fn);
   G4_REQUIRE(p.head_dim >= 2 && p.head_dim <= 2 * NT && p.head_dim % 2 == 0,
-             "g4_pagedAttnPrologue: head_dim %u must be even and <= %d", p.head_dim, 2 * NT);
+             "%s: head_dim %u must be even and <= %d", fn, p.head_dim, 2 * NT);
   G4_REQUIRE(p.page_size > 0 && p.max_pages > 0 && p.num_pages > 0 && p.max_seq_len > 0 &&
                  (uint64_t)p.max_seq_len <= (uint64_t)p.page_size * p.max_pages,
-             "g4_pagedAttnPrologue: max_seq_len %u exceeds the page table (%u x %u)", p.max_seq_len, p.max_pages,
+             "%s: max_seq_len %u exceeds the page table (%u x %u)", fn, p.max_seq_len, p.max_pages,
              p.page_size);
   ProArgs a{};
   a.q = q_parts;
@@ -1886,10 +1888,31 @@ int g4_pagedAttnPrologue(g4_ctx* ctx, const float* q_parts, const float* k_parts
   a.num_pages = p.num_pages;
   a.cap = p.max_seq_len;
   a.rope_cs = (const float2*)rope_cs;
+  a.table_stride = table_stride;
   hipLaunchKernelGGL(attn_prologue_kernel, dim3(p.num_q_heads + (kv ? p.num_kv_heads : 0u), p.num_seqs), dim3(NT), 0,
                      ctx->stream, a);
   G4_LAUNCHED(ctx, "attn_prologue");
   return G4_OK;
+}
+
+int g4_pagedAttnPrologue(g4_ctx* ctx, const float* q_parts, const float* k_parts, const float* v_parts,
+                         uint32_t nparts, const uint16_t* q_norm_w, const uint16_t* k_norm_w,
+                         const uint16_t* rope_freqs, float* q_out, uint16_t* k_pool, uint16_t* v_pool,
+                         const int32_t* page_table, const uint32_t* seq_lens, g4_paged_attn_fused_params p,
+                         const float* rope_cs, uint32_t rope_rows) {
+  G4_ENTER(ctx);
+  return paged_prologue(ctx, __func__, q_parts, k_parts, v_parts, nparts, q_norm_w, k_norm_w, rope_freqs, q_out,
+                        k_pool, v_pool, page_table, seq_lens, p, rope_cs, rope_rows, p.max_pages);
+}
+
+int g4_prefillAttnPrologue(g4_ctx* ctx, const float* q_raw, const float* k_raw, const float* v_raw,
+                           const uint16_t* q_norm_w, const uint16_t* k_norm_w, const uint16_t* rope_freqs,
+                           float* q_out, uint16_t* k_pool, uint16_t* v_pool, const int32_t* page_table,
+                           const uint32_t* lens, g4_paged_attn_fused_params p, const float* rope_cs,
+                           uint32_t rope_rows) {
+  G4_ENTER(ctx);
+  return paged_prologue(ctx, __func__, q_raw, k_raw, v_raw, 1, q_norm_w, k_norm_w, rope_freqs, q_out, k_pool, v_pool,
+                        page_table, lens, p, rope_cs, rope_rows, 0);
 }
 
 // g4_pagedAttnBlock: the one-launch plan (pmqf_kernel) when the window takes

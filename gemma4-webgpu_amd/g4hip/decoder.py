@@ -1180,8 +1180,8 @@ class BatchDecoder(_SyntheticModel):
         per decoder, longer than a chunk, and widths the prefill kernels take."""
         s = self.s
         return (self.shared_pages and self.embedding is not None and self.max_seq > self.B
-                and s.hidden in (1536, 2048) and s.ple_dim in (0, 256)
-                and all(s.q_dim_of(il) in (1536, 2048, 4096) and s.ffn_of(il) % 256 == 0
+                and s.hidden in (1536, 2048) and s.ple_dim in (0, 256) and s.n_q_heads == 8 * s.n_kv_heads
+                and all(s.hd(il) in (256, 512) and s.q_dim_of(il) in (1536, 2048, 4096) and s.ffn_of(il) % 256 == 0
                         and L.qt["wgate"] == L.qt["wup"] for il, L in enumerate(self.layers)))
 
     def _build_wide(self) -> None:
@@ -1196,14 +1196,18 @@ class BatchDecoder(_SyntheticModel):
         # split-K partial sums of o and down: four chunks of a full pass, more of a short one
         self.wide_parts = 4 * max(R, 512) * H
         w["parts"] = c.empty(self.wide_parts, f32)
-        need = 0
+        need, ws = 0, 0
         for il, L in enumerate(self.layers):
+            ws = max(ws, c.prefill_attn_workspace_bytes(c.paged_fused_params(
+                R, s.n_q_heads, s.n_kv_heads, s.hd(il), self.page_size, self.max_pages, self.max_seq, self.num_pages,
+                0, s.eps, 1.0, 0)))
             Q, KV, I = s.q_dim_of(il), s.kv_dim_of(il), s.ffn_of(il)
             qkv = [("wq", Q)] + ([("wk", KV), ("wv", KV)] if s.is_producer(il) else [])
             for ms, rows, n in [([m for m, _ in qkv], [r for _, r in qkv], H), (["wo"], [H], Q),
                                 (["wgate", "wup"], [I, I], H), (["wdown"], [H], I)]:
                 need = max([need] + [c.prefill_weight_bytes(L.qt[m], rows, n) for m in ms])
         w["wops"] = c.empty(need, np.uint8)
+        w["attn_ws"] = c.empty(ws, np.uint8)
         if s.ple_dim:
             LD = s.n_layers * s.ple_dim
             w.update(hidden3=c.empty(R * H, f32), ple_projected=c.empty(R * LD, f32), ple_inputs=c.empty(R * LD, f32),
@@ -1220,7 +1224,7 @@ class BatchDecoder(_SyntheticModel):
         n = 0
         for at in range(0, T + pad, self.wide_rows):
             n = min(self.wide_rows, T + pad - at)
-            self._wide_pass(dtok.offset(4 * at), dlen.offset(4 * at), n)
+            self._wide_pass(dtok.offset(4 * at), dlen.offset(4 * at), n, int(clen[at:at + n].max()))
         # the last B rows are what the last chunk of B rows leaves: the residual
         # stream, its tokens and lengths, then the head and the sample
         c.copy(self.hidden, w["hidden"].offset(4 * H * (n - B)), 4 * H * B)
@@ -1233,10 +1237,11 @@ class BatchDecoder(_SyntheticModel):
         dtok.free()
         dlen.free()
 
-    def _wide_pass(self, tokens, lens, n: int) -> None:
-        """n rows (a multiple of B) of one prompt through every layer; the
-        residual stream after the last layer is left in wide["hidden"]."""
-        c, s, B, w = self.ctx, self.s, self.B, self.wide
+    def _wide_pass(self, tokens, lens, n: int, end: int) -> None:
+        """n rows of one prompt, their lengths at most `end`, through every
+        layer; the residual stream after the last layer is left in
+        wide["hidden"]."""
+        c, s, w = self.ctx, self.s, self.wide
         H, wops = s.hidden, w["wops"]
         c.embeddingLookupBatch(self.embedding, s.vocab, w["hidden"], H, tokens, n)
         if s.ple_dim:
@@ -1266,16 +1271,15 @@ class BatchDecoder(_SyntheticModel):
             outs = [w["q"], w["k"], w["v"]] if prod else [w["q"]]
             for qt, ws, go, gr in qkv_groups(L, outs, [Q, KV, KV] if prod else [Q]):
                 c.prefillMatmul(qt, ws, go, gr, H, w["xops"], n, wops)
-            rope = self.rope_cs[s.is_global(il)]
-            for r in range(0, n, B):  # every row of the pass is appended before any is read
-                c.pagedAttnPrologue(w["q"].offset(4 * Q * r), w["k"].offset(4 * KV * r) if prod else None,
-                                    w["v"].offset(4 * KV * r) if prod else None, 1, L.q_norm, L.k_norm,
-                                    self.rope_freqs, w["q"].offset(4 * Q * r), L.k_cache if prod else None,
-                                    L.v_cache if prod else None, self.page_table, lens.offset(4 * r),
-                                    self.pro_params[il], rope, self.rope_rows)
-            for r in range(0, n, B):
-                c.pagedAttnDecode(w["q"].offset(4 * Q * r), L.k_cache, L.v_cache, self.page_table, lens.offset(4 * r),
-                                  w["attn"].offset(4 * Q * r), self.attn_params[il], self.attn_ws)
+            # every row of the pass is appended before any is read
+            glob = s.is_global(il)
+            p = c.paged_fused_params(n, s.n_q_heads, s.n_kv_heads, s.hd(il), self.page_size, self.max_pages, end,
+                                     self.num_pages, 0 if glob else s.window, s.eps,
+                                     s.theta_global if glob else s.theta_local, int(glob))
+            c.prefillAttnPrologue(w["q"], w["k"] if prod else None, w["v"] if prod else None, L.q_norm, L.k_norm,
+                                  self.rope_freqs, w["q"], L.k_cache if prod else None, L.v_cache if prod else None,
+                                  self.page_table, lens, p, self.rope_cs[glob], self.rope_rows)
+            c.prefillAttn(w["q"], L.k_cache, L.v_cache, self.page_table, lens, w["attn"], p, w["attn_ws"])
             c.prefillPrep(w["attn"], 1, None, None, None, None, None, None, Q, n, s.eps, ops=w["aops"])
             no = c.prefillMatmul(L.qt["wo"], [L.wo], [w["parts"]], [H], Q, w["aops"], n, wops, max_ks)
             c.prefillPrep(w["parts"], no, L.post_attn_norm, w["hidden"], None, L.pre_ffn_norm, w["hidden2"], None, H,

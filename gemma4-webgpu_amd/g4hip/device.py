@@ -365,6 +365,26 @@ class Context:
         check(lib().g4_prefillGateUp(self.h, PREFILL_TYPES[wtype], _p(w_gate), _p(w_up), _p(ops), _p(product_ops),
                                      M, N, vectors, _p(wops), wops.nbytes))
 
+    def prefillAttnPrologue(self, q_raw: Ptr, k_raw: Ptr, v_raw: Ptr, q_norm_w: Ptr, k_norm_w: Ptr, rope_freqs: Ptr,
+                            q_out: Ptr, k_pool: Ptr, v_pool: Ptr, page_table: Ptr, lens: Ptr, params,
+                            rope_cs: Ptr = None, rope_rows: int = 0) -> None:
+        """q/k norm + RoPE, v_norm and the K/V append of params.num_seqs rows of one page list."""
+        check(lib().g4_prefillAttnPrologue(self.h, _p(q_raw), _p(k_raw), _p(v_raw), _p(q_norm_w), _p(k_norm_w),
+                                           _p(rope_freqs), _p(q_out), _p(k_pool), _p(v_pool), _p(page_table),
+                                           _p(lens), params, _p(rope_cs), rope_rows))
+
+    @staticmethod
+    def prefill_attn_workspace_bytes(params) -> int:
+        n = ctypes.c_size_t()
+        check(lib().g4_prefillAttn_workspace_size(params, ctypes.byref(n)))
+        return int(n.value)
+
+    def prefillAttn(self, q: Ptr, k_pool: Ptr, v_pool: Ptr, page_table: Ptr, lens: Ptr, out: Ptr, params,
+                    workspace: Optional[Buffer] = None, scale: float = 1.0) -> None:
+        """Attention of params.num_seqs rows over one page list, row v over the positions below lens[v]."""
+        check(lib().g4_prefillAttn(self.h, _p(q), _p(k_pool), _p(v_pool), _p(page_table), _p(lens), _p(out), params,
+                                   scale, _p(workspace), workspace.nbytes if workspace is not None else 0))
+
     # ---- per-layer embeddings (shaders/ple_*.wgsl) ----
     def pleStage1Fuse(self, projected: Ptr, norm_w: Ptr, table: Ptr, table_rows: int, ple_inputs: Ptr,
                       num_layers: int, per_layer_dim: int = 256, eps: float = 1e-6, token: int = 0,

@@ -724,6 +724,25 @@ int g4_prefillMatmul(g4_ctx* ctx, int wtype, const void* const* weights, float* 
 int g4_prefillGateUp(g4_ctx* ctx, int wtype, const void* w_gate, const void* w_up, const void* ops,
                      void* product_ops, uint32_t M, uint32_t N, uint32_t vectors, void* wops,
                      size_t wops_bytes);
+/* The attention of p.num_seqs rows (1..65535) of one sequence over one page
+ * list (page_table [p.max_pages]; every row may read every position below
+ * its length, so appending all rows first makes the pass causal).
+ * g4_prefillAttnPrologue: g4_pagedAttnPrologue with that list and whole
+ * sums. g4_prefillAttn: out [num_seqs][num_q_heads * head_dim] from the roped
+ * q, 8 query heads per KV head of dim 256 or 512; row v attends to the
+ * positions below lens[v], the last p.sliding_window of them when non-zero;
+ * p.max_seq_len bounds the lengths (p.eps, theta and apply_divisor unused).
+ * workspace: split partials of short passes over long caches
+ * (g4_prefillAttn_workspace_size; a smaller one or NULL splits less). */
+int g4_prefillAttnPrologue(g4_ctx* ctx, const float* q_raw, const float* k_raw, const float* v_raw,
+                           const uint16_t* q_norm_w, const uint16_t* k_norm_w,
+                           const uint16_t* rope_freqs, float* q_out, uint16_t* k_pool, uint16_t* v_pool,
+                           const int32_t* page_table, const uint32_t* lens, g4_paged_attn_fused_params p,
+                           const float* rope_cs, uint32_t rope_rows);
+int g4_prefillAttn_workspace_size(g4_paged_attn_fused_params p, size_t* bytes);
+int g4_prefillAttn(g4_ctx* ctx, const float* q, const uint16_t* k_pool, const uint16_t* v_pool,
+                   const int32_t* page_table, const uint32_t* lens, float* out,
+                   g4_paged_attn_fused_params p, float scale, void* workspace, size_t workspace_bytes);
 
 /* ------------------------------------------------------------------------ */
 /* Debug / test exports                                                      */

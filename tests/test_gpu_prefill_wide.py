@@ -139,3 +139,44 @@ def test_wide_prefill_equals_chunks(ctx, layout, B, T, start):
         assert np.array_equal(got[4], want[4])
         for a, b in zip(got[5], want[5]):
             assert_close(a, b, what="cache")
+
+
+def _attn_case(ctx, hd, T, start, window, n_kv=1, short_ws=False):
+    """Rows at start .. start + T - 1 of one scattered page list against the oracle's paged attention."""
+    page, nq = 16, 8 * n_kv
+    L = start + T
+    pages = -(-L // page) + 2
+    table = np.random.default_rng(L).permutation(pages).astype(np.int32)
+    kp, vp = (O.gen_normal_f16(s, pages * page * n_kv * hd, 0.0, 1.0 if s == 42 else 0.25) for s in (41, 42))
+    q = O.gen_normal_f32(43, T * nq * hd, 0.0, 0.5).reshape(T, nq * hd)
+    lens = (start + 1 + np.arange(T)).astype(np.uint32)
+    if T > 2:
+        lens[-1] = lens[-2]   # a repeated row, as a padded chunk has
+    p = ctx.paged_fused_params(T, nq, n_kv, hd, page, pages, pages * page, pages, window, 1e-6, 1e4, 0)
+    out = ctx.zeros(T * nq * hd, np.float32)
+    ws = None if short_ws else ctx.alloc(ctx.prefill_attn_workspace_bytes(p))
+    ctx.prefillAttn(ctx.from_numpy(q), ctx.from_numpy(kp), ctx.from_numpy(vp), ctx.from_numpy(table),
+                    ctx.from_numpy(lens), out, p, ws)
+    got = out.download(np.float32).reshape(T, -1)
+    for v in sorted({0, 1, 6, 7, 8, T // 2, T - 2, T - 1} & set(range(T))):
+        want = O.attention_paged(q[v], kp, vp, table, page, nq, n_kv, hd, int(lens[v]), 1.0, window)
+        # q and P enter as 22-bit pairs, exp2 is within 1e-5 relative: 4e-5
+        assert_close(got[v], want, rel=4e-5, what=f"row {v}")
+
+
+@pytest.mark.parametrize("hd", [256, 512])
+@pytest.mark.parametrize("T,start,window", [
+    (1, 0, 0), (7, 0, 0), (8, 0, 32), (9, 0, 0), (33, 0, 0), (65, 500, 512), (17, 31, 40), (40, 600, 512),
+    (9, 3000, 0),      # few rows over a long cache: the window split over workgroups
+    (300, 700, 0),
+])
+def test_prefill_attention(ctx, hd, T, start, window):
+    _attn_case(ctx, hd, T, start, window)
+
+
+def test_prefill_attention_two_kv_heads(ctx):
+    _attn_case(ctx, 256, 21, 100, 64, n_kv=2)
+
+
+def test_prefill_attention_without_workspace(ctx):
+    _attn_case(ctx, 512, 9, 2000, 0, short_ws=True)
