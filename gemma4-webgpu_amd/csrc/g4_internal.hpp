@@ -351,7 +351,6 @@ struct OpsSub {
 //   scale [t][half][16] f32: 2^-e of vector 16t + lane%16
 struct PfOps {
   static constexpr uint32_t MAIN_T = Ops::MAIN_T;
-  static constexpr uint32_t STEP = 4 * 4096;  // 64 k of the four vector tiles
   static constexpr uint32_t SUMS = 4 * MAIN_T;
   static constexpr uint32_t SCALE = SUMS + 4 * 1024;
   static constexpr uint32_t BYTES = SCALE + 4 * 128;

@@ -15,10 +15,14 @@
 //  * pf_gemm_kernel: a workgroup (4 waves) owns 64 RT rows (RT 16-row tiles
 //    per wave) x 64 vectors. The weight operands go from memory (L2) straight
 //    into registers, 1 KB contiguous per wave load; the activation operands
-//    (f16 hi + lo, twice the bytes) are shared by the waves through a double
-//    LDS buffer of 64 k. With RT = 4 a wave issues 64 MFMAs per 16 KB of LDS
-//    reads, half the LDS rate; with all operands in LDS the reads would take
-//    as long as the products.
+//    (f16 hi + lo, twice the bytes) are shared by the waves through LDS. With
+//    RT = 4 a wave issues 32 MFMAs per 8 KB of LDS reads, half the LDS rate;
+//    with all operands in LDS the reads would take as long as the products.
+//    Both streams run three to four 32-k sub-blocks ahead (about 1.5 us): a
+//    form with the next 64 k in flight, whose loads the compiler moved next
+//    to their use, spent 13 us per super-block, eight times its products,
+//    waiting for memory (gate/up 2 x 6144 x 1536 at 1900 vectors 241 -> 156
+//    us, o 101 -> 55, down 12288 wide 159 -> 138: 1040 TFLOP/s of f16 products).
 // The arithmetic is that of mmf_kernel: x * 2^e as f16 hi + lo, exact f16
 // sc * q (Q6_K rounds once above 2048), f32 accumulation over a super-block,
 // then d and 2^-e in f32.
@@ -44,11 +48,18 @@ struct PfSeg {
 // Unpacked weights of one launch: rtn row tiles of 16 rows (each segment
 // padded to whole tiles, the padding repeating its last row).
 struct PfWeights {
-  uint8_t* A;   // [rtn][K/32][64 lanes] 16 B: f16 sc * q of row lane % 16, k = 32s + 8 (lane / 16) .. +7
-  uint8_t* Mn;  // Q4_K: [rtn][K/256][64 lanes] 16 B: the min operand
-  float* D;     // [K/256][16 rtn]: d
-  float* DM;    // Q4_K: 64 dmin
+  uint8_t* A;  // [rtn][K/32][64 lanes] 16 B: f16 sc * q of row lane % 16, k = 32s + 8 (lane / 16) .. +7
+  uint8_t* X;  // [rtn][K/256][Aux<QT>::BYTES]: see Aux
 };
+// A row tile and super-block's values beside the operands: d [16 rows] f32;
+// Q4_K also 64 dmin [16 rows] f32 and per lane the f16 mins of row lane % 16,
+// sub-blocks 2 (lane / 16) and + 1. CH: its 16-byte pieces.
+template <int QT>
+struct Aux {
+  static constexpr uint32_t BYTES = QT == 0 ? 384 : (QT == 1 ? 64 : 0);
+  static constexpr uint32_t DM = 64, MN = 128, CH = BYTES / 16;
+};
+uint32_t aux_bytes(int wtype) { return wtype == 0 ? Aux<0>::BYTES : (wtype == 1 ? Aux<1>::BYTES : 0u); }
 
 struct PfArgs {
   PfSeg s[kMaxSeg];
@@ -97,14 +108,35 @@ __global__ __launch_bounds__(NT) void unpack_kernel(PfArgs a) {
       dp[i] = g4d::f16_bits_to_f32(wr.dd[i] & 0xffffu);
       if constexpr (QT == 0) dmp[i] = g4d::f16_bits_to_f32(wr.dd[i] >> 16) * 64.0f;
     }
-    const size_t di = (size_t)sb * a.rtn * 16u + rt * 16u + 4u * q;
-    if (c == 0) *(float4*)(a.w.D + di) = d;
+    uint8_t* x = a.w.X + ((size_t)rt * a.nsb + sb) * Aux<QT>::BYTES;
+    if (c == 0) *(float4*)(x + 16 * q) = d;
     if constexpr (QT == 0) {
-      if (c == 0) *(float4*)(a.w.DM + di) = dm;
-      ((u32x4*)a.w.Mn)[((size_t)rt * a.nsb + sb) * 64u + l] = __builtin_bit_cast(u32x4, min_operand(wr, q));
+      if (c == 0) *(float4*)(x + Aux<0>::DM + 16 * q) = dm;
+      const h8 m = min_operand(wr, q);
+      *(uint32_t*)(x + Aux<0>::MN + 4 * l) = pack_h2(m[0], m[4]);
     }
   }
 }
+
+// One 32-k sub-block of the four vector tiles in LDS (f16 hi and lo, 2 KB a
+// tile), in a ring of four, and the values a super-block's sums need, in
+// turn: the vectors' part (their sub-block sums and 2^-e) and each wave's own
+// row tiles'. Separate LDS objects: the compiler then waits for a
+// global -> LDS load only where its own object is read.
+constexpr uint32_t SUB = 4 * 2048;
+constexpr uint32_t VAUX_LDS = 5120;  // an operand block's sums and scales (4608 B), in whole 1 KB loads
+constexpr uint32_t WAUX_LDS = 2048;  // a wave's row tiles' Aux values, likewise
+
+__device__ __forceinline__ void to_lds(const void* src, uint8_t* dst) {  // 16 bytes per lane, dst + 16 lane
+  __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+// Barrier after which LDS written before it (global -> LDS loads: by waves
+// that waited for them) is readable; waits for no load in flight.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // MODE 0: row group g is row tiles 4 RT g .. +4 RT - 1 of the segments in
 // order, RT consecutive tiles per wave. MODE 1 (gate/up, RT 4): segments 0
@@ -117,8 +149,11 @@ __global__ __launch_bounds__(NT) void unpack_kernel(PfArgs a) {
 template <int QT, int RT, int MODE, int SG>
 __global__ __launch_bounds__(NT, 2) void pf_gemm_kernel(PfArgs a) {
   static_assert(MODE == 0 || RT == 4, "gate/up: two tiles of each");
-  __shared__ __align__(16) uint8_t lds[2][PfOps::STEP];
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, q = l >> 4, c = l & 15;
+  __shared__ __align__(16) uint8_t b0[SUB], b1[SUB], b2[SUB], b3[SUB];
+  __shared__ __align__(16) uint8_t vaux[2 * VAUX_LDS], waux[QT == 2 ? 16 : 2 * 4 * WAUX_LDS];
+  uint8_t* const ring[4] = {b0, b1, b2, b3};
+  const int tid = threadIdx.x, l = tid & 63, q = l >> 4, c = l & 15;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   // Workgroups go to the XCDs in turn (linear id mod 8): XCD x takes the
   // x-th eighth of the items, in which the vector tiles of one row group and
   // K chunk are neighbours, so the group's operands come from that XCD's L2.
@@ -135,10 +170,11 @@ __global__ __launch_bounds__(NT, 2) void pf_gemm_kernel(PfArgs a) {
     if constexpr (MODE == 0) rt[r] = min((g * 4u + w) * RT + r, a.rtn - 1);  // (past the last tile: not stored)
     else rt[r] = (r >= 2 ? a.s[1].rt0 : 0u) + g * 8u + w * 2u + (r & 1);
   }
-  const u32x4* Ap[RT];
+  const u32x4* Ap[RT];  // (uniform)
 #pragma unroll
-  for (int r = 0; r < RT; ++r) Ap[r] = (const u32x4*)a.w.A + ((size_t)rt[r] * nsub + sb0 * 8u) * 64u + l;
+  for (int r = 0; r < RT; ++r) Ap[r] = (const u32x4*)a.w.A + ((size_t)rt[r] * nsub + sb0 * 8u) * 64u;
   const uint8_t* Bg = a.ops + ((size_t)tt * a.nsb + sb0) * PfOps::BYTES;
+  const uint32_t nwalk = a.kc * 8u;  // sub-blocks of the walk
 
   f4 acc[RT][4], C[RT][4];
 #pragma unroll
@@ -146,101 +182,134 @@ __global__ __launch_bounds__(NT, 2) void pf_gemm_kernel(PfArgs a) {
 #pragma unroll
     for (int t = 0; t < 4; ++t) acc[r][t] = f4{0.f, 0.f, 0.f, 0.f};
 
-  u32x4 bs[4];
-  auto stage = [&](const uint8_t* sb, int p) {  // 64 k (step p of the super-block) of every vector tile
-#pragma unroll
-    for (int t = 0; t < 4; ++t) bs[t] = *(const u32x4*)(sb + t * PfOps::MAIN_T + p * 4096 + tid * 16);
+  // sub-block u of the walk: 8 pieces of 1 KB, two per wave (vector tile w,
+  // hi and lo); past the end the last one again, so that every turn issues
+  // the same number of loads
+  auto stage = [&](uint32_t u, uint8_t* buf) {
+    const uint32_t v = min(u, nwalk - 1u);
+    const uint8_t* src = Bg + (size_t)(v >> 3) * PfOps::BYTES + w * PfOps::MAIN_T + (v & 7u) * 2048u + l * 16;
+    to_lds(src, buf + w * 2048);
+    to_lds(src + 1024, buf + w * 2048 + 1024);
   };
-  auto put = [&](int b) {
+  // the values super-block j's sums need
+  auto stage_aux = [&](uint32_t j) {
+    const uint32_t jc = min(j, a.kc - 1u);
+    const uint8_t* src = Bg + (size_t)jc * PfOps::BYTES + PfOps::SUMS;
+    uint8_t* vb = vaux + (j & 1u) * VAUX_LDS;
+    to_lds(src + w * 1024 + l * 16, vb + w * 1024);
+    if (w == 0) to_lds(src + 4096 + min(l, 31) * 16, vb + 4096);
+    if constexpr (QT != 2) {
+      constexpr uint32_t CH = Aux<QT>::CH;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) *(u32x4*)(lds[b] + t * 4096 + tid * 16) = bs[t];
+      for (uint32_t i = 0; i < (RT * CH + 63) / 64; ++i) {
+        const uint32_t ch = min(64u * i + l, RT * CH - 1), r = ch / CH;
+        uint32_t t = rt[0];
+#pragma unroll
+        for (int k = 1; k < RT; ++k) t = r == (uint32_t)k ? rt[k] : t;
+        to_lds(a.w.X + ((size_t)t * a.nsb + sb0 + jc) * Aux<QT>::BYTES + (ch - r * CH) * 16u,
+               waux + ((j & 1u) * 4u + w) * WAUX_LDS + i * 1024u);
+      }
+    }
   };
-  u32x4 A[RT], An[RT];
+
+  // weight operands: a ring of four sub-blocks in registers
+  u32x4 A[4][RT];
+  stage_aux(0);
 #pragma unroll
-  for (int r = 0; r < RT; ++r) A[r] = Ap[r][0];
-  stage(Bg, 0);
-  put(0);
-  __syncthreads();
+  for (int s = 0; s < 3; ++s) stage(s, ring[s]);
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+#pragma unroll
+    for (int r = 0; r < RT; ++r) A[s][r] = Ap[r][s * 64 + l];
+  // (the walk's first waits: known complete here, they cost the loop none)
+  wait_vmcnt<0>();
 
   for (uint32_t j = 0; j < a.kc; ++j) {
-    const bool last_sb = j + 1 == a.kc;  // (uniform)
-    const uint8_t* Bsb = Bg + (size_t)j * PfOps::BYTES;
-    const size_t drow = (size_t)(sb0 + j) * a.rtn * 16u;
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      // the next 64 k of the vectors are in flight during this step (the last
-      // step of the walk reads its own again)
-      stage(p < 3 ? Bsb : (last_sb ? Bsb : Bsb + PfOps::BYTES), (p + 1) & 3);
+    for (int s = 0; s < 8; ++s) {
+      // Sub-block s of the vectors, requested three turns ago, has arrived
+      // once at most what was issued after it is in flight: two turns' two
+      // LDS loads and three turns' RT weight loads (the others only make the
+      // wait stricter). Every wave has also left sub-block s - 1, whose
+      // buffer takes sub-block s + 3.
+      wait_vmcnt<4 + 3 * RT>();
+      lds_barrier();
+      if (s == 4) stage_aux(j + 1);
+      stage(j * 8u + s + 3, ring[(s + 3) & 3]);
+      __builtin_amdgcn_sched_barrier(0);
+      const uint8_t* base = ring[s & 3] + l * 16;
+      const bool first = SG == 2 ? (s & 3) == 0 : s == 0;
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int s = 2 * p + h;
-        {
-          const uint32_t nx = (s == 7 && last_sb) ? j * 8u + s : j * 8u + s + 1;
+      for (int t = 0; t < 4; ++t) {
+        const h8 bh = *(const h8*)(base + t * 2048), bl = *(const h8*)(base + t * 2048 + 1024);
 #pragma unroll
-          for (int r = 0; r < RT; ++r) An[r] = Ap[r][(size_t)nx * 64u];
-        }
-        const uint8_t* base = lds[p & 1] + h * 2048 + l * 16;
-        const bool first = SG == 2 ? (s & 3) == 0 : s == 0;
+        for (int r = 0; r < RT; ++r)
+          C[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, A[s & 3][r]), bh,
+                                                           first ? f4{0.f, 0.f, 0.f, 0.f} : C[r][t], 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+          C[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, A[s & 3][r]), bl, C[r][t], 0, 0, 0);
+      }
+      // the next tile's operands are read while one is multiplied
+      __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);  // LDS reads
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 2 * RT, 0);  // MFMAs
+        if (t < 2) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      }
+      {  // the weight operands four sub-blocks on (past the end: the last again)
+        const uint32_t off = min(j * 8u + s + 4, nwalk - 1u) * 64u + l;
+#pragma unroll
+        for (int r = 0; r < RT; ++r) A[s & 3][r] = Ap[r][off];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      // the super-block's (or its half's) d, min term and 2^-e
+      if (s == 7 || (SG == 2 && s == 3)) {
+        const int hf = SG == 2 ? s >> 2 : 0;
+        const uint8_t* vb = vaux + (j & 1u) * VAUX_LDS;
+        const uint8_t* wb = waux + (QT == 2 ? 0u : ((j & 1u) * 4u + w) * WAUX_LDS);
+        float fs[4];
+        h8 bm[QT == 0 ? 4 : 1];
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-          const h8 bh = *(const h8*)(base + t * 4096), bl = *(const h8*)(base + t * 4096 + 1024);
-#pragma unroll
-          for (int r = 0; r < RT; ++r)
-            C[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, A[r]), bh,
-                                                             first ? f4{0.f, 0.f, 0.f, 0.f} : C[r][t], 0, 0, 0);
-#pragma unroll
-          for (int r = 0; r < RT; ++r)
-            C[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, A[r]), bl, C[r][t], 0, 0, 0);
+          fs[t] = *(const float*)(vb + (PfOps::SCALE - PfOps::SUMS) + t * 128 + hf * 64 + c * 4);
+          if constexpr (QT == 0) bm[t] = *(const h8*)(vb + t * 1024 + l * 16);
         }
 #pragma unroll
-        for (int r = 0; r < RT; ++r) A[r] = An[r];
-        // the super-block's (or its half's) d, min term and 2^-e
-        if (s == 7 || (SG == 2 && s == 3)) {
-          const int hf = SG == 2 ? s >> 2 : 0;
-          float fs[4];
-          h8 bm[QT == 0 ? 4 : 1];
+        for (int r = 0; r < RT; ++r) {
+          if constexpr (QT == 2) {
 #pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            fs[t] = *(const float*)(Bsb + PfOps::SCALE + t * 128 + hf * 64 + c * 4);
-            if constexpr (QT == 0) bm[t] = *(const h8*)(Bsb + PfOps::SUMS + t * 1024 + l * 16);
-          }
+            for (int t = 0; t < 4; ++t)
 #pragma unroll
-          for (int r = 0; r < RT; ++r) {
-            if constexpr (QT == 2) {
+              for (int i = 0; i < 4; ++i) acc[r][t][i] += fs[t] * C[r][t][i];
+          } else {
+            const uint8_t* xr = wb + r * Aux<QT>::BYTES;
+            const f4 d = *(const f4*)(xr + 16 * q);
+            f4 dm = f4{0.f, 0.f, 0.f, 0.f};
+            h8 am = h8{};
+            if constexpr (QT == 0) {
+              dm = *(const f4*)(xr + Aux<0>::DM + 16 * q);
+              const h2 mn = *(const h2*)(xr + Aux<0>::MN + 4 * l);
+              // slots 8q .. 8q + 7 are sub-blocks 2q and 2q + 1: a half is two lane groups
+              if (SG == 1 || (q >> 1) == hf) am = h8{mn.x, mn.x, mn.x, mn.x, mn.y, mn.y, mn.y, mn.y};
+            }
 #pragma unroll
-              for (int t = 0; t < 4; ++t)
+            for (int t = 0; t < 4; ++t) {
+              f4 cm = f4{0.f, 0.f, 0.f, 0.f};
+              if constexpr (QT == 0) cm = __builtin_amdgcn_mfma_f32_16x16x32_f16(am, bm[t], cm, 0, 0, 0);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) acc[r][t][i] += fs[t] * C[r][t][i];
-            } else {
-              const f4 d = *(const f4*)(a.w.D + drow + rt[r] * 16u + 4u * q);
-              f4 dm = f4{0.f, 0.f, 0.f, 0.f};
-              h8 am = h8{};
-              if constexpr (QT == 0) {
-                dm = *(const f4*)(a.w.DM + drow + rt[r] * 16u + 4u * q);
-                am = *(const h8*)(a.w.Mn + ((size_t)rt[r] * a.nsb + sb0 + j) * 1024u + l * 16);
-                // slots 8q .. 8q + 7 are sub-blocks 2q and 2q + 1: a half is two lane groups
-                if (SG == 2 && (q >> 1) != hf) am = h8{};
-              }
-#pragma unroll
-              for (int t = 0; t < 4; ++t) {
-                f4 cm = f4{0.f, 0.f, 0.f, 0.f};
-                if constexpr (QT == 0) cm = __builtin_amdgcn_mfma_f32_16x16x32_f16(am, bm[t], cm, 0, 0, 0);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                  if constexpr (QT == 0) acc[r][t][i] += fs[t] * (d[i] * C[r][t][i] - dm[i] * cm[i]);
-                  else acc[r][t][i] += fs[t] * d[i] * C[r][t][i];
-                }
+              for (int i = 0; i < 4; ++i) {
+                if constexpr (QT == 0) acc[r][t][i] += fs[t] * (d[i] * C[r][t][i] - dm[i] * cm[i]);
+                else acc[r][t][i] += fs[t] * d[i] * C[r][t][i];
               }
             }
           }
         }
       }
-      // one barrier a step: the buffer written here was last read in the
-      // step before, which every wave had left at that step's barrier
-      put((p + 1) & 1);
-      __syncthreads();
     }
   }
+  wait_vmcnt<0>();  // no load into this workgroup's LDS outlives it
+  lds_barrier();
 
   // ---- outputs: lane (q, c) holds rows 4q + i of a row tile, vector 64 tt + 16t + c ----
   if constexpr (MODE == 0) {
@@ -275,7 +344,7 @@ __global__ __launch_bounds__(NT, 2) void pf_gemm_kernel(PfArgs a) {
     }
   } else {
     f4 y[2][4];
-    float* mx = (float*)lds[0];  // [wave][t][16]: the walk's last barrier ended every read of the buffers
+    float* mx = (float*)b0;  // [wave][t][16]
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const bool live = tt * 64u + 16u * t + c < a.T;
@@ -335,24 +404,10 @@ __global__ __launch_bounds__(NT, 2) void pf_gemm_kernel(PfArgs a) {
 // host
 // ---------------------------------------------------------------------------
 
-size_t up256(size_t n) { return (n + 255) / 256 * 256; }
-
-struct WLayout {
-  size_t a, mn, d, dm, total;
-};
-WLayout w_layout(int wtype, uint32_t rtn, uint32_t K) {
-  WLayout o{};
-  const size_t nsb = K / 256;
-  o.a = 0;
-  size_t at = (size_t)rtn * (K / 32) * 1024;
-  o.mn = at;
-  if (wtype == 0) at += (size_t)rtn * nsb * 1024;
-  o.d = at;
-  if (wtype != 2) at = up256(at + nsb * rtn * 16 * sizeof(float));
-  o.dm = at;
-  if (wtype == 0) at = up256(at + nsb * rtn * 16 * sizeof(float));
-  o.total = at;
-  return o;
+// Bytes of a launch's unpacked weights: the operands, then the Aux values.
+size_t w_operands(uint32_t rtn, uint32_t K) { return (size_t)rtn * (K / 32) * 1024; }
+size_t w_bytes(int wtype, uint32_t rtn, uint32_t K) {
+  return w_operands(rtn, K) + (size_t)rtn * (K / 256) * aux_bytes(wtype);
 }
 
 int check_pf(const char* fn, int wtype, const void* const* weights, const uint32_t* rows, int nseg, uint32_t N,
@@ -370,12 +425,12 @@ int check_pf(const char* fn, int wtype, const void* const* weights, const uint32
                "%s: weights misaligned (Q4_K and f16 16 B, Q6_K 4 B)", fn);
     rtn += ceil_div(rows[i], 16);
   }
-  G4_REQUIRE(wops_bytes >= w_layout(wtype, rtn, N).total, "%s: weight operand buffer of %zu bytes, %zu needed", fn,
-             wops_bytes, w_layout(wtype, rtn, N).total);
+  G4_REQUIRE(wops_bytes >= w_bytes(wtype, rtn, N), "%s: weight operand buffer of %zu bytes, %zu needed", fn,
+             wops_bytes, w_bytes(wtype, rtn, N));
   return G4_OK;
 }
 
-PfArgs pf_args(int wtype, const void* const* weights, float* const* outputs, const uint32_t* rows, int nseg, uint32_t N,
+PfArgs pf_args(const void* const* weights, float* const* outputs, const uint32_t* rows, int nseg, uint32_t N,
                const void* ops, uint32_t T, void* wops, uint32_t rtn) {
   PfArgs a{};
   uint32_t rt0 = 0;
@@ -384,9 +439,7 @@ PfArgs pf_args(int wtype, const void* const* weights, float* const* outputs, con
     rt0 += ceil_div(rows[i], 16);
   }
   a.n = nseg;
-  const WLayout o = w_layout(wtype, rtn, N);
-  uint8_t* b = (uint8_t*)wops;
-  a.w = PfWeights{b + o.a, b + o.mn, (float*)(b + o.d), (float*)(b + o.dm)};
+  a.w = PfWeights{(uint8_t*)wops, (uint8_t*)wops + w_operands(rtn, N)};
   a.rtn = rtn;
   a.K = N;
   a.nsb = N / 256;
@@ -412,8 +465,10 @@ int gemm_qt(g4_ctx* ctx, int wtype, PfArgs a, uint32_t groups) {
   a.groups = groups;
   a.items = groups * a.ksplit * a.ntt;
   const dim3 grid(ceil_div(a.items, 8) * 8);
-  if (wtype == 0) hipLaunchKernelGGL((pf_gemm_kernel<0, RT, MODE, SG>), grid, dim3(NT), 0, ctx->stream, a);
-  else if (wtype == 1) hipLaunchKernelGGL((pf_gemm_kernel<1, RT, MODE, SG>), grid, dim3(NT), 0, ctx->stream, a);
+  if (wtype == 0) {
+    if constexpr (RT == 4 && SG == 2) return G4_ERR_UNSUPPORTED;  // (pick_plan)
+    else hipLaunchKernelGGL((pf_gemm_kernel<0, RT, MODE, SG>), grid, dim3(NT), 0, ctx->stream, a);
+  } else if (wtype == 1) hipLaunchKernelGGL((pf_gemm_kernel<1, RT, MODE, SG>), grid, dim3(NT), 0, ctx->stream, a);
   else hipLaunchKernelGGL((pf_gemm_kernel<2, RT, MODE, SG>), grid, dim3(NT), 0, ctx->stream, a);
   G4_LAUNCHED(ctx, "prefill_gemm");
   return G4_OK;
@@ -428,11 +483,11 @@ struct Plan {
   int rt;
   uint32_t ks;
 };
-Plan pick_plan(const g4_ctx* ctx, const PfArgs& a, uint32_t max_split) {
+Plan pick_plan(const g4_ctx* ctx, const PfArgs& a, uint32_t max_split, bool two_only) {
   const uint32_t slots = 2u * (uint32_t)(ctx->num_cus > 0 ? ctx->num_cus : 256);
-  Plan best{4, 1};
+  Plan best{2, 1};
   double bt = 1e30;
-  for (int rt = 4; rt >= 2; rt -= 2)
+  for (int rt = two_only ? 2 : 4; rt >= 2; rt -= 2)
     for (uint32_t ks = 1; ks <= a.nsb && ks <= max_split; ++ks) {
       if (a.nsb % ks) continue;
       const uint32_t items = ceil_div(a.rtn, 4u * rt) * a.ntt * ks, rounds = ceil_div(items, slots);
@@ -457,7 +512,7 @@ int g4_prefillWeightBytes(int wtype, uint32_t rows, uint32_t N, size_t* bytes) {
   G4_REQUIRE(bytes && wtype >= 0 && wtype <= 2 && rows > 0 && rows <= (1u << 22) && N >= 256 && N % 256 == 0 &&
                  N <= 65536,
              "g4_prefillWeightBytes: bad shape");
-  *bytes = w_layout(wtype, ceil_div(rows, 16), N).total;
+  *bytes = w_bytes(wtype, ceil_div(rows, 16), N);
   return G4_OK;
 }
 
@@ -478,10 +533,12 @@ int g4_prefillMatmul(g4_ctx* ctx, int wtype, const void* const* weights, float* 
   G4_REQUIRE(outputs && ksplit && max_ksplit >= 1, "g4_prefillMatmul: null outputs, null ksplit or max_ksplit 0");
   for (int i = 0; i < nseg; ++i)
     G4_REQUIRE(outputs[i] && ((uintptr_t)outputs[i] & 15) == 0, "g4_prefillMatmul: output %d null or misaligned", i);
-  PfArgs a = pf_args(wtype, weights, outputs, rows, nseg, N, ops, vectors, wops, rtn);
+  PfArgs a = pf_args(weights, outputs, rows, nseg, N, ops, vectors, wops, rtn);
   rc = unpack(ctx, wtype, a);
   if (rc) return rc;
-  const Plan p = pick_plan(ctx, a, max_ksplit);
+  // (Q4_K over a product's operands: with four row tiles the two scale groups'
+  // min products spill 289 registers)
+  const Plan p = pick_plan(ctx, a, max_ksplit, wtype == 0 && product_ops);
   a.ksplit = p.ks;
   a.kc = a.nsb / p.ks;
   *ksplit = p.ks;
@@ -500,7 +557,7 @@ int g4_prefillGateUp(g4_ctx* ctx, int wtype, const void* w_gate, const void* w_u
   if (rc) return rc;
   G4_REQUIRE(M % 256 == 0, "g4_prefillGateUp: M=%u must be a multiple of 256", M);
   G4_REQUIRE(product_ops && ((uintptr_t)product_ops & 15) == 0, "g4_prefillGateUp: product operands null or misaligned");
-  PfArgs a = pf_args(wtype, weights, nullptr, rows, 2, N, ops, vectors, wops, rtn);
+  PfArgs a = pf_args(weights, nullptr, rows, 2, N, ops, vectors, wops, rtn);
   a.ops_out = (uint8_t*)product_ops;
   rc = unpack(ctx, wtype, a);
   if (rc) return rc;
