@@ -55,6 +55,7 @@ using g4d::pad_batch;
 // per-vector prologue: out = x' where x = sum of the nparts partials and
 //   PRO 0: x' = x;  PRO 1: x' = x * w1 / rms(x);
 //   PRO 2: h = residual + x * w1 / rms(x) (written to h_out), x' = h * w2 / rms(h)
+//   PRO 3: x' = gelu(x) * mul
 // (src/engine.ts:1545 rmsNorm, :1606-1607 fusedNormAdd + rmsNorm)
 // ---------------------------------------------------------------------------
 struct BPrepArgs {
@@ -70,7 +71,8 @@ struct BPrepArgs {
   uint8_t* ops;  // optional: operand blocks [K/256][Ops::bytes(ntv)]
   int ntv;
   const uint16_t* scale;  // mode 2: h = (residual + norm(x)) * f16 scale (NULL: 1)
-  bool prefill;           // ops are the prefill matmul's [B / 64][K/256][PfOps::BYTES]
+  const float* mul;       // PRO 3: x' = gelu(x) * mul[v * mul_stride + k]
+  uint32_t mul_stride;
 };
 
 __device__ __forceinline__ float4 mulw(float4 x, uint2 w, float s) {
@@ -84,7 +86,10 @@ __device__ __forceinline__ float4 add4(float4 a, float4 b) {
 
 // One workgroup per vector; thread t holds the float4s at 4t + 1024p. The
 // partials are read PMAX at a time, all loads of a pass issued together.
-template <int BPR, int PRO>
+// PF: the prefill pass's form: out may be null, ops are the prefill matmul's
+// [B / 64][K/256][PfOps::BYTES] (as a run-time choice it cost the decode
+// step's launches 0.2 us each).
+template <int BPR, int PRO, bool PF = false>
 __global__ __launch_bounds__(PNT) void bprep_kernel(BPrepArgs a) {
   constexpr int K = BPR * 256;
   constexpr int XP = (K + 4 * PNT - 1) / (4 * PNT);
@@ -93,7 +98,9 @@ __global__ __launch_bounds__(PNT) void bprep_kernel(BPrepArgs a) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const size_t vstride = (size_t)a.B * K;
   float4 x[XP], r[PRO == 2 ? XP : 1];
-  uint2 w1[PRO >= 1 ? XP : 1], w2[PRO == 2 ? XP : 1];
+  constexpr bool NORM = PRO == 1 || PRO == 2;
+  uint2 w1[NORM ? XP : 1], w2[PRO == 2 ? XP : 1];
+  float4 ml[PRO == 3 ? XP : 1];
   // (w2 read unconditionally, from w1 when there is none: a load under a
   // branch is waited for where the branch joins, before the partials below
   // are even requested)
@@ -104,7 +111,8 @@ __global__ __launch_bounds__(PNT) void bprep_kernel(BPrepArgs a) {
   for (int p = 0; p < XP; ++p) {
     const int f = 4 * tid + 4 * PNT * p, fc = f < K ? f : 0;
     x[p] = *(const float4*)(a.x + (size_t)v * K + fc);
-    if constexpr (PRO >= 1) w1[p] = *(const uint2*)(a.w1 + fc);
+    if constexpr (NORM) w1[p] = *(const uint2*)(a.w1 + fc);
+    if constexpr (PRO == 3) ml[p] = *(const float4*)(a.mul + (size_t)v * a.mul_stride + fc);
     if constexpr (PRO == 2) {
       r[p] = *(const float4*)(a.residual + (size_t)v * K + fc);
       w2[p] = *(const uint2*)(w2p + fc);
@@ -127,7 +135,13 @@ __global__ __launch_bounds__(PNT) void bprep_kernel(BPrepArgs a) {
 #pragma unroll
         for (int p = 0; p < XP; ++p) x[p] = add4(x[p], t[i][p]);
   }
-  if constexpr (PRO >= 1) {
+  if constexpr (PRO == 3) {
+#pragma unroll
+    for (int p = 0; p < XP; ++p)
+      x[p] = make_float4(g4d::gelu_tanh(x[p].x) * ml[p].x, g4d::gelu_tanh(x[p].y) * ml[p].y,
+                         g4d::gelu_tanh(x[p].z) * ml[p].z, g4d::gelu_tanh(x[p].w) * ml[p].w);
+  }
+  if constexpr (NORM) {
     float ss = 0.f;
 #pragma unroll
     for (int p = 0; p < XP; ++p) ss += (4 * tid + 4 * PNT * p < K) ? sq4(x[p]) : 0.f;
@@ -167,13 +181,13 @@ __global__ __launch_bounds__(PNT) void bprep_kernel(BPrepArgs a) {
 #pragma unroll
   for (int p = 0; p < XP; ++p) {
     const int f = 4 * tid + 4 * PNT * p;
-    if (a.out && f < K) *(float4*)(a.out + (size_t)v * K + f) = x[p];
+    if ((!PF || a.out) && f < K) *(float4*)(a.out + (size_t)v * K + f) = x[p];
   }
   if (!a.ops) return;
   // operand blocks: wave w of pass p holds super-block 4p + w, lanes 8j .. 8j+7 its sub-block j
-  const uint32_t sblk = a.prefill ? g4d::PfOps::BYTES : Ops::bytes(a.ntv);
-  uint8_t* const ops = a.ops + (a.prefill ? (size_t)(v / 64) * BPR * sblk : (size_t)0);
-  const uint32_t t = a.prefill ? v / 16 % 4 : v / 16, c = v % 16;
+  const uint32_t sblk = PF ? g4d::PfOps::BYTES : Ops::bytes(a.ntv);
+  uint8_t* const ops = a.ops + (PF ? (size_t)(v / 64) * BPR * sblk : (size_t)0);
+  const uint32_t t = PF ? v / 16 % 4 : v / 16, c = v % 16;
   const int s = lane >> 3;        // sub-block within the super-block
   const int kk = (lane & 7) * 4;  // first element within the sub-block
   const int q = kk >> 3;          // 8-element group
@@ -208,10 +222,11 @@ __global__ __launch_bounds__(PNT) void bprep_kernel(BPrepArgs a) {
       const float r1 = sum - (float)p0;
       const _Float16 p1 = (_Float16)r1;
       const _Float16 p2 = (_Float16)(r1 - (float)p1);
-      *(uint2*)(base + Ops::sums_off(a.ntv) + t * 1024 + (c + 16u * (uint32_t)(s >> 1)) * 16 + (s & 1) * 8) =
+      *(uint2*)(base + (PF ? g4d::PfOps::SUMS : Ops::sums_off(a.ntv)) + t * 1024 +
+                (c + 16u * (uint32_t)(s >> 1)) * 16 + (s & 1) * 8) =
           make_uint2(pack_h2(p0, p1), pack_h2(p2, (_Float16)0.f));
     }
-    if (a.prefill) {  // (both halves of the super-block share the scale)
+    if constexpr (PF) {  // (both halves of the super-block share the scale)
       if (lane < 2) *(float*)(base + g4d::PfOps::SCALE + t * 128 + lane * 64 + c * 4) = ldexpf(1.0f, -k);
     } else if (lane == 0) {
       *(float*)(base + Ops::scale_off(a.ntv) + t * 64 + c * 4) = ldexpf(1.0f, -k);
@@ -760,32 +775,32 @@ __global__ __launch_bounds__(64) void operand_check_kernel(const uint8_t* W, uin
 // host
 // ---------------------------------------------------------------------------
 
-template <int BPR>
+template <int BPR, bool PF>
 int bprep_bpr(g4_ctx* ctx, int pro, const BPrepArgs& p) {
   const dim3 grid(p.B);
-  if (pro == 0) hipLaunchKernelGGL((bprep_kernel<BPR, 0>), grid, dim3(PNT), 0, ctx->stream, p);
-  else if (pro == 1) hipLaunchKernelGGL((bprep_kernel<BPR, 1>), grid, dim3(PNT), 0, ctx->stream, p);
-  else hipLaunchKernelGGL((bprep_kernel<BPR, 2>), grid, dim3(PNT), 0, ctx->stream, p);
+  if (pro == 0) hipLaunchKernelGGL((bprep_kernel<BPR, 0, PF>), grid, dim3(PNT), 0, ctx->stream, p);
+  else if (pro == 1) hipLaunchKernelGGL((bprep_kernel<BPR, 1, PF>), grid, dim3(PNT), 0, ctx->stream, p);
+  else hipLaunchKernelGGL((bprep_kernel<BPR, 2, PF>), grid, dim3(PNT), 0, ctx->stream, p);
   G4_LAUNCHED(ctx, "batch_prep");
   return G4_OK;
 }
 
+template <bool PF = false>
 int bprep_launch(g4_ctx* ctx, uint32_t N, int pro, const BPrepArgs& p) {
   switch (N / 256) {
-    case 6: return bprep_bpr<6>(ctx, pro, p);
-    case 8: return bprep_bpr<8>(ctx, pro, p);
-    case 16:  // (operands of a head-dim-512 layer's attention output)
-      if (pro) return G4_ERR_UNSUPPORTED;
-      hipLaunchKernelGGL((bprep_kernel<16, 0>), dim3(p.B), dim3(PNT), 0, ctx->stream, p);
-      G4_LAUNCHED(ctx, "batch_prep");
-      return G4_OK;
-    case 1:  // (of a per-layer embedding's gated input)
-      if (pro) return G4_ERR_UNSUPPORTED;
-      hipLaunchKernelGGL((bprep_kernel<1, 0>), dim3(p.B), dim3(PNT), 0, ctx->stream, p);
-      G4_LAUNCHED(ctx, "batch_prep");
-      return G4_OK;
-    default: return G4_ERR_UNSUPPORTED;
+    case 6: return bprep_bpr<6, PF>(ctx, pro, p);
+    case 8: return bprep_bpr<8, PF>(ctx, pro, p);
+    default: break;
   }
+  if constexpr (PF) {
+    if (pro == 0 && (N == 4096 || N == 256)) {  // a head-dim-512 layer's attention output; a gated embedding
+      if (N == 4096) hipLaunchKernelGGL((bprep_kernel<16, 0, true>), dim3(p.B), dim3(PNT), 0, ctx->stream, p);
+      else hipLaunchKernelGGL((bprep_kernel<1, 0, true>), dim3(p.B), dim3(64), 0, ctx->stream, p);
+      G4_LAUNCHED(ctx, "batch_prep");
+      return G4_OK;
+    }
+  }
+  return G4_ERR_UNSUPPORTED;
 }
 
 bool mm_supported(uint32_t bpr) {
@@ -1151,8 +1166,31 @@ int g4_prefillPrep(g4_ctx* ctx, const float* x, uint32_t nparts, const uint16_t*
              "g4_prefillPrep: buffers must be 16-byte aligned");
   G4_REQUIRE((((uintptr_t)w1 | (uintptr_t)w2) & 7) == 0, "g4_prefillPrep: norm weights must be 8-byte aligned");
   const int pro = !w1 ? 0 : (residual ? 2 : 1);
-  const BPrepArgs p{x, nparts, vectors, w1, residual, w2, h_out, out, eps, (uint8_t*)ops, 4, out_scale, true};
-  return bprep_launch(ctx, N, pro, p);
+  const BPrepArgs p{x, nparts, vectors, w1, residual, w2, h_out, out, eps, (uint8_t*)ops, 4, out_scale};
+  return bprep_launch<true>(ctx, N, pro, p);
+}
+
+int g4_prefillPleGated(g4_ctx* ctx, const float* gate, uint32_t nparts, const float* ple_inputs, uint32_t stride,
+                       uint32_t layer_offset, float* out, void* ops, uint32_t vectors) {
+  G4_ENTER(ctx);
+  G4_REQUIRE(gate && nparts >= 1 && ple_inputs && (out || ops), "g4_prefillPleGated: null buffer or no parts");
+  G4_REQUIRE(vectors >= 1 && vectors <= 65535, "g4_prefillPleGated: %u vectors outside 1..65535", vectors);
+  G4_REQUIRE(stride % 4 == 0 && layer_offset % 4 == 0 && (uint64_t)layer_offset + 256 <= stride,
+             "g4_prefillPleGated: slice %u of rows of %u", layer_offset, stride);
+  G4_REQUIRE((((uintptr_t)gate | (uintptr_t)ple_inputs | (uintptr_t)out | (uintptr_t)ops) & 15) == 0,
+             "g4_prefillPleGated: buffers must be 16-byte aligned");
+  BPrepArgs p{};
+  p.x = gate;
+  p.nparts = nparts;
+  p.B = vectors;
+  p.out = out;
+  p.ops = (uint8_t*)ops;
+  p.ntv = 4;
+  p.mul = ple_inputs + layer_offset;
+  p.mul_stride = stride;
+  hipLaunchKernelGGL((bprep_kernel<1, 3, true>), dim3(vectors), dim3(64), 0, ctx->stream, p);
+  G4_LAUNCHED(ctx, "prefill_ple_gated");
+  return G4_OK;
 }
 
 int g4_matmulSegmentsBatchPartial(g4_ctx* ctx, int wtype, const float* x, const void* ops,

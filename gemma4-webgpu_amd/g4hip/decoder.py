@@ -1206,12 +1206,15 @@ class BatchDecoder(_SyntheticModel):
             for ms, rows, n in [([m for m, _ in qkv], [r for _, r in qkv], H), (["wo"], [H], Q),
                                 (["wgate", "wup"], [I, I], H), (["wdown"], [H], I)]:
                 need = max([need] + [c.prefill_weight_bytes(L.qt[m], rows, n) for m in ms])
+        if s.ple_dim:
+            need = max(need, *(c.prefill_weight_bytes("f16", [rows], n) for rows, n in
+                               [(s.n_layers * s.ple_dim, H), (s.ple_dim, H), (H, s.ple_dim)]))
         w["wops"] = c.empty(need, np.uint8)
         w["attn_ws"] = c.empty(ws, np.uint8)
         if s.ple_dim:
             LD = s.n_layers * s.ple_dim
             w.update(hidden3=c.empty(R * H, f32), ple_projected=c.empty(R * LD, f32), ple_inputs=c.empty(R * LD, f32),
-                     ple_gated=c.empty(R * s.ple_dim, f32), ple_out=c.empty(R * H, f32))
+                     ple_gate=c.empty(R * H, f32), pops=c.empty(ob(s.ple_dim, R), np.uint8), ple_out=c.empty(R * H, f32))
 
     def _prefill_wide(self, toks, start: int, pad: int, sample: str) -> None:
         """The prompt (its last token repeated `pad` times to whole chunks of
@@ -1246,7 +1249,8 @@ class BatchDecoder(_SyntheticModel):
         c.embeddingLookupBatch(self.embedding, s.vocab, w["hidden"], H, tokens, n)
         if s.ple_dim:
             LD = s.n_layers * s.ple_dim
-            c.matmulF16(w["hidden"], self.ple_model_proj, w["ple_projected"], LD, H, n)
+            c.prefillPrep(w["hidden"], 1, None, None, None, None, None, None, H, n, s.eps, ops=w["xops"])
+            c.prefillMatmul("f16", [self.ple_model_proj], [w["ple_projected"]], [LD], H, w["xops"], n, wops)
             c.pleStage1Fuse(w["ple_projected"], self.ple_proj_norm, self.ple_table, s.vocab, w["ple_inputs"],
                             s.n_layers, s.ple_dim, s.eps, tokens_dev=tokens, count=n)
         max_ks = max(1, self.wide_parts // (n * H))
@@ -1290,10 +1294,10 @@ class BatchDecoder(_SyntheticModel):
             if s.ple_dim:
                 D = s.ple_dim
                 c.prefillPrep(w["parts"], nd, L.post_ffn_norm, w["hidden2"], None, None, w["hidden3"], None, H, n,
-                              s.eps)
-                c.pleGate(w["hidden3"], None, None, None, L.ple_gate, w["ple_inputs"], s.n_layers * D, il * D,
-                          w["ple_gated"], D, H, s.eps, batch=n)
-                c.matmulF16(w["ple_gated"], L.ple_proj, w["ple_out"], H, D, n)
+                              s.eps, ops=w["xops"])
+                ng = c.prefillMatmul("f16", [L.ple_gate], [w["ple_gate"]], [D], H, w["xops"], n, wops, H // 256)
+                c.prefillPleGated(w["ple_gate"], ng, w["ple_inputs"], s.n_layers * D, il * D, None, n, ops=w["pops"])
+                c.prefillMatmul("f16", [L.ple_proj], [w["ple_out"]], [H], D, w["pops"], n, wops)
 
     def capture(self, sample: str = "argmax"):
         """The step as a HIP graph; each replay appends one token per sequence."""

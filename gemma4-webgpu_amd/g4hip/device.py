@@ -365,6 +365,12 @@ class Context:
         check(lib().g4_prefillGateUp(self.h, PREFILL_TYPES[wtype], _p(w_gate), _p(w_up), _p(ops), _p(product_ops),
                                      M, N, vectors, _p(wops), wops.nbytes))
 
+    def prefillPleGated(self, gate: Ptr, nparts: int, ple_inputs: Ptr, stride: int, layer_offset: int, out: Ptr,
+                        vectors: int, ops: Ptr = None) -> None:
+        """gelu(gate) * ple_inputs' slice of every vector, as values and / or proj's operand blocks."""
+        check(lib().g4_prefillPleGated(self.h, _p(gate), nparts, _p(ple_inputs), stride, layer_offset, _p(out),
+                                       _p(ops), vectors))
+
     def prefillAttnPrologue(self, q_raw: Ptr, k_raw: Ptr, v_raw: Ptr, q_norm_w: Ptr, k_norm_w: Ptr, rope_freqs: Ptr,
                             q_out: Ptr, k_pool: Ptr, v_pool: Ptr, page_table: Ptr, lens: Ptr, params,
                             rope_cs: Ptr = None, rope_rows: int = 0) -> None:

@@ -724,6 +724,12 @@ int g4_prefillMatmul(g4_ctx* ctx, int wtype, const void* const* weights, float* 
 int g4_prefillGateUp(g4_ctx* ctx, int wtype, const void* w_gate, const void* w_up, const void* ops,
                      void* product_ops, uint32_t M, uint32_t N, uint32_t vectors, void* wops,
                      size_t wops_bytes);
+/* The per-layer-embedding gate of a pass (g4_pleGate's epilogue,
+ * src/engine.ts:1608-1616): gelu(sum of the parts of gate [nparts][vectors][256])
+ * * ple_inputs [vectors][stride] at layer_offset, as `out` [vectors][256]
+ * and / or the operand blocks of proj (g4_prefillOperandBytes(256, vectors)). */
+int g4_prefillPleGated(g4_ctx* ctx, const float* gate, uint32_t nparts, const float* ple_inputs,
+                       uint32_t stride, uint32_t layer_offset, float* out, void* ops, uint32_t vectors);
 /* The attention of p.num_seqs rows (1..65535) of one sequence over one page
  * list (page_table [p.max_pages]; every row may read every position below
  * its length, so appending all rows first makes the pass causal).

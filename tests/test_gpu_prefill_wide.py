@@ -104,6 +104,25 @@ def test_prefill_ffn(ctx, wtype, down):
         assert O.rel_l2(got[v], want[v]) <= bar, v
 
 
+@pytest.mark.parametrize("T,parts", [(1, 1), (65, 3)])
+def test_prefill_ple_gated(ctx, T, parts):
+    """gelu(sum of the parts) * the layer's slice: the values, and their operand blocks through a product."""
+    D, stride, off = 256, 768, 512
+    gate = O.gen_normal_f32(31, parts * T * D, 0.0, 1.0).reshape(parts, T, D)
+    ple = O.gen_normal_f32(32, T * stride).reshape(T, stride)
+    out, ops = ctx.zeros(T * D, np.float32), ctx.alloc(ctx.prefill_operand_bytes(D, T))
+    ctx.prefillPleGated(ctx.from_numpy(gate), parts, ctx.from_numpy(ple), stride, off, out, T, ops=ops)
+    got = out.download(np.float32).reshape(T, D)
+    a = gate.astype(np.float64).sum(0)
+    t = np.clip(0.7978845608028654 * a * (1 + 0.044715 * a * a), -15, 15)
+    want = 0.5 * a * (1 + np.tanh(t)) * ple[:, off:off + D]
+    assert O.rel_l2(got, want) <= 2e-6
+    wb, w = _weights("f16", 33, 48, D)
+    y, wops = ctx.zeros(T * 48, np.float32), ctx.alloc(ctx.prefill_weight_bytes("f16", [48], D))
+    ctx.prefillMatmul("f16", [ctx.from_numpy(wb)], [y], [48], D, ops, T, wops)
+    assert O.rel_l2(y.download(np.float32).reshape(T, 48), got.astype(np.float64) @ w.T) <= BAR["f16"]
+
+
 @pytest.mark.parametrize("layout,B,T,start", [
     ("uniform", 64, 65, 0),      # one row past a chunk
     ("uniform", 64, 300, 600),   # past the window
