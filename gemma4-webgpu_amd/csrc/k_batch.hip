@@ -847,7 +847,10 @@ void mm_launch_kg(g4_ctx* ctx, const MmArgs& a, uint32_t groups, bool unroll) {
 }
 
 // K groups per workgroup: the gate/up pair (one workgroup per CU, a whole K
-// each) takes two; launches of about one workgroup per CU or fewer take
+// each) takes two, but one where 64-vector operands let a CU hold two
+// single-group workgroups and the launch has more than one per CU (FFN 12288:
+// 384 workgroups, 38.2 -> 32.4 us: two groups' 140 KB leave one workgroup per
+// CU and the second half of the launch waits for the first); launches of about one workgroup per CU or fewer take
 // three where kc allows (a wave per SIMD leaves the latency of every MFMA
 // and operand read exposed; 12 waves share one CU's work three ways).
 //
@@ -860,7 +863,7 @@ template <int QT, int BPR, int NTV, int MODE, int OPK>
 int mm_launch(g4_ctx* ctx, const MmArgs& a, uint32_t groups) {
   const uint32_t cus = (uint32_t)(ctx->num_cus > 0 ? ctx->num_cus : 256);
   const bool few = groups * a.ksplit <= cus;
-  if (MODE == 1 && a.kc % 2 == 0) {
+  if (MODE == 1 && a.kc % 2 == 0 && (NTV <= 2 || few)) {
     if constexpr (MODE == 1) mm_launch_kg<QT, BPR, NTV, MODE, OPK, 2>(ctx, a, groups, few);
   } else if (NTV <= 2 && few && a.kc % 3 == 0 && (a.kc == 3 || a.kc == 6)) {
     if constexpr (NTV <= 2) mm_launch_kg<QT, BPR, NTV, MODE, OPK, 3>(ctx, a, groups, true);
