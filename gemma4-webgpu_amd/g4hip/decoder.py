@@ -969,7 +969,8 @@ class BatchDecoder(_SyntheticModel):
                 total += n * 2 * s.kv_dim_of(il) * 2
         return total
 
-    def step(self, sample: str = "argmax", probe=None, head: bool = True) -> None:
+    def step(self, sample: str = "argmax", probe=None, head: bool = True,
+             rows: Optional[int] = None) -> None:
         """One token for every sequence. Per layer:
           1. [sum of the previous down chunks -> post-FFN norm-add ->] attn rmsNorm
           2. q/k/v projections (split-K partial sums)
@@ -993,8 +994,10 @@ class BatchDecoder(_SyntheticModel):
 
         head=False stops after the layers (no final norm, LM head or sample):
         a prefill chunk whose logits nobody reads (the reference's prefill
-        forwards run no LM head either, src/engine.ts:1896-1900)."""
-        c, s, B = self.ctx, self.s, self.B
+        forwards run no LM head either, src/engine.ts:1896-1900). rows: only
+        the first rows take the step (a prefill chunk's, the rest spare);
+        every length advances."""
+        c, s, B = self.ctx, self.s, rows or self.B
         H = s.hidden
         if self.embedding is not None:
             c.embeddingLookupBatch(self.embedding, s.vocab, self.hidden, H, self.tokens, B)
@@ -1003,7 +1006,7 @@ class BatchDecoder(_SyntheticModel):
             c.matmulF16(self.hidden, self.ple_model_proj, self.ple_projected, LD, H, B)
             c.pleStage1Fuse(self.ple_projected, self.ple_proj_norm, self.ple_table, s.vocab, self.ple_inputs,
                             s.n_layers, s.ple_dim, s.eps, tokens_dev=self.tokens, count=B)
-        c.advanceSeqLens(self.seq_lens, B, 1)
+        c.advanceSeqLens(self.seq_lens, self.B, 1)
         nd = 0
         for il, L in enumerate(self.layers):
             Q, KV, I = s.q_dim_of(il), s.kv_dim_of(il), s.ffn_of(il)
@@ -1045,13 +1048,14 @@ class BatchDecoder(_SyntheticModel):
             else:
                 c.pagedAttnPrologue(self.q_parts, self.k_parts if prod else None, self.v_parts if prod else None, nq,
                                     L.q_norm, L.k_norm, self.rope_freqs, self.q, L.k_cache if prod else None,
-                                    L.v_cache if prod else None, self.page_table, self.seq_lens, self.pro_params[il],
+                                    L.v_cache if prod else None, self.page_table, self.seq_lens,
+                                    self._for_rows(self.pro_params[il], B),
                                     self.rope_cs[s.is_global(il)], self.rope_rows)
                 c.pagedAttnDecode(self.q, L.k_cache, L.v_cache, self.page_table, self.seq_lens, self.attn,
-                                  self.attn_params[il], self.attn_ws, ops=ops)
+                                  self._for_rows(self.attn_params[il], B), self.attn_ws, ops=ops)
             if probe:
                 probe("attn", il, 0)
-            no = self._mm_batch(L.qt["wo"], self.attn, L.wo, self.o_parts, H, Q, self.ks_q, ops)
+            no = self._mm_batch(L.qt["wo"], self.attn, L.wo, self.o_parts, H, Q, self.ks_q, ops, B)
             c.batchPrep(self.o_parts, no, L.post_attn_norm, self.hidden, L.pre_ffn_norm, self.hidden2, self.xn, H, B,
                         s.eps, ops=self.xops)
             if probe:
@@ -1065,10 +1069,10 @@ class BatchDecoder(_SyntheticModel):
                 if L.qt["wgate"] == "q4k" and L.qt["wup"] == "q4k":
                     c.gateUpGeluBatch(self.xn, L.wgate, L.wup, self.act, I, H, B, ops=self.xops)
                 else:  # gate and up apart (whole sums), then the GELU product
-                    self._mm_batch(L.qt["wgate"], self.xn, L.wgate, self.gate_b, I, H, 1, self.xops)
-                    self._mm_batch(L.qt["wup"], self.xn, L.wup, self.up_b, I, H, 1, self.xops)
+                    self._mm_batch(L.qt["wgate"], self.xn, L.wgate, self.gate_b, I, H, 1, self.xops, B)
+                    self._mm_batch(L.qt["wup"], self.xn, L.wup, self.up_b, I, H, 1, self.xops, B)
                     c.geluMul(self.gate_b, self.up_b, self.act, B * I)
-                nd = self._mm_batch(L.qt["wdown"], self.act, L.wdown, self.down_parts, H, I, self.ks_f, None)
+                nd = self._mm_batch(L.qt["wdown"], self.act, L.wdown, self.down_parts, H, I, self.ks_f, None, B)
             if probe:
                 probe("ffn", il, nd)
             if s.ple_dim:
@@ -1091,14 +1095,23 @@ class BatchDecoder(_SyntheticModel):
                         H, B, s.eps, ops=self.xops)
         if probe:
             probe("prep", s.n_layers, 0)
-        self._head(sample)
+        self._head(sample, B)
         if probe and self.lm_head is not None:
             probe("head", s.n_layers, 0)
         self.lens_host = self.lens_host + 1
 
-    def _head(self, sample: str) -> None:
-        """LM head + softcap over the normalised rows in xn / xops, then the sample of every row."""
-        c, s, B, H = self.ctx, self.s, self.B, self.s.hidden
+    @staticmethod
+    def _for_rows(params, rows: int):
+        """The attention parameters of a step over the first `rows` rows."""
+        if params.num_seqs == rows:
+            return params
+        p = type(params).from_buffer_copy(params)
+        p.num_seqs = rows
+        return p
+
+    def _head(self, sample: str, B: int) -> None:
+        """LM head + softcap over the B normalised rows in xn / xops, then the sample of each."""
+        c, s, H = self.ctx, self.s, self.s.hidden
         if self.lm_head is None:
             return
         if self.lm_type == "f16":
@@ -1120,14 +1133,14 @@ class BatchDecoder(_SyntheticModel):
         return (L.qt["wgate"] == "q4k" and L.qt["wup"] == "q4k" and L.qt["wdown"] == "q6k"
                 and self.s.ffn_of(il) in (6144, 12288))
 
-    def _mm_batch(self, qt: str, x, w, y, M: int, N: int, max_ksplit: int, ops) -> int:
-        """y = W . x for the B rows: f16 rows through the f16 matvec (one
+    def _mm_batch(self, qt: str, x, w, y, M: int, N: int, max_ksplit: int, ops, B: int) -> int:
+        """y = W . x for B rows: f16 rows through the f16 matvec (one
         chunk), block formats split-K into at most max_ksplit chunks. Returns
         the chunk count."""
         if qt == "f16":
-            self.ctx.matmulF16(x, w, y, M, N, self.B)
+            self.ctx.matmulF16(x, w, y, M, N, B)
             return 1
-        return self.ctx.matmulSegmentsBatchPartial(qt, x, [w], [y], [M], N, self.B, max_ksplit, ops=ops)
+        return self.ctx.matmulSegmentsBatchPartial(qt, x, [w], [y], [M], N, B, max_ksplit, ops=ops)
 
     def prefill(self, tokens, start: int = 0, sample: str = "argmax", probe=None) -> int:
         """Batched prefill of one sequence (a shared_pages decoder with an
@@ -1144,7 +1157,8 @@ class BatchDecoder(_SyntheticModel):
         prefill matmuls (each weight read and unpacked once per pass), and
         leaves the same rows as its last chunk would. A short last
         chunk repeats its last token and position in the spare rows
-        (identical rows, identical writes). Returns the row of the final
+        (identical rows, identical writes); a prompt of one chunk leaves out
+        spare rows past the 16 or 32 that hold it. Returns the row of the final
         chunk that holds the prompt's last token: its logits and `tokens`
         entry are the first sample. probe (tests): passed to every chunk's
         step."""
@@ -1165,11 +1179,13 @@ class BatchDecoder(_SyntheticModel):
         ctok = np.concatenate([toks, np.repeat(toks[-1], pad)]).astype(np.uint32)
         cpos = np.concatenate([start + np.arange(T), np.repeat(start + T - 1, pad)]).astype(np.uint32)
         dtok, dpos = self.ctx.from_numpy(ctok), self.ctx.from_numpy(cpos)
+        # a single chunk takes only as many rows as its matrix-core tiles need
+        rows = next((r for r in (16, 32) if T <= r < B), B) if nch == 1 and probe is None else B
         for k in range(nch):
             self.ctx.copy(self.tokens, dtok.offset(4 * B * k), 4 * B)
             self.ctx.copy(self.seq_lens, dpos.offset(4 * B * k), 4 * B)
             self.lens_host = cpos[B * k:B * (k + 1)].copy()
-            self.step(sample, probe=probe, head=k == nch - 1)
+            self.step(sample, probe=probe, head=k == nch - 1, rows=rows)
         self.ctx.sync()
         dtok.free()
         dpos.free()
@@ -1235,7 +1251,7 @@ class BatchDecoder(_SyntheticModel):
         c.copy(self.seq_lens, dlen.offset(4 * (T + pad - B)), 4 * B)
         self.lens_host = clen[-B:].copy()
         c.batchPrep(self.hidden, 1, self.final_norm, None, None, None, self.xn, H, B, s.eps, ops=self.xops)
-        self._head(sample)
+        self._head(sample, B)
         c.sync()
         dtok.free()
         dlen.free()

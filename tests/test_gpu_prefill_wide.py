@@ -1,7 +1,7 @@
 """GPU parity of the whole-prompt path: the prefill matmuls against a float64
 product of the same dequantized weights, at the edges of their 64-vector and
-256- / 128- / 16-row tiles, and prompts of more than one chunk against the
-chunk-by-chunk path on the same weights (itself held to the oracle's
+256- / 128- / 16-row tiles, and prompts (of more than one chunk,
+and of a part of one) against the chunk-by-chunk path on the same weights (itself held to the oracle's
 sequential forwards in test_gpu_prefill.py).
 
 Tolerances: Q4_K and f16 weights enter the matrix cores exactly and the
@@ -129,6 +129,10 @@ def test_prefill_ple_gated(ctx, T, parts):
     ("real", 64, 131, 37),
     ("real", 7, 23, 0),          # odd chunks
     ("uniform", 1, 3, 5),
+    ("uniform", 64, 9, 0),       # one chunk: 16 and 32 of its rows, and all
+    ("real", 64, 27, 700),
+    ("uniform", 64, 33, 0),
+    ("uniform", 20, 17, 500),
 ])
 def test_wide_prefill_equals_chunks(ctx, layout, B, T, start):
     s = (E2BShape(n_layers=2, global_layers=(1,), vocab=4096) if layout == "uniform" else
