@@ -746,7 +746,7 @@ __global__ __launch_bounds__(MW_NT) void attn_merge_wide_kernel(const float* ws,
 }
 
 // ---------------------------------------------------------------------------
-// matrix-core split-K decode attention: 8 query heads per KV head, head_dim 256
+// matrix-core split-K decode attention: 8 query heads per KV head, head_dim 256 or 512
 // ---------------------------------------------------------------------------
 //
 // Workgroup = (chunk of 64 * nstep consecutive positions of one sequence's
@@ -764,9 +764,15 @@ __global__ __launch_bounds__(MW_NT) void attn_merge_wide_kernel(const float* ws,
 //    positions x 16 dims of V; 16 dim tiles.
 // At the end the four waves' (m, l, o) are combined in LDS and one partial
 // per head is written for attn_merge_kernel.
+// Head dim 512: eight waves (one workgroup per CU); wave w takes row tile
+// w % 4 and the 256 dims from 256 (w / 4) on, and the two waves of a row tile
+// add their halves of the scores through LDS, in the same order in both.
+// The VALU form it replaces there (attn_kernel, one 32-position split per
+// workgroup) wrote and re-read a partial per 32 positions, half as many bytes
+// again as the K/V rows.
 
 struct MqArgs {
-  const float* q;  // [num_seqs][nqh][256]
+  const float* q;  // [num_seqs][nqh][head dim]
   const uint16_t* kc;
   const uint16_t* vc;
   const int32_t* page_table;  // paged: [num_seqs][max_pages]
@@ -781,13 +787,16 @@ struct MqArgs {
 
 constexpr int kMqPages = 96;  // page-table entries of a chunk held in LDS (1024 positions of 16-row pages)
 
-template <bool PAGED>
-__global__ __launch_bounds__(NT, 2) void mq_attn_kernel(MqArgs a) {
-  __shared__ __align__(16) _Float16 kt[MQ_STEP * MQ_RS];
-  __shared__ __align__(16) _Float16 vt[MQ_STEP * MQ_RS];
+template <bool PAGED, int HD>
+__global__ __launch_bounds__(HD, 2) void mq_attn_kernel(MqArgs a) {
+  constexpr int RS = HD + 8;  // K/V row stride in LDS (halves)
+  __shared__ __align__(16) _Float16 kt[MQ_STEP * RS];
+  __shared__ __align__(16) _Float16 vt[MQ_STEP * RS];
+  __shared__ __align__(16) mf4 xs[HD == 512 ? 8 * 64 : 1];  // halves of the scores
   __shared__ uint32_t s_seq, s_chunk;
   __shared__ int32_t s_pg[kMqPages];
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, q = l >> 4, c = l & 15;
+  const int wt = HD == 256 ? w : w & 3, wd = HD == 256 ? 0 : w >> 2;  // row tile, 256-dim half
   const uint32_t kvh = blockIdx.y;
   const uint32_t CH = MQ_STEP * a.nstep;
 
@@ -849,33 +858,33 @@ __global__ __launch_bounds__(NT, 2) void mq_attn_kernel(MqArgs a) {
     }
     return pos;
   };
-  // K (pieces 0-7) and V (8-15) of one step: piece tid + 256i covers row
-  // (tid + 256i) / 32 % 64, dims 8 * (tid % 32) .. +7; rows past the chunk
+  // K (pieces 0-7) and V (8-15) of one step: piece tid + HD i covers row
+  // (tid + HD i) / (HD / 8) % 64, dims 8 * (tid % (HD / 8)) .. +7; rows past the chunk
   // repeat its last live position (masked in the scores)
   mu4 pf[16];
   auto load_step = [&](uint32_t st) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const uint32_t pc = (uint32_t)tid + 256u * (uint32_t)(i & 7);
-      const uint32_t r = pc >> 5, col = (pc & 31) * 8;
+      const uint32_t pc = (uint32_t)tid + (uint32_t)HD * (uint32_t)(i & 7);
+      const uint32_t r = pc / (HD / 8), col = pc % (HD / 8) * 8;
       const uint32_t pos = min(wstart + c0 + st * MQ_STEP + r, last);
       const uint16_t* base = i < 8 ? a.kc : a.vc;
-      pf[i] = *(const mu4*)(base + (row_of(pos) * a.nkh + kvh) * MQ_HD + col);
+      pf[i] = *(const mu4*)(base + (row_of(pos) * a.nkh + kvh) * HD + col);
     }
   };
   auto store_step = [&]() {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const uint32_t pc = (uint32_t)tid + 256u * (uint32_t)(i & 7);
-      const uint32_t r = pc >> 5, col = (pc & 31) * 8;
-      _Float16* dst = (i < 8 ? kt : vt) + r * MQ_RS + col;
+      const uint32_t pc = (uint32_t)tid + (uint32_t)HD * (uint32_t)(i & 7);
+      const uint32_t r = pc / (HD / 8), col = pc % (HD / 8) * 8;
+      _Float16* dst = (i < 8 ? kt : vt) + r * RS + col;
       *(mu4*)dst = pf[i];
     }
   };
 
   load_step(0);
-  // q as the scores' B operand: column c = (part c/8, head c%8), dims 32j + 8q .. +7
-  const float* qg = a.q + ((size_t)seq * a.nqh + kvh * MQ_G + (c & 7)) * MQ_HD;
+  // q as the scores' B operand: column c = (part c/8, head c%8), dims 256 wd + 32j + 8q .. +7
+  const float* qg = a.q + ((size_t)seq * a.nqh + kvh * MQ_G + (c & 7)) * HD + 256 * wd;
   float4 qr[16];
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
@@ -909,15 +918,20 @@ __global__ __launch_bounds__(NT, 2) void mq_attn_kernel(MqArgs a) {
     mf4 S = mf4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const mh8 A = *(const mh8*)(kt + (16 * w + c) * MQ_RS + 32 * j + 8 * q);
+      const mh8 A = *(const mh8*)(kt + (16 * wt + c) * RS + 256 * wd + 32 * j + 8 * q);
       S = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, qb[j], S, 0, 0, 0);
+    }
+    if constexpr (HD == 512) {
+      xs[w * 64 + l] = S;
+      __syncthreads();
+      S = xs[wt * 64 + l] + xs[(wt + 4) * 64 + l];
     }
     float sc[4];
     float mx = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float v = S[i] + g4d::dpp<kDppRor8>(S[i]);  // q_hi + q_lo columns
-      const uint32_t off = c0 + st * MQ_STEP + 16u * w + 4u * q + i;
+      const uint32_t off = c0 + st * MQ_STEP + 16u * wt + 4u * q + i;
       sc[i] = off < cend ? v * a.scale : -INFINITY;
       mx = fmaxf(mx, sc[i]);
     }
@@ -952,7 +966,7 @@ __global__ __launch_bounds__(NT, 2) void mq_attn_kernel(MqArgs a) {
     for (int dt = 0; dt < 16; ++dt) {
       mh4 Bv;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) Bv[i] = vt[(16 * w + 4 * q + i) * MQ_RS + 16 * dt + c];
+      for (int i = 0; i < 4; ++i) Bv[i] = vt[(16 * wt + 4 * q + i) * RS + 256 * wd + 16 * dt + c];
       mf4 o = O[dt];
 #pragma unroll
       for (int i = 0; i < 4; ++i) o[i] *= ar[i];
@@ -970,18 +984,18 @@ __global__ __launch_bounds__(NT, 2) void mq_attn_kernel(MqArgs a) {
   for (int dt = 0; dt < 16; ++dt)
 #pragma unroll
     for (int i = 0; i < 4; ++i) O[dt][i] = g4d::xsum32(O[dt][i]);
-  float* ow = (float*)kt;                 // [4 waves][8 heads][256]
+  float* ow = (float*)kt;                 // [4 row tiles][8 heads][HD]
   float* mw = (float*)vt;                 // [4][8]
   float* lw = mw + 32;                    // [4][8]
   if (q < 2) {
 #pragma unroll
     for (int dt = 0; dt < 16; ++dt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) ow[(w * MQ_G + 4 * q + i) * MQ_HD + 16 * dt + c] = O[dt][i];
+      for (int i = 0; i < 4; ++i) ow[(wt * MQ_G + 4 * q + i) * HD + 256 * wd + 16 * dt + c] = O[dt][i];
   }
-  if (q == 0 && c < MQ_G) {
-    mw[w * MQ_G + c] = m_run;
-    lw[w * MQ_G + c] = l_run;
+  if (wd == 0 && q == 0 && c < MQ_G) {
+    mw[wt * MQ_G + c] = m_run;
+    lw[wt * MQ_G + c] = l_run;
   }
   __syncthreads();
   const size_t part = (((size_t)seq * a.nkh + kvh) * a.max_chunks + chunk) * MQ_G;
@@ -998,11 +1012,11 @@ __global__ __launch_bounds__(NT, 2) void mq_attn_kernel(MqArgs a) {
 #pragma unroll
     for (int ww = 0; ww < 4; ++ww) {
       const float m = mw[ww * MQ_G + h];
-      const float wt = m == -INFINITY ? 0.f : mq_exp(m - M);
-      L += wt * lw[ww * MQ_G + h];
-      o += wt * ow[(ww * MQ_G + h) * MQ_HD + tid];
+      const float wgt = m == -INFINITY ? 0.f : mq_exp(m - M);
+      L += wgt * lw[ww * MQ_G + h];
+      o += wgt * ow[(ww * MQ_G + h) * HD + tid];
     }
-    ws_o[(part + h) * MQ_HD + tid] = o;
+    ws_o[(part + h) * HD + tid] = o;
     if (tid == 0) {
       ws_m[part + h] = M;
       ws_l[part + h] = L;
@@ -1305,25 +1319,37 @@ int merge(g4_ctx* ctx, const AttnArgs& a, float* out, const SplitPlan& sp, uint3
 }
 
 // The matrix-core kernel serves the paged batch: 8 query heads per KV head at
-// head_dim 256 and up to 64 sequences (its chunk numbering runs in one wave).
+// head_dim 256 or 512 and up to 64 sequences (its chunk numbering runs in one wave).
 // One dense sequence takes the VALU form (attn_kernel), measured faster on
 // its own at every context of the single-sequence shape (8 query heads,
 // 1 KV head x 256: 9.0 against 11.8 us at 512 positions, 11.2 against
 // 13.9 at 4096, 20.7 against 21.5 at 32768); in the decode step the fused
 // form (mqf_kernel) keeps the matrix cores.
-bool mq_fits(uint32_t G, uint32_t hd, uint32_t num_seqs) { return G == 8 && hd == 256 && num_seqs <= 64; }
+// Head dim 512 takes it for windows past 512 positions: below, the VALU form's
+// 32-position workgroups, several to a CU, are done sooner (ten layers, 15
+// sequences to 268 positions 714 against 722-739 us; 40 to 900: 1172 against
+// 1133, 64 to 4096: 1405 against 1330).
+bool mq_fits(uint32_t G, uint32_t hd, uint32_t num_seqs, uint32_t eff) {
+  return G == 8 && (hd == 256 || (hd == 512 && eff > 512)) && num_seqs <= 64;
+}
 
 // Steps per workgroup from the largest window, sized for about four
-// workgroups per CU when every sequence is that long.
+// workgroups per CU when every sequence is that long. At head dim 512 a CU
+// holds one workgroup at a time: sized for two where that is a step or two
+// (the live half of the windows then fits the chip once), four beyond, so
+// that the last round is short (64 sequences to 4096 positions, ten layers:
+// two, six and eight cost 41, 18 and 19 us more).
+template <int HD>
 int mq_decode(g4_ctx* ctx, const char* fn, const AttnArgs& base, uint32_t num_seqs, float* out, size_t ws_len,
               uint8_t* ops = nullptr) {
   const uint32_t eff = eff_len(base.cap, base.window);
   const uint64_t cus = ctx->num_cus > 0 ? (uint64_t)ctx->num_cus : 256;
   const uint64_t want = ((uint64_t)num_seqs * eff + 64 * 4 * cus - 1) / (64 * 4 * cus);
-  const uint32_t nstep = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(want, 1), 16);
+  const uint64_t two = ((uint64_t)num_seqs * eff + 64 * 2 * cus - 1) / (64 * 2 * cus);
+  const uint32_t nstep = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(HD == 512 && two <= 2 ? two : want, 1), 16);
   const uint32_t chunk = MQ_STEP * nstep;
   const uint32_t max_chunks = ceil_div(eff == 0 ? 1 : eff, chunk);
-  const size_t need = ws_bytes(num_seqs, base.nkh, max_chunks, MQ_G, MQ_HD);
+  const size_t need = ws_bytes(num_seqs, base.nkh, max_chunks, MQ_G, HD);
   G4_REQUIRE(ws_len >= need, "%s: workspace %zu bytes < %zu required", fn, ws_len, need);
   MqArgs m{};
   m.q = base.q;
@@ -1342,9 +1368,9 @@ int mq_decode(g4_ctx* ctx, const char* fn, const AttnArgs& base, uint32_t num_se
   m.max_chunks = max_chunks;
   m.ws = base.ws;
   const dim3 grid(num_seqs * max_chunks, base.nkh);
-  hipLaunchKernelGGL(mq_attn_kernel<true>, grid, dim3(NT), 0, ctx->stream, m);
+  hipLaunchKernelGGL((mq_attn_kernel<true, HD>), grid, dim3(HD), 0, ctx->stream, m);
   G4_LAUNCHED(ctx, "attn_decode_mfma");
-  return merge_launch(ctx, base.ws, out, base.nqh, base.nkh, MQ_G, MQ_HD, max_chunks, num_seqs, m.len, chunk, ops);
+  return merge_launch(ctx, base.ws, out, base.nqh, base.nkh, MQ_G, HD, max_chunks, num_seqs, m.len, chunk, ops);
 }
 
 int check_heads(const char* fn, uint32_t nqh, uint32_t nkh, uint32_t hd) {
@@ -1784,8 +1810,9 @@ int g4_pagedAttnDecodeOps(g4_ctx* ctx, const float* q, const uint16_t* k_pool, c
   int rc = paged_setup(__func__, k_pool, v_pool, page_table, seq_lens, p, workspace, workspace_bytes, a, sp);
   if (rc) return rc;
   a.q = q;
-  if (mq_fits(p.num_q_heads / p.num_kv_heads, p.head_dim, p.num_seqs))
-    return mq_decode(ctx, __func__, a, p.num_seqs, output, workspace_bytes, (uint8_t*)ops);
+  if (mq_fits(p.num_q_heads / p.num_kv_heads, p.head_dim, p.num_seqs, eff_len(p.max_seq_len, p.sliding_window)))
+    return p.head_dim == 256 ? mq_decode<256>(ctx, __func__, a, p.num_seqs, output, workspace_bytes, (uint8_t*)ops)
+                             : mq_decode<512>(ctx, __func__, a, p.num_seqs, output, workspace_bytes, (uint8_t*)ops);
   rc = launch_attn<true, false>(ctx, a, p.num_q_heads / p.num_kv_heads, p.head_dim, sp.cp,
                                 dim3(sp.nsplit, p.num_kv_heads, p.num_seqs));
   if (rc) return rc;
