@@ -1152,8 +1152,8 @@ class BatchDecoder(_SyntheticModel):
         launch reads them, so the chunk is causal). The reference runs one
         full forward per prompt token instead (src/engine.ts:1923-1938) and
         samples from the last one (src/engine.ts:2014-2017); as there, only
-        the last chunk runs the LM head. A prompt of more than one chunk
-        takes the layers up to `wide_rows` rows at a time instead, through the
+        the last chunk runs the LM head. A prompt of more than two chunks
+        (of more than one past 32 rows) takes the layers up to `wide_rows` rows at a time instead, through the
         prefill matmuls (each weight read and unpacked once per pass), and
         leaves the same rows as its last chunk would. A short last
         chunk repeats its last token and position in the spare rows
@@ -1171,7 +1171,11 @@ class BatchDecoder(_SyntheticModel):
         nch = -(-T // B)
         n = T - (nch - 1) * B
         pad = nch * B - T
-        if nch > 1 and self.wide_rows and probe is None:
+        # (two chunks of at most 32 rows are as fast as one pass: 20 tokens by
+        # 16 rows over ten layers 1.22 against 1.49 ms, 40 by 32 1.36 against
+        # 1.53; three, or two of 64, are slower: 40 by 16 1.77 against 1.52, 70
+        # by 64 1.73 against 1.51)
+        if nch > (1 if B > 32 else 2) and self.wide_rows and probe is None:
             self._prefill_wide(toks, start, pad, sample)
             return n - 1
         # every chunk's tokens and lengths (before the step appends each row)

@@ -1,7 +1,7 @@
 """GPU parity of the whole-prompt path: the prefill matmuls against a float64
 product of the same dequantized weights, at the edges of their 64-vector and
-256- / 128- / 16-row tiles, and prompts (of more than one chunk,
-and of a part of one) against the chunk-by-chunk path on the same weights (itself held to the oracle's
+256- / 128- / 16-row tiles, and prompts (of several chunks, and of a
+part of one) against the chunk-by-chunk path on the same weights (itself held to the oracle's
 sequential forwards in test_gpu_prefill.py).
 
 Tolerances: Q4_K and f16 weights enter the matrix cores exactly and the
