@@ -64,6 +64,14 @@ int g4_internal_dequant_f16_q58(g4_ctx* ctx, int wtype, const void* blocks, uint
 // [batch][256][nparts]) and result[r][512] receives (value, index bits).
 int g4_internal_topk_final(g4_ctx* ctx, const void* parts, int nparts, uint32_t batch, float* result);
 
+// Y [B][M] = a Q6_K matrix of M rows times B <= 32 vectors given as operand
+// blocks (g4d::Ops), K 1536 or 2048, M at least 16 rows per two workgroups of
+// every CU (k_head.hip: a code object of its own, since beside the batched
+// matmuls its kernels cost each of their launches 0.1-0.5 us, a 7-sequence
+// slice of five layers 252 -> 255 us).
+int g4_internal_tall_q6k(g4_ctx* ctx, const uint8_t* W, float* Y, uint32_t M, uint32_t K, const uint8_t* ops,
+                         uint32_t B, float cap);
+
 // Matrix-core matmul of `batch` activation vectors (k_batch.hip).
 int g4_internal_batch_matmul(g4_ctx* ctx, const char* fn, int qt, const float* x, const void* w, float* y,
                              uint32_t M, uint32_t N, uint32_t batch);
