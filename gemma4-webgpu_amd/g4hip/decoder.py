@@ -994,10 +994,14 @@ class BatchDecoder(_SyntheticModel):
 
         head=False stops after the layers (no final norm, LM head or sample):
         a prefill chunk whose logits nobody reads (the reference's prefill
-        forwards run no LM head either, src/engine.ts:1896-1900). rows: only
-        the first rows take the step (a prefill chunk's, the rest spare);
-        every length advances."""
-        c, s, B = self.ctx, self.s, rows or self.B
+        forwards run no LM head either, src/engine.ts:1896-1900). rows (1..B,
+        shared_pages only): only the first rows take the step (a prefill
+        chunk's, the rest spare); every length advances. Rows with page lists
+        of their own step together: their attention block numbers the q/k/v
+        partial sums and the appended rows by all B sequences."""
+        if rows is not None and not (self.shared_pages and 1 <= rows <= self.B):
+            raise ValueError(f"step: rows={rows} needs shared_pages and 1..{self.B} rows")
+        c, s, B = self.ctx, self.s, self.B if rows is None else rows
         H = s.hidden
         if self.embedding is not None:
             c.embeddingLookupBatch(self.embedding, s.vocab, self.hidden, H, self.tokens, B)
