@@ -16,11 +16,18 @@
 //    32-deep A operand of the PV product as they lie in registers (V's
 //    positions are stored in that order), P as f16 hi + lo;
 //  * head dim 512: two waves share a column tile, each 256 dims; their score
-//    halves are added through LDS (same order in both).
+//    halves are added through LDS (same order in both);
+//  * a token's V rows are those of its own window only: in the steps at the
+//    ends of the workgroup's windows a wave multiplies V once for each of its
+//    two tokens, with the rows outside that token's window zeroed (P is 0
+//    there, but 0 x Inf is NaN: one non-finite row would reach tokens before
+//    it). These steps go first, in a loop of their own: as a branch of one loop
+//    they cost it 30 spilled registers.
 // A wave's LDS reads take as long as its products (1 KB per two MFMAs), which
 // bounds the kernel; a window of few tokens over a long cache is split over
 // workgroups (partials merged in split order by merge_kernel).
 #include <algorithm>
+#include <type_traits>
 
 #include "mm_operand.hpp"
 
@@ -71,29 +78,40 @@ __global__ __launch_bounds__(Shape<HD>::NT, 2) void pf_attn_kernel(PaArgs a) {
   __shared__ __align__(16) _Float16 kt[STEP * KS];
   __shared__ __align__(16) _Float16 vt[HD * VS];
   __shared__ __align__(16) f4 xs[HD == 512 ? 8 * NPT * 64 : 1];  // score halves
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, q = l >> 4, c = l & 15;
+  const int tid = threadIdx.x, l = tid & 63, q = l >> 4, c = l & 15;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wc = w & 3, wd = w >> 2;  // column tile, 256-dim half
   const uint32_t kvh = blockIdx.y;
   // the last tiles of a prompt have the longest windows: they start first
   const uint32_t tile = gridDim.x - 1 - blockIdx.x, split = blockIdx.z;
   const uint32_t t0 = tile * TOK;
 
-  // the tokens' windows (uniform loads), this column's and their union
-  uint32_t lo = 0xffffffffu, hi = 0, clo = 0, chi = 0;
+  // the tokens' windows (uniform loads): the wave's two, their union and common part over the workgroup
+  uint32_t lo = 0xffffffffu, hi = 0, wlo[2] = {0, 0}, whi[2] = {0, 0}, ilo = 0, ihi = 0xffffffffu;
 #pragma unroll
   for (int i = 0; i < TOK; ++i) {
     const uint32_t L = min(a.lens[min(t0 + i, a.T - 1)], a.cap);
     const uint32_t s = a.window && L > a.window ? L - a.window : 0u;
     lo = min(lo, s);
     hi = max(hi, L);
-    if (i == 2 * wc + (c >> 3)) {
-      clo = s;
-      chi = L;
+    ilo = max(ilo, s);
+    ihi = min(ihi, L);
+    if ((i >> 1) == wc) {
+      wlo[i & 1] = s;
+      whi[i & 1] = L;
     }
   }
+  const uint32_t clo = wlo[c >> 3], chi = whi[c >> 3];  // this column's
   const uint32_t steps = hi > lo ? (hi - lo + STEP - 1) / STEP : 0u;
   const uint32_t per = (steps + a.nsplit - 1) / a.nsplit;
   const uint32_t s0 = min(split * per, steps), s1 = min(s0 + per, steps);
+  // Steps e0 .. e1 - 1 lie inside every token's window. The others, at its
+  // ends, go first: turn k of the n is step step_of(k).
+  const uint32_t n = s1 - s0;
+  const uint32_t e0 = min(max((ilo - lo + STEP - 1) / STEP, s0), s1);
+  const uint32_t e1 = max(min(ihi > lo ? (ihi - lo) / STEP : 0u, s1), e0);
+  const uint32_t ends = n - (e1 - e0);
+  auto step_of = [&](uint32_t k) { return k < e0 - s0 ? s0 + k : (k < ends ? e1 + (k - (e0 - s0)) : e0 + (k - ends)); };
   const uint32_t last = hi ? hi - 1 : 0u;  // rows past the window repeat its last position (masked)
 
   auto row_of = [&](uint32_t pos) -> size_t {
@@ -158,17 +176,23 @@ __global__ __launch_bounds__(Shape<HD>::NT, 2) void pf_attn_kernel(PaArgs a) {
     }
   }
 
+  // V operands of the even and odd dim tiles (positions 4q .. + 3 and 16 + 4q .. + 3; rows 16 dt apart)
+  const _Float16* vb[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+    vb[k] = vt + (256 * wd + c) * VS + ((uint32_t)q ^ ((2u * k + (c >> 3)) & (NB - 1))) * 8;
+
   f4 O[16];
 #pragma unroll
   for (int dt = 0; dt < 16; ++dt) O[dt] = f4{0.f, 0.f, 0.f, 0.f};
   float m_run = -INFINITY, l_run = 0.f;  // of column c
 
-  if (s0 < s1) load_step(s0);
-  for (uint32_t st = s0; st < s1; ++st) {
+  auto turn = [&](uint32_t k, auto inside) __attribute__((always_inline)) {
+    const uint32_t st = step_of(k);
     __syncthreads();  // every wave is done with the previous step's rows
     store_step();
     __syncthreads();
-    if (st + 1 < s1) load_step(st + 1);  // (uniform) in flight during this step
+    if (k + 1 < n) load_step(step_of(k + 1));  // (uniform) in flight during this step
 
     f4 S[NPT];
 #pragma unroll
@@ -196,7 +220,7 @@ __global__ __launch_bounds__(Shape<HD>::NT, 2) void pf_attn_kernel(PaArgs a) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const uint32_t pos = pb + 16u * p + i;
-        S[p][i] = pos >= clo && pos < chi ? S[p][i] * a.scale : -INFINITY;
+        S[p][i] = decltype(inside)::value || (pos >= clo && pos < chi) ? S[p][i] * a.scale : -INFINITY;
         mx = fmaxf(mx, S[p][i]);
       }
     mx = g4d::xmax32(g4d::xmax16(mx));
@@ -226,16 +250,45 @@ __global__ __launch_bounds__(Shape<HD>::NT, 2) void pf_attn_kernel(PaArgs a) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) O[dt][i] *= ar[i];
     }
-#pragma unroll
-    for (int g = 0; g < NPT / 2; ++g)
+    static_assert(NPT == 2 && NB == 4, "one 32-position operand per step");
+    if constexpr (decltype(inside)::value) {
 #pragma unroll
       for (int dt = 0; dt < 16; ++dt) {
-        const uint32_t d = 256u * wd + 16u * dt + c;
-        const h8 B = *(const h8*)(vt + d * VS + ((uint32_t)(4 * g + q) ^ (d / 8 & (NB - 1))) * 8);
-        O[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph[g], B, O[dt], 0, 0, 0);
-        O[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl[g], B, O[dt], 0, 0, 0);
+        const h8 B = *(const h8*)(vb[dt & 1] + dt * 16 * VS);
+        O[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph[0], B, O[dt], 0, 0, 0);
+        O[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl[0], B, O[dt], 0, 0, 0);
       }
-  }
+    } else {
+      u32x4 keep[2];  // of this lane's eight positions, each token's
+      const uint32_t p0 = lo + st * STEP;
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const uint32_t n0 = whi[k] > p0 ? min(whi[k] - p0, 32u) : 0u, n1 = wlo[k] > p0 ? min(wlo[k] - p0, 32u) : 0u;
+        const uint32_t live = (uint32_t)(((1ull << n0) - 1) & ~((1ull << n1) - 1)) >> (4 * q);  // (bit = position)
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          const uint32_t two = live >> ((m < 2 ? 0 : 16) + 2 * (m & 1));
+          keep[k][m] = (two & 1u) * 0xffffu | (two >> 1 & 1u) * 0xffff0000u;
+        }
+      }
+#pragma unroll
+      for (int dt = 0; dt < 16; ++dt) {
+        const u32x4 B = *(const u32x4*)(vb[dt & 1] + dt * 16 * VS);
+        f4 o[2];  // O's rows 4q + i are of token q / 2
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const h8 Bk = __builtin_bit_cast(h8, B & keep[k]);
+          o[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl[0], Bk, f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+          o[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph[0], Bk, o[k], 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) O[dt][i] += q < 2 ? o[0][i] : o[1][i];
+      }
+    }
+  };
+  if (n) load_step(step_of(0));
+  for (uint32_t k = 0; k < ends; ++k) turn(k, std::false_type{});
+  for (uint32_t k = ends; k < n; ++k) turn(k, std::true_type{});
 
   // columns 4q + i: token 2 wc + (4q + i) / 8, head (4q + i) % 8
   float inv[4];

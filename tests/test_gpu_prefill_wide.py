@@ -203,3 +203,37 @@ def test_prefill_attention_two_kv_heads(ctx):
 
 def test_prefill_attention_without_workspace(ctx):
     _attn_case(ctx, 512, 9, 2000, 0, short_ws=True)
+
+
+@pytest.mark.parametrize("hd", [256, 512])
+@pytest.mark.parametrize("window", [0, 32])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_prefill_attention_non_finite_rows(ctx, hd, window, bad):
+    """A non-finite V element reaches the rows whose window holds it, in its own dim, and no others: not those
+    before it, nor (with a window) those past it, nor the rows of a tail step that repeats the last position."""
+    page, nq, T, start = 16, 8, 45, 40
+    L = start + T
+    pages = -(-L // page)
+    table = np.random.default_rng(3).permutation(pages).astype(np.int32)
+    kp, vp = (O.gen_normal_f16(s, pages * page * hd, 0.0, 1.0 if s == 62 else 0.25) for s in (61, 62))
+    q = O.gen_normal_f32(63, T * nq * hd, 0.0, 0.5).reshape(T, nq * hd)
+    lens = (start + 1 + np.arange(T)).astype(np.uint32)
+    poison = {start + 5: 3, start + 17: 130, 20: 7, L - 1: 200}  # position: dim
+    rows = vp.view(np.float16).reshape(-1, hd)
+    clean = rows.copy()
+    for pos, d in poison.items():
+        r = table[pos // page] * page + pos % page
+        rows[r, d] = bad
+        clean[r, d] = 0
+    p = ctx.paged_fused_params(T, nq, 1, hd, page, pages, pages * page, pages, window, 1e-6, 1e4, 0)
+    out = ctx.from_numpy(np.full(T * nq * hd, 7.0, np.float32))
+    ctx.prefillAttn(ctx.from_numpy(q), ctx.from_numpy(kp), ctx.from_numpy(vp), ctx.from_numpy(table),
+                    ctx.from_numpy(lens), out, p, ctx.alloc(ctx.prefill_attn_workspace_bytes(p)))
+    got = out.download(np.float32).reshape(T, nq, hd)
+    for v in range(T):
+        n = int(lens[v])
+        seen = {d for pos, d in poison.items() if (n - window if window else 0) <= pos < n}
+        ok = [d for d in range(hd) if d not in seen]
+        assert not np.isfinite(got[v][:, sorted(seen)]).any(), v
+        want = O.attention_paged(q[v], kp, clean.view(np.uint16).reshape(-1), table, page, nq, 1, hd, n, 1.0, window)
+        assert_close(got[v][:, ok], want.reshape(nq, hd)[:, ok], rel=4e-5, what=f"row {v}")
