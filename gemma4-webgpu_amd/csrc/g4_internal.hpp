@@ -352,6 +352,17 @@ struct OpsSub {
   __host__ __device__ static constexpr uint32_t scale_off(int ntv) { return (uint32_t)ntv * MAIN_T; }
   __host__ __device__ static constexpr uint32_t bytes(int ntv) { return (uint32_t)ntv * (MAIN_T + 512); }
 };
+// The power of two that brings am to 2^13 .. 2^14 (1 for 0 and what is not
+// finite), and its inverse: values of at most am, so scaled, are f16 hi + lo
+// pairs of 22 bits down to 2^-16 of am and do not overflow.
+__device__ __forceinline__ float f16_pair_scale(float am, float& inverse) {
+  int ex = 0;
+  (void)frexpf(am, &ex);
+  const int k = am > 0.f && am < INFINITY ? min(max(14 - ex, -120), 120) : 0;
+  inverse = ldexpf(1.0f, -k);
+  return ldexpf(1.0f, k);
+}
+
 // Operand blocks of the prefill matmul (k_prefill.hip), one per 64 vectors
 // and super-block of K: main and sums as Ops with 4 vector tiles, but one
 // 2^e per vector and half super-block (equal halves where a whole super-block

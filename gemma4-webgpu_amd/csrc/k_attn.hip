@@ -767,6 +767,12 @@ __global__ __launch_bounds__(MW_NT) void attn_merge_wide_kernel(const float* ws,
 // Head dim 512: eight waves (one workgroup per CU); wave w takes row tile
 // w % 4 and the 256 dims from 256 (w / 4) on, and the two waves of a row tile
 // add their halves of the scores through LDS, in the same order in both.
+// There q is scaled by a power of two per head and half and P by 2^14, and the
+// scores' 32-dim products are added in f32: for the accuracy over all of f32
+// that the VALU form had (16 sequences to 4000 positions, scores of spread 2:
+// 3.5e-7 of float64's result, as attn_kernel; unscaled and chained 4.8e-7, and
+// with a dominant key of small V 1e-5, |q| past 65504 infinite). 64 sequences
+// to 4096: 93 -> 95 us.
 // The VALU form it replaces there (attn_kernel, one 32-position split per
 // workgroup) wrote and re-read a partial per 32 positions, half as many bytes
 // again as the K/V rows.
@@ -882,8 +888,10 @@ __global__ __launch_bounds__(HD, 2) void mq_attn_kernel(MqArgs a) {
     }
   };
 
-  load_step(0);
-  // q as the scores' B operand: column c = (part c/8, head c%8), dims 256 wd + 32j + 8q .. +7
+  // q as the scores' B operand: column c = (part c/8, head c%8), dims 256 wd + 32j + 8q .. +7.
+  // (At head dim 512 its loads go first and it is converted while the rows are
+  // in flight: its scale needs the maximum of the whole half.)
+  if constexpr (HD == 256) load_step(0);
   const float* qg = a.q + ((size_t)seq * a.nqh + kvh * MQ_G + (c & 7)) * HD + 256 * wd;
   float4 qr[16];
 #pragma unroll
@@ -891,6 +899,18 @@ __global__ __launch_bounds__(HD, 2) void mq_attn_kernel(MqArgs a) {
     qr[2 * j] = *(const float4*)(qg + 32 * j + 8 * q);
     qr[2 * j + 1] = *(const float4*)(qg + 32 * j + 8 * q + 4);
   }
+  float up = 1.f, unscale = 1.f;
+  if constexpr (HD == 512) {
+    __builtin_amdgcn_sched_barrier(0);
+    load_step(0);
+    __builtin_amdgcn_sched_barrier(0);
+    float am = 0.f;
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+      am = fmaxf(fmaxf(fmaxf(am, fabsf(qr[j].x)), fmaxf(fabsf(qr[j].y), fabsf(qr[j].z))), fabsf(qr[j].w));
+    up = g4d::f16_pair_scale(g4d::xmax32(g4d::xmax16(am)), unscale);
+  }
+  constexpr float kP = HD == 512 ? 16384.f : 1.f;  // P's scale
   mh8 qb[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
@@ -898,8 +918,9 @@ __global__ __launch_bounds__(HD, 2) void mq_attn_kernel(MqArgs a) {
                          qr[2 * j + 1].x, qr[2 * j + 1].y, qr[2 * j + 1].z, qr[2 * j + 1].w};
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const _Float16 hi = (_Float16)xs[e];
-      qb[j][e] = c < 8 ? hi : (_Float16)(xs[e] - (float)hi);
+      const float x = HD == 512 ? xs[e] * up : xs[e];
+      const _Float16 hi = (_Float16)x;
+      qb[j][e] = c < 8 ? hi : (_Float16)(x - (float)hi);
     }
   }
   store_step();
@@ -916,15 +937,43 @@ __global__ __launch_bounds__(HD, 2) void mq_attn_kernel(MqArgs a) {
 
     // ---- scores of the wave's 16 positions ----
     mf4 S = mf4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (HD == 256) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const mh8 A = *(const mh8*)(kt + (16 * wt + c) * RS + 256 * wd + 32 * j + 8 * q);
-      S = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, qb[j], S, 0, 0, 0);
-    }
-    if constexpr (HD == 512) {
-      xs[w * 64 + l] = S;
+      for (int j = 0; j < 8; ++j) {
+        const mh8 A = *(const mh8*)(kt + (16 * wt + c) * RS + 256 * wd + 32 * j + 8 * q);
+        S = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, qb[j], S, 0, 0, 0);
+      }
+    } else {
+      // (f32 additions in pairs: a product that adds to a running accumulator
+      // does so with about twice their error)
+      mf4 half[2];
+#pragma unroll
+      for (int j = 0; j < 8; j += 4) {
+        mf4 t[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const mh8 A = *(const mh8*)(kt + (16 * wt + c) * RS + 256 * wd + 32 * (j + e) + 8 * q);
+          t[e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, qb[j + e], mf4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        }
+        half[j / 4] = (t[0] + t[1]) + (t[2] + t[3]);
+      }
+      S = half[0] + half[1];
+      xs[w * 64 + l] = S * unscale;
       __syncthreads();
       S = xs[wt * 64 + l] + xs[(wt + 4) * 64 + l];
+    }
+    if constexpr (HD == 512) {
+      // (a non-finite K element: the hi product decides, the lo one may cancel its infinity)
+      bool fin = true;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) fin = fin && fabsf(S[i]) < INFINITY;
+      if (__ballot(!fin)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float other = g4d::dpp<kDppRor8>(S[i]), hi = c < 8 ? S[i] : other;
+          S[i] = fabsf(hi) < INFINITY ? S[i] : (c < 8 ? hi : 0.f);
+        }
+      }
     }
     float sc[4];
     float mx = -INFINITY;
@@ -959,8 +1008,9 @@ __global__ __launch_bounds__(HD, 2) void mq_attn_kernel(MqArgs a) {
     mh4 P;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const _Float16 hi = (_Float16)p[i];
-      P[i] = c < 8 ? hi : (_Float16)(p[i] - (float)hi);
+      const float x = HD == 512 ? p[i] * kP : p[i];
+      const _Float16 hi = (_Float16)x;
+      P[i] = c < 8 ? hi : (_Float16)(x - (float)hi);
     }
 #pragma unroll
     for (int dt = 0; dt < 16; ++dt) {
@@ -1016,7 +1066,7 @@ __global__ __launch_bounds__(HD, 2) void mq_attn_kernel(MqArgs a) {
       L += wgt * lw[ww * MQ_G + h];
       o += wgt * ow[(ww * MQ_G + h) * HD + tid];
     }
-    ws_o[(part + h) * HD + tid] = o;
+    ws_o[(part + h) * HD + tid] = HD == 512 ? o * (1.f / kP) : o;
     if (tid == 0) {
       ws_m[part + h] = M;
       ws_l[part + h] = L;
