@@ -11,10 +11,23 @@
 //  * a wave holds 16 columns (2 tokens x 8 heads) of q in registers as f16 hi
 //    and lo operands and their output sums; K and V rows go through LDS in
 //    steps of 32 positions, K as stored, V transposed;
-//  * scores S[pos][col] = K q with v_mfma_f32_16x16x32_f16, hi then lo; the
-//    online softmax runs per column; two 16-position score tiles are the
+//  * scores S[pos][col] = K q with v_mfma_f32_16x16x32_f16, lo apart from hi;
+//    the online softmax runs per column; two 16-position score tiles are the
 //    32-deep A operand of the PV product as they lie in registers (V's
 //    positions are stored in that order), P as f16 hi + lo;
+//  * q is scaled by a power of two that brings its column's (and half's)
+//    largest element to 2^13 .. 2^14, P (at most 1) by 2^14: hi + lo then hold
+//    22 bits of every element down to 2^-16 of the largest, and no f32 q
+//    overflows f16. Unscaled, a P below 2^-25 left the product (not the sum
+//    it is divided by): one key 14 above 1900 others, whose V is small, cost
+//    3e-5 of the result;
+//  * sums over steps and over more than 32 dims (64 at head dim 256) are f32
+//    additions: a product that adds to a running accumulator does so with about
+//    twice an addition's error. Relative error against float64, 100 rows to
+//    1900 positions, scores of spread 2: head dim 256 3.5e-7 and 512 3.5e-7,
+//    where the ragged step's attention has 5.6e-7 (mq_attn_kernel) and 3.5e-7
+//    (attn_kernel); chained products on unscaled pairs had 8e-7 and 7e-7. Cost
+//    of both at 1900 rows: head dim 256, window 512 53 -> 55 us, 512 225 -> 237;
 //  * head dim 512: two waves share a column tile, each 256 dims; their score
 //    halves are added through LDS (same order in both);
 //  * a token's V rows are those of its own window only: in the steps at the
@@ -40,6 +53,7 @@ typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 constexpr int TOK = 8;     // tokens of a workgroup
 constexpr int HEADS = 8;   // query heads per KV head
 constexpr uint32_t kMaxSplit = 16;
+constexpr float kPScale = 16384.f;  // P's power of two
 
 struct PaArgs {
   const float* q;  // [T][nqh][HD], normed and roped
@@ -68,8 +82,10 @@ struct Shape {
   static constexpr int PV = PK / 4;              // 4-position x 8-dim pieces of V
 };
 
-// exp(x) for x <= 0 on the hardware exp2
-__device__ __forceinline__ float exp_h(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504f); }
+// The softmax works in powers of two (scores times log2 e, in one product with
+// the scale): P = exp2(fma(score, scale, -max)) rounds its exponent once.
+constexpr float kLog2e = 1.44269504f;
+__device__ __forceinline__ float exp2_h(float x) { return __builtin_amdgcn_exp2f(x); }
 
 template <int HD>
 __global__ __launch_bounds__(Shape<HD>::NT, 2) void pf_attn_kernel(PaArgs a) {
@@ -159,22 +175,34 @@ __global__ __launch_bounds__(Shape<HD>::NT, 2) void pf_attn_kernel(PaArgs a) {
     }
   };
 
-  // q of this wave's columns: dims 256 wd + 32 j + 8q .. + 7, hi and lo
+  // q of this wave's columns: dims 256 wd + 32 j + 8q .. + 7, times 2^k, hi and lo
   h8 qh[8], ql[8];
+  float unscale;  // 2^-k
   {
     const uint32_t tok = min(t0 + 2u * wc + (c >> 3), a.T - 1);
     const float* qg = a.q + ((size_t)tok * a.nqh + kvh * HEADS + (c & 7)) * HD + 256 * wd + 8 * q;
+    float x[8][8], am = 0.f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const float4 x0 = *(const float4*)(qg + 32 * j), x1 = *(const float4*)(qg + 32 * j + 4);
-      const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+      const float y[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        qh[j][e] = (_Float16)x[e];
-        ql[j][e] = (_Float16)(x[e] - (float)qh[j][e]);
+        x[j][e] = y[e];
+        am = fmaxf(am, fabsf(y[e]));
       }
     }
+    const float up = g4d::f16_pair_scale(g4d::xmax32(g4d::xmax16(am)), unscale);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float y = x[j][e] * up;
+        qh[j][e] = (_Float16)y;
+        ql[j][e] = (_Float16)(y - (float)qh[j][e]);
+      }
   }
+  const float s_scale = (HD == 256 ? a.scale * unscale : a.scale) * kLog2e;
 
   // V operands of the even and odd dim tiles (positions 4q .. + 3 and 16 + 4q .. + 3; rows 16 dt apart)
   const _Float16* vb[2];
@@ -194,20 +222,32 @@ __global__ __launch_bounds__(Shape<HD>::NT, 2) void pf_attn_kernel(PaArgs a) {
     __syncthreads();
     if (k + 1 < n) load_step(step_of(k + 1));  // (uniform) in flight during this step
 
+    const f4 zero = f4{0.f, 0.f, 0.f, 0.f};
+    constexpr int CH = HD == 256 ? 2 : 4;
     f4 S[NPT];
 #pragma unroll
     for (int p = 0; p < NPT; ++p) {
-      S[p] = f4{0.f, 0.f, 0.f, 0.f};
+      f4 Sl = zero;
+      S[p] = zero;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const h8 A = *(const h8*)(kt + (16 * p + c) * KS + 256 * wd + 32 * j + 8 * q);
-        S[p] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, qh[j], S[p], 0, 0, 0);
-        S[p] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, ql[j], S[p], 0, 0, 0);
+      for (int j = 0; j < 8; j += CH) {
+        f4 t[CH];
+#pragma unroll
+        for (int e = 0; e < CH; ++e) {
+          const h8 A = *(const h8*)(kt + (16 * p + c) * KS + 256 * wd + 32 * (j + e) + 8 * q);
+          t[e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, qh[j + e], HD == 256 && e ? t[e - 1] : zero, 0, 0, 0);
+          Sl = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, ql[j + e], Sl, 0, 0, 0);
+        }
+        if constexpr (HD == 256) S[p] += t[1];
+        else S[p] += (t[0] + t[1]) + (t[2] + t[3]);
       }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)  // (a non-finite K element: the lo product may cancel the hi one's infinity)
+        S[p][i] = fabsf(S[p][i]) < INFINITY ? S[p][i] + Sl[i] : S[p][i];
     }
     if constexpr (HD == 512) {
 #pragma unroll
-      for (int p = 0; p < NPT; ++p) xs[(w * NPT + p) * 64 + l] = S[p];
+      for (int p = 0; p < NPT; ++p) xs[(w * NPT + p) * 64 + l] = S[p] * unscale;
       __syncthreads();
 #pragma unroll
       for (int p = 0; p < NPT; ++p)
@@ -215,28 +255,29 @@ __global__ __launch_bounds__(Shape<HD>::NT, 2) void pf_attn_kernel(PaArgs a) {
     }
     float mx = -INFINITY;
     const uint32_t pb = lo + st * STEP + 4u * q;
+    auto live = [&](int p, int i) {
+      const uint32_t pos = pb + 16u * p + i;
+      return decltype(inside)::value || (pos >= clo && pos < chi);
+    };
 #pragma unroll
     for (int p = 0; p < NPT; ++p)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t pos = pb + 16u * p + i;
-        S[p][i] = decltype(inside)::value || (pos >= clo && pos < chi) ? S[p][i] * a.scale : -INFINITY;
-        mx = fmaxf(mx, S[p][i]);
-      }
+      for (int i = 0; i < 4; ++i) mx = fmaxf(mx, live(p, i) ? S[p][i] * s_scale : -INFINITY);
     mx = g4d::xmax32(g4d::xmax16(mx));
-    const float m_new = fmaxf(m_run, mx);
-    const float alpha = m_new == -INFINITY ? 1.f : exp_h(m_run - m_new);
+    const float m_new = fmaxf(m_run, mx), m_fin = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = exp2_h(m_run - m_fin);  // (nothing live yet: 0, times sums of 0)
     float ps = 0.f;
     h8 ph[NPT / 2], pl[NPT / 2];
 #pragma unroll
     for (int p = 0; p < NPT; ++p)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float e = S[p][i] == -INFINITY ? 0.f : exp_h(S[p][i] - m_new);
+        const float e = live(p, i) ? exp2_h(fmaf(S[p][i], s_scale, -m_fin)) : 0.f;
         ps += e;
-        const _Float16 h = (_Float16)e;
+        const float es = e * kPScale;
+        const _Float16 h = (_Float16)es;
         ph[p / 2][(p & 1) * 4 + i] = h;
-        pl[p / 2][(p & 1) * 4 + i] = (_Float16)(e - (float)h);
+        pl[p / 2][(p & 1) * 4 + i] = (_Float16)(es - (float)h);
       }
     ps = g4d::xsum32(g4d::xsum16(ps));
     l_run = l_run * alpha + ps;
@@ -255,8 +296,8 @@ __global__ __launch_bounds__(Shape<HD>::NT, 2) void pf_attn_kernel(PaArgs a) {
 #pragma unroll
       for (int dt = 0; dt < 16; ++dt) {
         const h8 B = *(const h8*)(vb[dt & 1] + dt * 16 * VS);
-        O[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph[0], B, O[dt], 0, 0, 0);
-        O[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl[0], B, O[dt], 0, 0, 0);
+        const f4 t = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl[0], B, zero, 0, 0, 0);
+        O[dt] += __builtin_amdgcn_mfma_f32_16x16x32_f16(ph[0], B, t, 0, 0, 0);
       }
     } else {
       u32x4 keep[2];  // of this lane's eight positions, each token's
@@ -278,7 +319,7 @@ __global__ __launch_bounds__(Shape<HD>::NT, 2) void pf_attn_kernel(PaArgs a) {
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
           const h8 Bk = __builtin_bit_cast(h8, B & keep[k]);
-          o[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl[0], Bk, f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+          o[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl[0], Bk, zero, 0, 0, 0);
           o[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph[0], Bk, o[k], 0, 0, 0);
         }
 #pragma unroll
@@ -295,7 +336,7 @@ __global__ __launch_bounds__(Shape<HD>::NT, 2) void pf_attn_kernel(PaArgs a) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const float L = __shfl(l_run, 4 * q + i, 64);
-    inv[i] = a.nsplit > 1 ? 1.f : (L > 0.f ? 1.0f / L : 0.f);
+    inv[i] = (a.nsplit > 1 ? 1.f : (L > 0.f ? 1.0f / L : 0.f)) * (1.f / kPScale);
   }
   const uint32_t tok = t0 + 2u * wc + (q >> 1);
   const size_t rows = (size_t)a.T * a.nqh;
@@ -328,7 +369,7 @@ __global__ __launch_bounds__(HD / 4) void merge_kernel(const float* ws, float* o
   const float* ow = ws + (size_t)2 * nsplit * rows;
   for (uint32_t s = 0; s < nsplit; ++s) {
     const float m = ws[(size_t)s * rows + row];
-    const float wt = m == -INFINITY ? 0.f : exp_h(m - M);
+    const float wt = m == -INFINITY ? 0.f : exp2_h(m - M);
     const float4 v = *(const float4*)(ow + ((size_t)s * rows + row) * HD + d);
     L += wt * lw[(size_t)s * rows + row];
     o.x += wt * v.x;

@@ -1,4 +1,5 @@
-"""The matrix-core attention of the paged batch at head dim 512 over the range of f32 queries and probabilities, against float64:
+"""The matrix-core attentions of the paged batch (head dim 512) and of a prompt
+(256 and 512) over the range of f32 queries and probabilities, against float64:
 a dominant key whose V is small (the other probabilities, down to e^-20, carry
 the result), query elements past f16's largest, tiny queries, and a key whose
 score is -infinity through an infinite element (left out, as exp(-inf) is 0).
@@ -49,6 +50,15 @@ def _want(q, k, v, n):
     return p @ v[:n].astype(np.float64) / p.sum(-1, keepdims=True)
 
 
+def _pool(x, table, hd):
+    """Positions to pool rows."""
+    pool = np.zeros((table.size * PAGE, hd), np.float16)
+    for i, pg in enumerate(table):
+        rows = x[i * PAGE:(i + 1) * PAGE]
+        pool[pg * PAGE:pg * PAGE + len(rows)] = rows
+    return pool
+
+
 def _check(got, want, what):
     assert np.all(np.isfinite(got)), what
     r = O.rel_l2(got.reshape(-1), want.reshape(-1))
@@ -78,3 +88,20 @@ def test_paged_512(ctx, kind):
     got = out.download(np.float32).reshape(q.shape)
     for b in range(B):
         _check(got[b], _want(q[b], k, v, lens[b]), (kind, b))
+
+
+@pytest.mark.parametrize("hd", [256, 512])
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("T", [11, 300])  # windows split over workgroups, and whole
+def test_prompt(ctx, kind, hd, T):
+    q, k, v = _inputs(kind, hd, T)
+    table = np.random.default_rng(3).permutation(-(-L // PAGE)).astype(np.int32)
+    lens = (L - T + 1 + np.arange(T)).astype(np.uint32)
+    p = ctx.paged_fused_params(T, NQ, 1, hd, PAGE, table.size, L, table.size, 0, 1e-6, 1e4, 0)
+    out = ctx.from_numpy(np.full(q.size, 7.0, np.float32))
+    ctx.prefillAttn(ctx.from_numpy(q), ctx.from_numpy(_pool(k, table, hd).view(np.uint16)),
+                    ctx.from_numpy(_pool(v, table, hd).view(np.uint16)), ctx.from_numpy(table), ctx.from_numpy(lens),
+                    out, p, ctx.alloc(ctx.prefill_attn_workspace_bytes(p)))
+    got = out.download(np.float32).reshape(q.shape)
+    for t in sorted({0, 1, 7, 8, T // 2, T - 1}):
+        _check(got[t], _want(q[t], k, v, int(lens[t])), (kind, t))
