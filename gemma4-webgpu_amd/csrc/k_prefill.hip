@@ -24,8 +24,14 @@
 //    waiting for memory (gate/up 2 x 6144 x 1536 at 1900 vectors 241 -> 156
 //    us, o 101 -> 55, down 12288 wide 159 -> 138: 1040 TFLOP/s of f16 products).
 // The arithmetic is that of mmf_kernel: x * 2^e as f16 hi + lo, exact f16
-// sc * q (Q6_K rounds once above 2048), f32 accumulation over a super-block,
-// then d and 2^-e in f32.
+// sc * q (Q6_K rounds once above 2048), f32 accumulation over half a
+// super-block, then d and 2^-e in f32 (the min term with the super-block's
+// second half). mmf_kernel keeps the hi and the lo sums of a super-block apart,
+// which there are no registers for here; the lo products before the hi ones and
+// half the chain match its accuracy. Relative error against float64, 64 vectors
+// x 1536, Q4_K and Q6_K with exact operands: mmf_kernel 2.7e-7 and 1.23e-7, this
+// 2.7e-7 and 1.24e-7, whole super-blocks with hi first 3.4e-7 and 1.6e-7 (gate/up
+// 2 x 12288 at 1900 vectors 331 us so, 329 as it is; o 55.5 and 56; q/k/v 66 both).
 #include <algorithm>
 
 #include "mm_operand.hpp"
@@ -149,6 +155,7 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 template <int QT, int RT, int MODE, int SG>
 __global__ __launch_bounds__(NT, 2) void pf_gemm_kernel(PfArgs a) {
   static_assert(MODE == 0 || RT == 4, "gate/up: two tiles of each");
+  constexpr int FL = 4;  // sub-blocks accumulated on the matrix cores
   __shared__ __align__(16) uint8_t b0[SUB], b1[SUB], b2[SUB], b3[SUB];
   __shared__ __align__(16) uint8_t vaux[2 * VAUX_LDS], waux[QT == 2 ? 16 : 2 * 4 * WAUX_LDS];
   uint8_t* const ring[4] = {b0, b1, b2, b3};
@@ -238,17 +245,17 @@ __global__ __launch_bounds__(NT, 2) void pf_gemm_kernel(PfArgs a) {
       stage(j * 8u + s + 3, ring[(s + 3) & 3]);
       __builtin_amdgcn_sched_barrier(0);
       const uint8_t* base = ring[s & 3] + l * 16;
-      const bool first = SG == 2 ? (s & 3) == 0 : s == 0;
+      const bool first = s % FL == 0;
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const h8 bh = *(const h8*)(base + t * 2048), bl = *(const h8*)(base + t * 2048 + 1024);
 #pragma unroll
         for (int r = 0; r < RT; ++r)
-          C[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, A[s & 3][r]), bh,
+          C[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, A[s & 3][r]), bl,
                                                            first ? f4{0.f, 0.f, 0.f, 0.f} : C[r][t], 0, 0, 0);
 #pragma unroll
         for (int r = 0; r < RT; ++r)
-          C[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, A[s & 3][r]), bl, C[r][t], 0, 0, 0);
+          C[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, A[s & 3][r]), bh, C[r][t], 0, 0, 0);
       }
       // the next tile's operands are read while one is multiplied
       __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);  // LDS reads
@@ -263,9 +270,11 @@ __global__ __launch_bounds__(NT, 2) void pf_gemm_kernel(PfArgs a) {
         for (int r = 0; r < RT; ++r) A[s & 3][r] = Ap[r][off];
       }
       __builtin_amdgcn_sched_barrier(0);
-      // the super-block's (or its half's) d, min term and 2^-e
-      if (s == 7 || (SG == 2 && s == 3)) {
+      // these sub-blocks' products times d and 2^-e; the super-block's (or its
+      // half's) min term with its last ones
+      if (s % FL == FL - 1) {
         const int hf = SG == 2 ? s >> 2 : 0;
+        const bool mins = QT == 0 && (s == 7 || (SG == 2 && s == 3));
         const uint8_t* vb = vaux + (j & 1u) * VAUX_LDS;
         const uint8_t* wb = waux + (QT == 2 ? 0u : ((j & 1u) * 4u + w) * WAUX_LDS);
         float fs[4];
@@ -273,7 +282,7 @@ __global__ __launch_bounds__(NT, 2) void pf_gemm_kernel(PfArgs a) {
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           fs[t] = *(const float*)(vb + (PfOps::SCALE - PfOps::SUMS) + t * 128 + hf * 64 + c * 4);
-          if constexpr (QT == 0) bm[t] = *(const h8*)(vb + t * 1024 + l * 16);
+          if (mins) bm[t] = *(const h8*)(vb + t * 1024 + l * 16);
         }
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
@@ -287,7 +296,7 @@ __global__ __launch_bounds__(NT, 2) void pf_gemm_kernel(PfArgs a) {
             const f4 d = *(const f4*)(xr + 16 * q);
             f4 dm = f4{0.f, 0.f, 0.f, 0.f};
             h8 am = h8{};
-            if constexpr (QT == 0) {
+            if (mins) {
               dm = *(const f4*)(xr + Aux<0>::DM + 16 * q);
               const h2 mn = *(const h2*)(xr + Aux<0>::MN + 4 * l);
               // slots 8q .. 8q + 7 are sub-blocks 2q and 2q + 1: a half is two lane groups
@@ -296,12 +305,10 @@ __global__ __launch_bounds__(NT, 2) void pf_gemm_kernel(PfArgs a) {
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
               f4 cm = f4{0.f, 0.f, 0.f, 0.f};
-              if constexpr (QT == 0) cm = __builtin_amdgcn_mfma_f32_16x16x32_f16(am, bm[t], cm, 0, 0, 0);
+              if (mins) cm = __builtin_amdgcn_mfma_f32_16x16x32_f16(am, bm[t], cm, 0, 0, 0);
 #pragma unroll
-              for (int i = 0; i < 4; ++i) {
-                if constexpr (QT == 0) acc[r][t][i] += fs[t] * (d[i] * C[r][t][i] - dm[i] * cm[i]);
-                else acc[r][t][i] += fs[t] * d[i] * C[r][t][i];
-              }
+              for (int i = 0; i < 4; ++i)
+                acc[r][t][i] += mins ? fs[t] * (d[i] * C[r][t][i] - dm[i] * cm[i]) : fs[t] * d[i] * C[r][t][i];
             }
           }
         }

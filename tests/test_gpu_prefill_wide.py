@@ -76,6 +76,76 @@ def test_prefill_matmul(ctx, wtype, rows, N, T, split):
         assert O.rel_l2(got, want) <= BAR[wtype]
 
 
+def _exact_blocks(wtype, seed, M, N):
+    """Blocks whose operands f16 holds exactly (Q6_K: scales of at most 63), and their float64 values."""
+    b = (synth.q4k_centered if wtype == "q4k" else synth.q6k_wide)(seed, M * N // 256)
+    if wtype == "q6k":
+        r = b.reshape(-1, 210)
+        r[:, 192:208] = (r[:, 192:208].view(np.int8) // 2).view(np.uint8)
+    return b, (O.np_dequant_q4k if wtype == "q4k" else O.np_dequant_q6k)(b).astype(np.float64).reshape(M, N)
+
+
+def _step_ops(ctx, X):
+    T, N = X.shape
+    ops, xn = ctx.alloc(ctx.batch_operand_bytes(N, T)), ctx.zeros(T * N, np.float32)
+    ctx.batchPrep(ctx.from_numpy(X), 1, None, None, None, None, xn, N, T, ops=ops)
+    return ops, xn
+
+
+@pytest.mark.parametrize("wtype", ["q4k", "q6k"])
+def test_prefill_matmul_as_exact_as_the_step(ctx, wtype):
+    """The same vectors through the ragged step's matmul and the prompt's: what is left with exact weights, f32
+    accumulation, is of the same size (1.1: the two sum in different orders; measured 0.98 and 1.01)."""
+    M, N, T = 2048, 1536, 64
+    b, w = _exact_blocks(wtype, 51, M, N)
+    X = O.gen_normal_f32(52, T * N).reshape(T, N)
+    want = X.astype(np.float64) @ w.T
+    db, y = ctx.from_numpy(b), ctx.zeros(T * M, np.float32)
+    ops, xn = _step_ops(ctx, X)
+    ctx.matmulSegmentsBatchPartial(wtype, xn, [db], [y], [M], N, T, 1, ops=ops)
+    step = O.rel_l2(y.download(np.float32).reshape(T, M), want)
+    ctx.prefillMatmul(wtype, [db], [y], [M], N, _ops(ctx, X), T, ctx.alloc(ctx.prefill_weight_bytes(wtype, [M], N)))
+    got = O.rel_l2(y.download(np.float32).reshape(T, M), want)
+    print(f"[prefill] {wtype}: step {step:.3e}, prompt {got:.3e}", flush=True)
+    assert got <= 1.1 * step
+
+
+@pytest.mark.parametrize("spread", [0, 20])  # of the gate rows' sizes from 32 to 32, in powers of two
+def test_prefill_ffn_as_exact_as_the_step(ctx, spread):
+    """The same through gate/up and down: the step scales the product per 32 rows, the prompt per 128."""
+    M, N, T, H = 6144, 1536, 64, 1536
+    gb, _ = _exact_blocks("q4k", 53, M, N)
+    if spread:
+        r = gb.reshape(M, -1, 144)
+        d = r[:, :, 0:2].copy().view(np.float16)[..., 0].astype(np.float32)
+        s = np.exp2(-spread * np.random.default_rng(4).random(M // 32)).repeat(32).astype(np.float32)
+        d = (d * s[:, None]).astype(np.float16)
+        r[:, :, 0:2] = d[..., None].view(np.uint8)
+        r[:, :, 2:4] = (d.astype(np.float32) * 7.5).astype(np.float16)[..., None].view(np.uint8)
+    g = O.np_dequant_q4k(gb).astype(np.float64).reshape(M, N)
+    (ub, u), (db, d) = _exact_blocks("q4k", 54, M, N), _exact_blocks("q6k", 55, H, M)
+    X = O.gen_normal_f32(56, T * N, 0.0, 0.5).reshape(T, N)
+    a = X.astype(np.float64) @ g.T
+    t = np.clip(0.7978845608028654 * a * (1 + 0.044715 * a * a), -15, 15)
+    want = (0.5 * a * (1 + np.tanh(t)) * (X.astype(np.float64) @ u.T)) @ d.T
+    dg, du, dd = (ctx.from_numpy(x) for x in (gb, ub, db))
+    y = ctx.zeros(M // 256 * T * H, np.float32)
+
+    def total(n):
+        return O.rel_l2(y.download(np.float32, n * T * H).reshape(n, T, H).astype(np.float64).sum(0), want)
+
+    ops, xn = _step_ops(ctx, X)
+    prod = ctx.alloc(ctx.batch_sub_operand_bytes(M, T))
+    ctx.gateUpGeluBatchOps(xn, ops, dg, du, None, prod, M, N, T)
+    step = total(ctx.matmulSubBatchPartial(prod, dd, y, H, M, T, M // 768))
+    prod = ctx.alloc(ctx.prefill_operand_bytes(M, T))
+    wops = ctx.alloc(max(ctx.prefill_weight_bytes("q4k", [M, M], N), ctx.prefill_weight_bytes("q6k", [H], M)))
+    ctx.prefillGateUp("q4k", dg, du, _ops(ctx, X), prod, M, N, T, wops)
+    got = total(ctx.prefillMatmul("q6k", [dd], [y], [H], M, prod, T, wops, M // 768, product_ops=True))
+    print(f"[prefill] ffn spread {spread}: step {step:.3e}, prompt {got:.3e}", flush=True)
+    assert got <= 1.1 * step
+
+
 @pytest.mark.parametrize("wtype", ["q4k", "q6k", "f16"])
 @pytest.mark.parametrize("down", ["q4k", "q6k", "f16"])
 def test_prefill_ffn(ctx, wtype, down):
