@@ -373,6 +373,9 @@ struct PfOps {
   static constexpr uint32_t SUMS = 4 * MAIN_T;
   static constexpr uint32_t SCALE = SUMS + 4 * 1024;
   static constexpr uint32_t BYTES = SCALE + 4 * 128;
+  // the third f16 term x * 2^e - hi - lo, in a buffer of its own (f16 matrices):
+  // [4 vector tiles][8 sub-blocks][64 lanes] 16 B
+  static constexpr uint32_t LO_BYTES = 4 * 8192;
 };
 
 }  // namespace g4d

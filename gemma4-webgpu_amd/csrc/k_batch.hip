@@ -73,6 +73,7 @@ struct BPrepArgs {
   const uint16_t* scale;  // mode 2: h = (residual + norm(x)) * f16 scale (NULL: 1)
   const float* mul;       // PRO 3: x' = gelu(x) * mul[v * mul_stride + k]
   uint32_t mul_stride;
+  uint8_t* ops_lo;        // PF: optional: the third f16 term, [B / 64][K/256][PfOps::LO_BYTES]
 };
 
 __device__ __forceinline__ float4 mulw(float4 x, uint2 w, float s) {
@@ -217,6 +218,16 @@ __global__ __launch_bounds__(PNT) void bprep_kernel(BPrepArgs a) {
     uint8_t* mp = base + t * Ops::MAIN_T + s * 2048 + (c + 16u * q) * 16 + (kk & 7) * 2;
     *(uint2*)mp = make_uint2(pack_h2(hi[0], hi[1]), pack_h2(hi[2], hi[3]));
     *(uint2*)(mp + 1024) = make_uint2(pack_h2(lo[0], lo[1]), pack_h2(lo[2], lo[3]));
+    if constexpr (PF) {
+      if (a.ops_lo) {  // (uniform)
+        _Float16 l3[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) l3[e] = (_Float16)((xs[e] - (float)hi[e]) - (float)lo[e]);
+        uint8_t* lp = a.ops_lo + ((size_t)(v / 64) * BPR + sb) * g4d::PfOps::LO_BYTES + t * 8192u + s * 1024u +
+                      (c + 16u * q) * 16 + (kk & 7) * 2;
+        *(uint2*)lp = make_uint2(pack_h2(l3[0], l3[1]), pack_h2(l3[2], l3[3]));
+      }
+    }
     if ((lane & 7) == 0) {
       const _Float16 p0 = (_Float16)sum;
       const float r1 = sum - (float)p0;
@@ -1165,6 +1176,12 @@ int g4_batchPrepScale(g4_ctx* ctx, const float* x, uint32_t nparts, const uint16
 int g4_prefillPrep(g4_ctx* ctx, const float* x, uint32_t nparts, const uint16_t* w1, const float* residual,
                    const uint16_t* out_scale, const uint16_t* w2, float* h_out, float* out, void* ops, uint32_t N,
                    uint32_t vectors, float eps) {
+  return g4_prefillPrepLo(ctx, x, nparts, w1, residual, out_scale, w2, h_out, out, ops, nullptr, N, vectors, eps);
+}
+
+int g4_prefillPrepLo(g4_ctx* ctx, const float* x, uint32_t nparts, const uint16_t* w1, const float* residual,
+                     const uint16_t* out_scale, const uint16_t* w2, float* h_out, float* out, void* ops,
+                     void* ops_lo, uint32_t N, uint32_t vectors, float eps) {
   G4_ENTER(ctx);
   G4_REQUIRE(x && nparts >= 1 && (out || ops || h_out), "g4_prefillPrep: null buffer or no parts");
   G4_REQUIRE(vectors >= 1 && vectors <= 65535, "g4_prefillPrep: %u vectors outside 1..65535", vectors);
@@ -1175,13 +1192,21 @@ int g4_prefillPrep(g4_ctx* ctx, const float* x, uint32_t nparts, const uint16_t*
   G4_REQUIRE((((uintptr_t)x | (uintptr_t)out | (uintptr_t)ops | (uintptr_t)residual | (uintptr_t)h_out) & 15) == 0,
              "g4_prefillPrep: buffers must be 16-byte aligned");
   G4_REQUIRE((((uintptr_t)w1 | (uintptr_t)w2) & 7) == 0, "g4_prefillPrep: norm weights must be 8-byte aligned");
+  G4_REQUIRE(ops || !ops_lo, "g4_prefillPrep: ops_lo without ops");
+  G4_REQUIRE(((uintptr_t)ops_lo & 15) == 0, "g4_prefillPrep: ops_lo must be 16-byte aligned");
   const int pro = !w1 ? 0 : (residual ? 2 : 1);
-  const BPrepArgs p{x, nparts, vectors, w1, residual, w2, h_out, out, eps, (uint8_t*)ops, 4, out_scale};
+  BPrepArgs p{x, nparts, vectors, w1, residual, w2, h_out, out, eps, (uint8_t*)ops, 4, out_scale};
+  p.ops_lo = (uint8_t*)ops_lo;
   return bprep_launch<true>(ctx, N, pro, p);
 }
 
 int g4_prefillPleGated(g4_ctx* ctx, const float* gate, uint32_t nparts, const float* ple_inputs, uint32_t stride,
                        uint32_t layer_offset, float* out, void* ops, uint32_t vectors) {
+  return g4_prefillPleGatedLo(ctx, gate, nparts, ple_inputs, stride, layer_offset, out, ops, nullptr, vectors);
+}
+
+int g4_prefillPleGatedLo(g4_ctx* ctx, const float* gate, uint32_t nparts, const float* ple_inputs, uint32_t stride,
+                         uint32_t layer_offset, float* out, void* ops, void* ops_lo, uint32_t vectors) {
   G4_ENTER(ctx);
   G4_REQUIRE(gate && nparts >= 1 && ple_inputs && (out || ops), "g4_prefillPleGated: null buffer or no parts");
   G4_REQUIRE(vectors >= 1 && vectors <= 65535, "g4_prefillPleGated: %u vectors outside 1..65535", vectors);
@@ -1189,7 +1214,10 @@ int g4_prefillPleGated(g4_ctx* ctx, const float* gate, uint32_t nparts, const fl
              "g4_prefillPleGated: slice %u of rows of %u", layer_offset, stride);
   G4_REQUIRE((((uintptr_t)gate | (uintptr_t)ple_inputs | (uintptr_t)out | (uintptr_t)ops) & 15) == 0,
              "g4_prefillPleGated: buffers must be 16-byte aligned");
+  G4_REQUIRE(ops || !ops_lo, "g4_prefillPleGated: ops_lo without ops");
+  G4_REQUIRE(((uintptr_t)ops_lo & 15) == 0, "g4_prefillPleGated: ops_lo must be 16-byte aligned");
   BPrepArgs p{};
+  p.ops_lo = (uint8_t*)ops_lo;
   p.x = gate;
   p.nparts = nparts;
   p.B = vectors;

@@ -73,6 +73,7 @@ struct PfArgs {
   PfWeights w;
   uint32_t rtn, K, nsb;  // row tiles; width; super-blocks of the width
   const uint8_t* ops;    // [T / 64][nsb][PfOps::BYTES]
+  const uint8_t* ops_lo; // f16 matrices: the third term, [T / 64][nsb][PfOps::LO_BYTES], or null
   uint32_t T, ntt;       // vectors, tiles of 64
   uint32_t ksplit, kc;
   uint32_t groups, items;
@@ -151,14 +152,25 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // exchange; the product leaves as the down projection's operands, one
 // 32-row sub-block per wave, one 2^e per vector and 128 rows (the four
 // waves' maxima meet in LDS). SG: scale groups per super-block of the
-// operands read (2 for that product, 1 otherwise: both halves equal).
-template <int QT, int RT, int MODE, int SG>
+// operands read (2 for that product, 1 otherwise: both halves equal). TERMS 3
+// (f16 matrices): the vectors with their third term, each sub-block's products
+// added in f32 to the super-block's sums (even and odd ones apart), for the
+// accuracy of the f32 matvec (hmv_kernel) that f16 matrices take in a step:
+// relative error against float64, 256 x 1536 and 1536 x 256, matvec 9.2e-8 and
+// 7.8e-8, three terms 9.4e-8 and 6.9e-8, two terms 1.6e-7 and 1.5e-7. At 1900
+// vectors the 8960-row model projection 123 -> 208 us for it, a layer's gate and
+// proj 14 -> 17 and 14 -> 16 (as matvecs all of them took 9.5 ms of that prompt).
+template <int QT, int RT, int MODE, int SG, int TERMS = 2>
 __global__ __launch_bounds__(NT, 2) void pf_gemm_kernel(PfArgs a) {
   static_assert(MODE == 0 || RT == 4, "gate/up: two tiles of each");
-  constexpr int FL = 4;  // sub-blocks accumulated on the matrix cores
+  static_assert(TERMS == 2 || (QT == 2 && RT == 2 && MODE == 0 && SG == 1), "three terms: f16 rows");
+  constexpr int FL = TERMS == 3 ? 8 : 4;  // sub-blocks summed before d and 2^-e
   __shared__ __align__(16) uint8_t b0[SUB], b1[SUB], b2[SUB], b3[SUB];
   __shared__ __align__(16) uint8_t vaux[2 * VAUX_LDS], waux[QT == 2 ? 16 : 2 * 4 * WAUX_LDS];
+  constexpr uint32_t SUB3 = TERMS == 3 ? 4 * 1024 : 16;
+  __shared__ __align__(16) uint8_t c0[SUB3], c1[SUB3], c2[SUB3], c3[SUB3];
   uint8_t* const ring[4] = {b0, b1, b2, b3};
+  uint8_t* const ring3[4] = {c0, c1, c2, c3};
   const int tid = threadIdx.x, l = tid & 63, q = l >> 4, c = l & 15;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   // Workgroups go to the XCDs in turn (linear id mod 8): XCD x takes the
@@ -181,22 +193,25 @@ __global__ __launch_bounds__(NT, 2) void pf_gemm_kernel(PfArgs a) {
 #pragma unroll
   for (int r = 0; r < RT; ++r) Ap[r] = (const u32x4*)a.w.A + ((size_t)rt[r] * nsub + sb0 * 8u) * 64u;
   const uint8_t* Bg = a.ops + ((size_t)tt * a.nsb + sb0) * PfOps::BYTES;
+  const uint8_t* Bl = TERMS == 3 ? a.ops_lo + ((size_t)tt * a.nsb + sb0) * PfOps::LO_BYTES : nullptr;
   const uint32_t nwalk = a.kc * 8u;  // sub-blocks of the walk
 
-  f4 acc[RT][4], C[RT][4];
+  f4 acc[RT][4], C[RT][TERMS == 3 ? 8 : 4];  // (three terms: the even and the odd sub-blocks' sums)
 #pragma unroll
   for (int r = 0; r < RT; ++r)
 #pragma unroll
     for (int t = 0; t < 4; ++t) acc[r][t] = f4{0.f, 0.f, 0.f, 0.f};
 
-  // sub-block u of the walk: 8 pieces of 1 KB, two per wave (vector tile w,
-  // hi and lo); past the end the last one again, so that every turn issues
+  // sub-block u of the walk: 8 or 12 pieces of 1 KB, each wave its vector
+  // tile's two or three; past the end the last one again, so that every turn issues
   // the same number of loads
-  auto stage = [&](uint32_t u, uint8_t* buf) {
+  auto stage = [&](uint32_t u, uint8_t* buf, uint8_t* buf3) {
     const uint32_t v = min(u, nwalk - 1u);
     const uint8_t* src = Bg + (size_t)(v >> 3) * PfOps::BYTES + w * PfOps::MAIN_T + (v & 7u) * 2048u + l * 16;
     to_lds(src, buf + w * 2048);
     to_lds(src + 1024, buf + w * 2048 + 1024);
+    if constexpr (TERMS == 3)
+      to_lds(Bl + (size_t)(v >> 3) * PfOps::LO_BYTES + w * 8192u + (v & 7u) * 1024u + l * 16, buf3 + w * 1024);
   };
   // the values super-block j's sums need
   auto stage_aux = [&](uint32_t j) {
@@ -223,7 +238,7 @@ __global__ __launch_bounds__(NT, 2) void pf_gemm_kernel(PfArgs a) {
   u32x4 A[4][RT];
   stage_aux(0);
 #pragma unroll
-  for (int s = 0; s < 3; ++s) stage(s, ring[s]);
+  for (int s = 0; s < 3; ++s) stage(s, ring[s], ring3[s]);
 #pragma unroll
   for (int s = 0; s < 4; ++s)
 #pragma unroll
@@ -235,34 +250,48 @@ __global__ __launch_bounds__(NT, 2) void pf_gemm_kernel(PfArgs a) {
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
       // Sub-block s of the vectors, requested three turns ago, has arrived
-      // once at most what was issued after it is in flight: two turns' two
+      // once at most what was issued after it is in flight: two turns' TERMS
       // LDS loads and three turns' RT weight loads (the others only make the
       // wait stricter). Every wave has also left sub-block s - 1, whose
       // buffer takes sub-block s + 3.
-      wait_vmcnt<4 + 3 * RT>();
+      wait_vmcnt<2 * TERMS + 3 * RT>();
       lds_barrier();
       if (s == 4) stage_aux(j + 1);
-      stage(j * 8u + s + 3, ring[(s + 3) & 3]);
+      stage(j * 8u + s + 3, ring[(s + 3) & 3], ring3[(s + 3) & 3]);
       __builtin_amdgcn_sched_barrier(0);
       const uint8_t* base = ring[s & 3] + l * 16;
       const bool first = s % FL == 0;
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const h8 bh = *(const h8*)(base + t * 2048), bl = *(const h8*)(base + t * 2048 + 1024);
+        auto mul = [&](int r, h8 b, f4 z) {
+          return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, A[s & 3][r]), b, z, 0, 0, 0);
+        };
+        const f4 zero = f4{0.f, 0.f, 0.f, 0.f};
+        if constexpr (TERMS == 3) {
+          const h8 b3 = *(const h8*)(ring3[s & 3] + t * 1024 + l * 16);
+          f4 z[RT];
 #pragma unroll
-        for (int r = 0; r < RT; ++r)
-          C[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, A[s & 3][r]), bl,
-                                                           first ? f4{0.f, 0.f, 0.f, 0.f} : C[r][t], 0, 0, 0);
+          for (int r = 0; r < RT; ++r) z[r] = mul(r, b3, zero);
 #pragma unroll
-        for (int r = 0; r < RT; ++r)
-          C[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, A[s & 3][r]), bh, C[r][t], 0, 0, 0);
+          for (int r = 0; r < RT; ++r) z[r] = mul(r, bl, z[r]);
+#pragma unroll
+          for (int r = 0; r < RT; ++r) z[r] = mul(r, bh, z[r]);
+#pragma unroll
+          for (int r = 0; r < RT; ++r) C[r][4 * (s & 1) + t] = s < 2 ? z[r] : C[r][4 * (s & 1) + t] + z[r];
+        } else {
+#pragma unroll
+          for (int r = 0; r < RT; ++r) C[r][t] = mul(r, bl, first ? zero : C[r][t]);
+#pragma unroll
+          for (int r = 0; r < RT; ++r) C[r][t] = mul(r, bh, C[r][t]);
+        }
       }
       // the next tile's operands are read while one is multiplied
-      __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);  // LDS reads
+      __builtin_amdgcn_sched_group_barrier(0x100, 2 * TERMS, 0);  // LDS reads
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 2 * RT, 0);  // MFMAs
-        if (t < 2) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, TERMS * RT, 0);  // MFMAs
+        if (t < 2) __builtin_amdgcn_sched_group_barrier(0x100, TERMS, 0);
       }
       {  // the weight operands four sub-blocks on (past the end: the last again)
         const uint32_t off = min(j * 8u + s + 4, nwalk - 1u) * 64u + l;
@@ -290,7 +319,8 @@ __global__ __launch_bounds__(NT, 2) void pf_gemm_kernel(PfArgs a) {
 #pragma unroll
             for (int t = 0; t < 4; ++t)
 #pragma unroll
-              for (int i = 0; i < 4; ++i) acc[r][t][i] += fs[t] * C[r][t][i];
+              for (int i = 0; i < 4; ++i)
+                acc[r][t][i] += fs[t] * (TERMS == 3 ? C[r][t][i] + C[r][TERMS == 3 ? 4 + t : t][i] : C[r][t][i]);
           } else {
             const uint8_t* xr = wb + r * Aux<QT>::BYTES;
             const f4 d = *(const f4*)(xr + 16 * q);
@@ -467,7 +497,7 @@ int unpack(g4_ctx* ctx, int wtype, const PfArgs& a) {
   return G4_OK;
 }
 
-template <int RT, int MODE, int SG>
+template <int RT, int MODE, int SG, int F16_TERMS = 2>
 int gemm_qt(g4_ctx* ctx, int wtype, PfArgs a, uint32_t groups) {
   a.groups = groups;
   a.items = groups * a.ksplit * a.ntt;
@@ -476,7 +506,7 @@ int gemm_qt(g4_ctx* ctx, int wtype, PfArgs a, uint32_t groups) {
     if constexpr (RT == 4 && SG == 2) return G4_ERR_UNSUPPORTED;  // (pick_plan)
     else hipLaunchKernelGGL((pf_gemm_kernel<0, RT, MODE, SG>), grid, dim3(NT), 0, ctx->stream, a);
   } else if (wtype == 1) hipLaunchKernelGGL((pf_gemm_kernel<1, RT, MODE, SG>), grid, dim3(NT), 0, ctx->stream, a);
-  else hipLaunchKernelGGL((pf_gemm_kernel<2, RT, MODE, SG>), grid, dim3(NT), 0, ctx->stream, a);
+  else hipLaunchKernelGGL((pf_gemm_kernel<2, RT, MODE, SG, F16_TERMS>), grid, dim3(NT), 0, ctx->stream, a);
   G4_LAUNCHED(ctx, "prefill_gemm");
   return G4_OK;
 }
@@ -530,9 +560,24 @@ int g4_prefillOperandBytes(uint32_t N, uint32_t vectors, size_t* bytes) {
   return G4_OK;
 }
 
+int g4_prefillOperandLoBytes(uint32_t N, uint32_t vectors, size_t* bytes) {
+  G4_REQUIRE(bytes && N >= 256 && N % 256 == 0 && N <= 65536 && vectors >= 1 && vectors <= 65535,
+             "g4_prefillOperandLoBytes: bad shape");
+  *bytes = (size_t)ceil_div(vectors, 64) * (N / 256) * PfOps::LO_BYTES;
+  return G4_OK;
+}
+
 int g4_prefillMatmul(g4_ctx* ctx, int wtype, const void* const* weights, float* const* outputs, const uint32_t* rows,
                      int nseg, uint32_t N, const void* ops, int product_ops, uint32_t vectors, void* wops,
                      size_t wops_bytes, uint32_t max_ksplit, uint32_t* ksplit) {
+  return g4_prefillMatmulLo(ctx, wtype, weights, outputs, rows, nseg, N, ops, nullptr, product_ops, vectors, wops,
+                            wops_bytes, max_ksplit, ksplit);
+}
+
+int g4_prefillMatmulLo(g4_ctx* ctx, int wtype, const void* const* weights, float* const* outputs,
+                       const uint32_t* rows, int nseg, uint32_t N, const void* ops, const void* ops_lo,
+                       int product_ops, uint32_t vectors, void* wops, size_t wops_bytes, uint32_t max_ksplit,
+                       uint32_t* ksplit) {
   G4_ENTER(ctx);
   uint32_t rtn;
   int rc = check_pf(__func__, wtype, weights, rows, nseg, N, ops, vectors, wops, wops_bytes, rtn);
@@ -540,16 +585,20 @@ int g4_prefillMatmul(g4_ctx* ctx, int wtype, const void* const* weights, float* 
   G4_REQUIRE(outputs && ksplit && max_ksplit >= 1, "g4_prefillMatmul: null outputs, null ksplit or max_ksplit 0");
   for (int i = 0; i < nseg; ++i)
     G4_REQUIRE(outputs[i] && ((uintptr_t)outputs[i] & 15) == 0, "g4_prefillMatmul: output %d null or misaligned", i);
+  G4_REQUIRE(!ops_lo || (wtype == 2 && !product_ops && ((uintptr_t)ops_lo & 15) == 0),
+             "g4_prefillMatmul: ops_lo goes with f16 rows, not with product_ops, 16-byte aligned");
   PfArgs a = pf_args(weights, outputs, rows, nseg, N, ops, vectors, wops, rtn);
   rc = unpack(ctx, wtype, a);
   if (rc) return rc;
+  a.ops_lo = (const uint8_t*)ops_lo;
   // (Q4_K over a product's operands: with four row tiles the two scale groups'
-  // min products spill 289 registers)
-  const Plan p = pick_plan(ctx, a, max_ksplit, wtype == 0 && product_ops);
+  // min products spill 289 registers; so do the sums of three terms)
+  const Plan p = pick_plan(ctx, a, max_ksplit, (wtype == 0 && product_ops) || ops_lo);
   a.ksplit = p.ks;
   a.kc = a.nsb / p.ks;
   *ksplit = p.ks;
   const uint32_t groups = ceil_div(rtn, 4u * (uint32_t)p.rt);
+  if (ops_lo) return gemm_qt<2, 0, 1, 3>(ctx, wtype, a, groups);
   if (product_ops) return p.rt == 4 ? gemm_qt<4, 0, 2>(ctx, wtype, a, groups) : gemm_qt<2, 0, 2>(ctx, wtype, a, groups);
   return p.rt == 4 ? gemm_qt<4, 0, 1>(ctx, wtype, a, groups) : gemm_qt<2, 0, 1>(ctx, wtype, a, groups);
 }

@@ -217,6 +217,11 @@ SIGNATURES = {
     "g4_prefillPrep": (_I, [_P, _P, _U32, _P, _P, _P, _P, _P, _P, _P, _U32, _U32, _F]),
     "g4_prefillMatmul": (_I, [_P, _I, ctypes.POINTER(_P), ctypes.POINTER(_P), ctypes.POINTER(_U32), _I, _U32, _P, _I,
                               _U32, _P, _SZ, _U32, ctypes.POINTER(_U32)]),
+    "g4_prefillOperandLoBytes": (_I, [_U32, _U32, ctypes.POINTER(_SZ)]),
+    "g4_prefillPrepLo": (_I, [_P, _P, _U32, _P, _P, _P, _P, _P, _P, _P, _P, _U32, _U32, _F]),
+    "g4_prefillMatmulLo": (_I, [_P, _I, ctypes.POINTER(_P), ctypes.POINTER(_P), ctypes.POINTER(_U32), _I, _U32, _P,
+                                _P, _I, _U32, _P, _SZ, _U32, ctypes.POINTER(_U32)]),
+    "g4_prefillPleGatedLo": (_I, [_P, _P, _U32, _P, _U32, _U32, _P, _P, _P, _U32]),
     "g4_prefillGateUp": (_I, [_P, _I, _P, _P, _P, _P, _U32, _U32, _U32, _P, _SZ]),
     "g4_prefillPleGated": (_I, [_P, _P, _U32, _P, _U32, _U32, _P, _P, _U32]),
     "g4_prefillAttnPrologue": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, PagedAttnFusedParams, _P, _U32]),

@@ -1201,12 +1201,14 @@ class BatchDecoder(_SyntheticModel):
 
     def _wide_prefill(self) -> bool:
         """Whether prompts may take the layers many rows at a time: one prompt
-        per decoder, longer than a chunk, and widths the prefill kernels take."""
+        per decoder, longer than a chunk, and widths and formats the prefill kernels take (an f16 FFN stays
+        with the steps, whose sums are f32: the fused gate/up has no third term)."""
         s = self.s
         return (self.shared_pages and self.embedding is not None and self.max_seq > self.B
                 and s.hidden in (1536, 2048) and s.ple_dim in (0, 256) and s.n_q_heads == 8 * s.n_kv_heads
                 and all(s.hd(il) in (256, 512) and s.q_dim_of(il) in (1536, 2048, 4096) and s.ffn_of(il) % 256 == 0
-                        and L.qt["wgate"] == L.qt["wup"] for il, L in enumerate(self.layers)))
+                        and L.qt["wgate"] == L.qt["wup"] and "f16" not in (L.qt["wgate"], L.qt["wdown"])
+                        for il, L in enumerate(self.layers)))
 
     def _build_wide(self) -> None:
         c, s, R, f32 = self.ctx, self.s, self.wide_rows, np.float32
@@ -1235,8 +1237,16 @@ class BatchDecoder(_SyntheticModel):
                                [(s.n_layers * s.ple_dim, H), (s.ple_dim, H), (H, s.ple_dim)]))
         w["wops"] = c.empty(need, np.uint8)
         w["attn_ws"] = c.empty(ws, np.uint8)
+        # f16 matrices take their vectors' third term too (f32's 24 bits, as in a step)
+        lo = c.prefill_operand_lo_bytes
+        f16 = {m: any(L.qt[m] == "f16" for L in self.layers) for m in ("wq", "wk", "wv", "wo")}
+        if s.ple_dim or f16["wq"] or f16["wk"] or f16["wv"]:
+            w["xops_lo"] = c.empty(lo(H, R), np.uint8)
+        if f16["wo"]:
+            w["aops_lo"] = c.empty(lo(s.q_dim, R), np.uint8)
         if s.ple_dim:
             LD = s.n_layers * s.ple_dim
+            w["pops_lo"] = c.empty(lo(s.ple_dim, R), np.uint8)
             w.update(hidden3=c.empty(R * H, f32), ple_projected=c.empty(R * LD, f32), ple_inputs=c.empty(R * LD, f32),
                      ple_gate=c.empty(R * H, f32), pops=c.empty(ob(s.ple_dim, R), np.uint8), ple_out=c.empty(R * H, f32))
 
@@ -1273,8 +1283,10 @@ class BatchDecoder(_SyntheticModel):
         c.embeddingLookupBatch(self.embedding, s.vocab, w["hidden"], H, tokens, n)
         if s.ple_dim:
             LD = s.n_layers * s.ple_dim
-            c.prefillPrep(w["hidden"], 1, None, None, None, None, None, None, H, n, s.eps, ops=w["xops"])
-            c.prefillMatmul("f16", [self.ple_model_proj], [w["ple_projected"]], [LD], H, w["xops"], n, wops)
+            c.prefillPrep(w["hidden"], 1, None, None, None, None, None, None, H, n, s.eps, ops=w["xops"],
+                          ops_lo=w["xops_lo"])
+            c.prefillMatmul("f16", [self.ple_model_proj], [w["ple_projected"]], [LD], H, w["xops"], n, wops,
+                            ops_lo=w["xops_lo"])
             c.pleStage1Fuse(w["ple_projected"], self.ple_proj_norm, self.ple_table, s.vocab, w["ple_inputs"],
                             s.n_layers, s.ple_dim, s.eps, tokens_dev=tokens, count=n)
         max_ks = max(1, self.wide_parts // (n * H))
@@ -1282,23 +1294,27 @@ class BatchDecoder(_SyntheticModel):
         for il in range(s.n_layers + 1):
             L = self.layers[il] if il < s.n_layers else None
             norm, ops = (L.attn_norm, w["xops"]) if L else (None, None)
+            groups = []
+            if L:
+                Q, KV, I = s.q_dim_of(il), s.kv_dim_of(il), s.ffn_of(il)
+                prod = s.is_producer(il)
+                outs = [w["q"], w["k"], w["v"]] if prod else [w["q"]]
+                groups = qkv_groups(L, outs, [Q, KV, KV] if prod else [Q])
+            lo = w["xops_lo"] if any(g[0] == "f16" for g in groups) else None
             if il == 0:
-                c.prefillPrep(w["hidden"], 1, norm, None, None, None, None, None, H, n, s.eps, ops=ops)
+                c.prefillPrep(w["hidden"], 1, norm, None, None, None, None, None, H, n, s.eps, ops=ops, ops_lo=lo)
             elif s.ple_dim:
                 prev = self.layers[il - 1]
                 c.prefillPrep(w["ple_out"], 1, prev.ple_post_norm, w["hidden3"], prev.ple_scale, norm, w["hidden"],
-                              None, H, n, s.eps, ops=ops)
+                              None, H, n, s.eps, ops=ops, ops_lo=lo)
             else:
                 prev = self.layers[il - 1]
                 c.prefillPrep(w["parts"], nd, prev.post_ffn_norm, w["hidden2"], None, norm, w["hidden"], None, H, n,
-                              s.eps, ops=ops)
+                              s.eps, ops=ops, ops_lo=lo)
             if L is None:
                 return
-            Q, KV, I = s.q_dim_of(il), s.kv_dim_of(il), s.ffn_of(il)
-            prod = s.is_producer(il)
-            outs = [w["q"], w["k"], w["v"]] if prod else [w["q"]]
-            for qt, ws, go, gr in qkv_groups(L, outs, [Q, KV, KV] if prod else [Q]):
-                c.prefillMatmul(qt, ws, go, gr, H, w["xops"], n, wops)
+            for qt, ws, go, gr in groups:
+                c.prefillMatmul(qt, ws, go, gr, H, w["xops"], n, wops, ops_lo=lo if qt == "f16" else None)
             # every row of the pass is appended before any is read
             glob = s.is_global(il)
             p = c.paged_fused_params(n, s.n_q_heads, s.n_kv_heads, s.hd(il), self.page_size, self.max_pages, end,
@@ -1308,8 +1324,9 @@ class BatchDecoder(_SyntheticModel):
                                   self.rope_freqs, w["q"], L.k_cache if prod else None, L.v_cache if prod else None,
                                   self.page_table, lens, p, self.rope_cs[glob], self.rope_rows)
             c.prefillAttn(w["q"], L.k_cache, L.v_cache, self.page_table, lens, w["attn"], p, w["attn_ws"])
-            c.prefillPrep(w["attn"], 1, None, None, None, None, None, None, Q, n, s.eps, ops=w["aops"])
-            no = c.prefillMatmul(L.qt["wo"], [L.wo], [w["parts"]], [H], Q, w["aops"], n, wops, max_ks)
+            lo = w["aops_lo"] if L.qt["wo"] == "f16" else None
+            c.prefillPrep(w["attn"], 1, None, None, None, None, None, None, Q, n, s.eps, ops=w["aops"], ops_lo=lo)
+            no = c.prefillMatmul(L.qt["wo"], [L.wo], [w["parts"]], [H], Q, w["aops"], n, wops, max_ks, ops_lo=lo)
             c.prefillPrep(w["parts"], no, L.post_attn_norm, w["hidden"], None, L.pre_ffn_norm, w["hidden2"], None, H,
                           n, s.eps, ops=w["xops"])
             c.prefillGateUp(L.qt["wgate"], L.wgate, L.wup, w["xops"], w["fops"], I, H, n, wops)
@@ -1318,10 +1335,13 @@ class BatchDecoder(_SyntheticModel):
             if s.ple_dim:
                 D = s.ple_dim
                 c.prefillPrep(w["parts"], nd, L.post_ffn_norm, w["hidden2"], None, None, w["hidden3"], None, H, n,
-                              s.eps, ops=w["xops"])
-                ng = c.prefillMatmul("f16", [L.ple_gate], [w["ple_gate"]], [D], H, w["xops"], n, wops, H // 256)
-                c.prefillPleGated(w["ple_gate"], ng, w["ple_inputs"], s.n_layers * D, il * D, None, n, ops=w["pops"])
-                c.prefillMatmul("f16", [L.ple_proj], [w["ple_out"]], [H], D, w["pops"], n, wops)
+                              s.eps, ops=w["xops"], ops_lo=w["xops_lo"])
+                ng = c.prefillMatmul("f16", [L.ple_gate], [w["ple_gate"]], [D], H, w["xops"], n, wops, H // 256,
+                                     ops_lo=w["xops_lo"])
+                c.prefillPleGated(w["ple_gate"], ng, w["ple_inputs"], s.n_layers * D, il * D, None, n, ops=w["pops"],
+                                  ops_lo=w["pops_lo"])
+                c.prefillMatmul("f16", [L.ple_proj], [w["ple_out"]], [H], D, w["pops"], n, wops,
+                                ops_lo=w["pops_lo"])
 
     def capture(self, sample: str = "argmax"):
         """The step as a HIP graph; each replay appends one token per sequence."""

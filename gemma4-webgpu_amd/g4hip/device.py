@@ -341,22 +341,31 @@ class Context:
         check(lib().g4_prefillOperandBytes(N, vectors, ctypes.byref(n)))
         return int(n.value)
 
+    @staticmethod
+    def prefill_operand_lo_bytes(N: int, vectors: int) -> int:
+        n = ctypes.c_size_t()
+        check(lib().g4_prefillOperandLoBytes(N, vectors, ctypes.byref(n)))
+        return int(n.value)
+
     def prefillPrep(self, x_parts: Ptr, nparts: int, w1: Ptr, residual: Ptr, out_scale: Ptr, w2: Ptr, h_out: Ptr,
-                    out: Ptr, N: int, vectors: int, eps: float = 1e-6, ops: Ptr = None) -> None:
-        """batchPrepScale over any number of vectors; `ops` receives the prefill matmul's operand blocks."""
-        check(lib().g4_prefillPrep(self.h, _p(x_parts), nparts, _p(w1), _p(residual), _p(out_scale), _p(w2),
-                                   _p(h_out), _p(out), _p(ops), N, vectors, eps))
+                    out: Ptr, N: int, vectors: int, eps: float = 1e-6, ops: Ptr = None, ops_lo: Ptr = None) -> None:
+        """batchPrepScale over any number of vectors; `ops` receives the prefill matmul's operand blocks,
+        `ops_lo` their third term (f16 matrices: f32's 24 bits instead of 22)."""
+        check(lib().g4_prefillPrepLo(self.h, _p(x_parts), nparts, _p(w1), _p(residual), _p(out_scale), _p(w2),
+                                     _p(h_out), _p(out), _p(ops), _p(ops_lo), N, vectors, eps))
 
     def prefillMatmul(self, wtype: str, weights, outputs, rows, N: int, ops: Ptr, vectors: int, wops: Buffer,
-                      max_ksplit: int = 1, product_ops: bool = False) -> int:
-        """outputs[i] [ksplit][vectors][rows[i]] = each weight times the vectors behind `ops`; returns ksplit."""
+                      max_ksplit: int = 1, product_ops: bool = False, ops_lo: Ptr = None) -> int:
+        """outputs[i] [ksplit][vectors][rows[i]] = each weight times the vectors behind `ops` (f16: and
+        `ops_lo`); returns ksplit."""
         n = len(weights)
         W = (ctypes.c_void_p * n)(*[_p(w).value for w in weights])
         Y = (ctypes.c_void_p * n)(*[_p(y).value for y in outputs])
         R = (ctypes.c_uint32 * n)(*rows)
         ks = ctypes.c_uint32(0)
-        check(lib().g4_prefillMatmul(self.h, PREFILL_TYPES[wtype], W, Y, R, n, N, _p(ops), int(product_ops), vectors,
-                                     _p(wops), wops.nbytes, max_ksplit, ctypes.byref(ks)))
+        check(lib().g4_prefillMatmulLo(self.h, PREFILL_TYPES[wtype], W, Y, R, n, N, _p(ops), _p(ops_lo),
+                                       int(product_ops), vectors, _p(wops), wops.nbytes, max_ksplit,
+                                       ctypes.byref(ks)))
         return int(ks.value)
 
     def prefillGateUp(self, wtype: str, w_gate: Ptr, w_up: Ptr, ops: Ptr, product_ops: Ptr, M: int, N: int,
@@ -366,10 +375,10 @@ class Context:
                                      M, N, vectors, _p(wops), wops.nbytes))
 
     def prefillPleGated(self, gate: Ptr, nparts: int, ple_inputs: Ptr, stride: int, layer_offset: int, out: Ptr,
-                        vectors: int, ops: Ptr = None) -> None:
+                        vectors: int, ops: Ptr = None, ops_lo: Ptr = None) -> None:
         """gelu(gate) * ple_inputs' slice of every vector, as values and / or proj's operand blocks."""
-        check(lib().g4_prefillPleGated(self.h, _p(gate), nparts, _p(ple_inputs), stride, layer_offset, _p(out),
-                                       _p(ops), vectors))
+        check(lib().g4_prefillPleGatedLo(self.h, _p(gate), nparts, _p(ple_inputs), stride, layer_offset, _p(out),
+                                         _p(ops), _p(ops_lo), vectors))
 
     def prefillAttnPrologue(self, q_raw: Ptr, k_raw: Ptr, v_raw: Ptr, q_norm_w: Ptr, k_norm_w: Ptr, rope_freqs: Ptr,
                             q_out: Ptr, k_pool: Ptr, v_pool: Ptr, page_table: Ptr, lens: Ptr, params,

@@ -718,6 +718,19 @@ int g4_prefillPrep(g4_ctx* ctx, const float* x, uint32_t nparts, const uint16_t*
 int g4_prefillMatmul(g4_ctx* ctx, int wtype, const void* const* weights, float* const* outputs,
                      const uint32_t* rows, int nseg, uint32_t N, const void* ops, int product_ops,
                      uint32_t vectors, void* wops, size_t wops_bytes, uint32_t max_ksplit, uint32_t* ksplit);
+/* With f32's 24 bits of every vector, for f16 matrices (wtype 2): g4_prefillPrepLo
+ * and g4_prefillPleGatedLo also write ops_lo, the third f16 term of each element
+ * (g4_prefillOperandLoBytes(N, vectors) bytes; NULL: as the forms without it),
+ * which g4_prefillMatmulLo multiplies too. `ops` alone hold 22 bits. ops_lo goes
+ * with wtype 2 and not with product_ops. */
+int g4_prefillOperandLoBytes(uint32_t N, uint32_t vectors, size_t* bytes);
+int g4_prefillPrepLo(g4_ctx* ctx, const float* x, uint32_t nparts, const uint16_t* w1,
+                     const float* residual, const uint16_t* out_scale, const uint16_t* w2, float* h_out,
+                     float* out, void* ops, void* ops_lo, uint32_t N, uint32_t vectors, float eps);
+int g4_prefillMatmulLo(g4_ctx* ctx, int wtype, const void* const* weights, float* const* outputs,
+                       const uint32_t* rows, int nseg, uint32_t N, const void* ops, const void* ops_lo,
+                       int product_ops, uint32_t vectors, void* wops, size_t wops_bytes, uint32_t max_ksplit,
+                       uint32_t* ksplit);
 /* gelu(W_gate . x) * (W_up . x), left as operand blocks of the down
  * projection (product_ops, g4_prefillOperandBytes(M, vectors) bytes); M a
  * multiple of 256. */
@@ -730,6 +743,9 @@ int g4_prefillGateUp(g4_ctx* ctx, int wtype, const void* w_gate, const void* w_u
  * and / or the operand blocks of proj (g4_prefillOperandBytes(256, vectors)). */
 int g4_prefillPleGated(g4_ctx* ctx, const float* gate, uint32_t nparts, const float* ple_inputs,
                        uint32_t stride, uint32_t layer_offset, float* out, void* ops, uint32_t vectors);
+int g4_prefillPleGatedLo(g4_ctx* ctx, const float* gate, uint32_t nparts, const float* ple_inputs,
+                         uint32_t stride, uint32_t layer_offset, float* out, void* ops, void* ops_lo,
+                         uint32_t vectors);
 /* The attention of p.num_seqs rows (1..65535) of one sequence over one page
  * list (page_table [p.max_pages]; every row may read every position below
  * its length, so appending all rows first makes the pass causal).

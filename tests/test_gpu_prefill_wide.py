@@ -110,6 +110,42 @@ def test_prefill_matmul_as_exact_as_the_step(ctx, wtype):
     assert got <= 1.1 * step
 
 
+@pytest.mark.parametrize("M,N,T,split", [
+    (256, 1536, 129, 6),   # per-layer embeddings: the gate
+    (1536, 256, 70, 1),    # and proj, one super-block
+    (8960, 1536, 65, 1),   # the model projection, one vector past a tile
+    (33, 2048, 1, 8),      # rows that fill no tile, one vector
+])
+@pytest.mark.parametrize("heavy", [False, True])
+def test_prefill_f16_as_exact_as_the_matvec(ctx, M, N, T, split, heavy):
+    """f16 rows with the vectors' third term against the f32 matvec of a step (1.1, the one vector 1.5: sums in
+    different orders, over fewer of them), also where a few elements are far above the others."""
+    wb, w = _weights("f16", 57, M, N)
+    X = O.gen_normal_f32(58, T * N).reshape(T, N)
+    if heavy:
+        X *= np.exp(3.0 * np.random.default_rng(5).standard_normal(X.shape)).astype(np.float32)
+    want = X.astype(np.float64) @ w.T
+    dw, dx, y = ctx.from_numpy(wb), ctx.from_numpy(X), ctx.zeros(split * T * M, np.float32)
+    ctx.matmulF16(dx, dw, y, M, N, T)
+    step = O.rel_l2(y.download(np.float32, T * M).reshape(T, M), want)
+    ops, lo = ctx.alloc(ctx.prefill_operand_bytes(N, T)), ctx.alloc(ctx.prefill_operand_lo_bytes(N, T))
+    if N == 256:  # (gelu(20) is 20 in f32)
+        one = ctx.from_numpy(np.full(T * N, 20.0, np.float32))
+        ctx.prefillPleGated(one, 1, ctx.from_numpy(X / np.float32(20.0)), N, 0, None, T, ops=ops, ops_lo=lo)
+        want = (np.float32(20.0) * (X / np.float32(20.0))).astype(np.float64) @ w.T
+    else:
+        ctx.prefillPrep(dx, 1, None, None, None, None, None, None, N, T, ops=ops, ops_lo=lo)
+    ks = ctx.prefillMatmul("f16", [dw], [y], [M], N, ops, T, ctx.alloc(ctx.prefill_weight_bytes("f16", [M], N)),
+                           split, ops_lo=lo)
+    parts = y.download(np.float32, ks * T * M).reshape(ks, T, M)
+    got = parts[0].copy()
+    for p in parts[1:]:
+        got += p
+    got = O.rel_l2(got, want)
+    print(f"[prefill] f16 {M}x{N} T={T} heavy={heavy}: matvec {step:.3e}, prompt {got:.3e}", flush=True)
+    assert got <= (1.5 if T == 1 else 1.1) * step
+
+
 @pytest.mark.parametrize("spread", [0, 20])  # of the gate rows' sizes from 32 to 32, in powers of two
 def test_prefill_ffn_as_exact_as_the_step(ctx, spread):
     """The same through gate/up and down: the step scales the product per 32 rows, the prompt per 128."""
