@@ -101,6 +101,15 @@ __global__ __launch_bounds__(NT) void advance_many_kernel(uint32_t* p, uint32_t 
   if (i < n) p[i] += delta;
 }
 
+// Bound by its writes: 32 rows of 262144 words (a batch's logits) are 32 MB.
+__global__ __launch_bounds__(NT) void repeat_row_kernel(uint32_t* rows, uint32_t words, uint32_t src, uint32_t first,
+                                                        uint32_t count) {
+  const uint32_t i = blockIdx.x * NT + threadIdx.x;
+  if (i >= words) return;
+  const uint32_t x = rows[(size_t)src * words + i];
+  for (uint32_t r = 0; r < count; ++r) rows[((size_t)first + r) * words + i] = x;
+}
+
 __global__ __launch_bounds__(NT) void softcap_kernel(float* logits, uint32_t n, float cap) {
   const uint32_t i = blockIdx.x * NT + threadIdx.x;
   if (i >= n) return;
@@ -530,6 +539,18 @@ int g4_embeddingLookupBatch(g4_ctx* ctx, const uint16_t* embedding, uint32_t num
   G4_REQUIRE(tokens_dev, "g4_embeddingLookupBatch: null tokens");
   G4_REQUIRE(count <= 65535, "g4_embeddingLookupBatch: %u rows > 65535", count);
   return embedding_lookup(ctx, embedding, num_rows, output, g4_embedding_params{hidden_size, 0u}, tokens_dev, count);
+}
+
+int g4_repeatRow(g4_ctx* ctx, void* rows, uint32_t words, uint32_t src, uint32_t first, uint32_t count) {
+  G4_ENTER(ctx);
+  G4_REQUIRE(rows && ((uintptr_t)rows & 3) == 0, "g4_repeatRow: null or misaligned buffer");
+  G4_REQUIRE((src < first || src - first >= count) && (uint64_t)first + count <= UINT32_MAX,
+             "g4_repeatRow: row %u is one of the %u from %u", src, count, first);
+  if (!words || !count) return G4_OK;
+  hipLaunchKernelGGL(repeat_row_kernel, dim3(ceil_div(words, NT)), dim3(NT), 0, ctx->stream, (uint32_t*)rows, words,
+                     src, first, count);
+  G4_LAUNCHED(ctx, "repeat_row");
+  return G4_OK;
 }
 
 int g4_logitSoftcap(g4_ctx* ctx, float* logits, g4_softcap_params p) {

@@ -1161,8 +1161,9 @@ class BatchDecoder(_SyntheticModel):
         prefill matmuls (each weight read and unpacked once per pass), and
         leaves the same rows as its last chunk would. A short last
         chunk repeats its last token and position in the spare rows
-        (identical rows, identical writes); a prompt of one chunk leaves out
-        spare rows past the 16 or 32 that hold it. Returns the row of the final
+        (identical rows, identical writes); a prompt of one chunk runs without
+        the spare rows past the 16 or 32 that hold it, whose residual rows,
+        logits and samples are then copies of the last token's. Returns the row of the final
         chunk that holds the prompt's last token: its logits and `tokens`
         entry are the first sample. probe (tests): passed to every chunk's
         step."""
@@ -1194,6 +1195,12 @@ class BatchDecoder(_SyntheticModel):
             self.ctx.copy(self.seq_lens, dpos.offset(4 * B * k), 4 * B)
             self.lens_host = cpos[B * k:B * (k + 1)].copy()
             self.step(sample, probe=probe, head=k == nch - 1, rows=rows)
+        if rows < B:  # the rows left out: the last token's again, as in a step over all B
+            outs = [(self.hidden, self.s.hidden)]
+            if self.lm_head is not None:
+                outs += [(self.logits, self.s.vocab)] + ([(self.tokens, 1)] if sample == "argmax" else [(self.topk, 512)])
+            for buf, words in outs:
+                self.ctx.repeatRow(buf, words, n - 1, rows, B - rows)
         self.ctx.sync()
         dtok.free()
         dpos.free()

@@ -737,6 +737,11 @@ class Context:
         check(lib().g4_embeddingLookupBatch(self.h, _p(embedding), num_rows, _p(out), hidden_size, _p(tokens_dev),
                                             count))
 
+    def repeatRow(self, rows: Buffer, words: int, src: int, first: int, count: int) -> None:
+        """Rows first .. first + count - 1 of `rows` [][words] (32-bit words) become copies of row src."""
+        assert 4 * words * max(src + 1, first + count) <= rows.nbytes, "repeatRow past the end of the buffer"
+        check(lib().g4_repeatRow(self.h, _p(rows), words, src, first, count))
+
     def advancePosition(self, position_dev: Ptr, delta: int = 1) -> None:
         check(lib().g4_advancePosition(self.h, _p(position_dev), delta))
 

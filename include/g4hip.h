@@ -510,6 +510,10 @@ int g4_embeddingLookup_dev(g4_ctx* ctx, const uint16_t* embedding, uint32_t num_
 int g4_embeddingLookupBatch(g4_ctx* ctx, const uint16_t* embedding, uint32_t num_rows, float* output,
                             uint32_t hidden_size, const uint32_t* tokens_dev, uint32_t count);
 
+/* Rows first .. first + count - 1 of `rows` [][words] (32-bit words) = row src,
+ * which is none of them: the spare rows of a batch that runs without them. */
+int g4_repeatRow(g4_ctx* ctx, void* rows, uint32_t words, uint32_t src, uint32_t first, uint32_t count);
+
 /* *position_dev += delta on the stream: the device-side step counter that lets
  * a captured decode graph be replayed token after token (the role of the
  * per-forward uniform patches, src/engine.ts:1487-1504). */

@@ -14,6 +14,7 @@ import pytest
 
 import oracle as O
 import synth
+from g4hip import G4Error
 from g4hip.decoder import BatchDecoder, E2BShape
 from gpu_util import assert_close
 
@@ -343,3 +344,40 @@ def test_prefill_attention_non_finite_rows(ctx, hd, window, bad):
         assert not np.isfinite(got[v][:, sorted(seen)]).any(), v
         want = O.attention_paged(q[v], kp, clean.view(np.uint16).reshape(-1), table, page, nq, 1, hd, n, 1.0, window)
         assert_close(got[v][:, ok], want.reshape(nq, hd)[:, ok], rel=4e-5, what=f"row {v}")
+
+
+@pytest.mark.parametrize("sample", ["argmax", "topk"])
+@pytest.mark.parametrize("B,T", [(64, 1), (64, 16), (64, 17), (64, 32), (64, 33), (20, 9), (20, 16), (20, 20)])
+def test_one_chunk_spare_rows_repeat_the_last_token(ctx, B, T, sample):
+    """The rows of a one-chunk prompt past its last token hold that token's residual row, logits and sample, also
+    where the step ran over 16 or 32 rows only; nothing of an earlier step is left in them."""
+    s = E2BShape(n_layers=1, global_layers=(), vocab=1024)
+    d = BatchDecoder(ctx, [0] * B, s, seed=33, reserve=2 * B + 40, shared_pages=True, embed=True)
+    for buf in (d.hidden, d.logits, d.topk):
+        buf.upload(np.full(buf.nbytes // 4, np.nan, np.float32))
+    d.tokens.upload(np.full(B, 4000000000, np.uint32))
+    toks = np.random.default_rng(T).integers(0, s.vocab, T).astype(np.uint32)
+    n = d.prefill(toks, 7, sample=sample)
+    assert n == T - 1
+    outs = [d.hidden.download(np.uint32).reshape(B, -1), d.logits.download(np.uint32).reshape(B, -1)]
+    if sample == "topk":
+        outs.append(d.topk.download(np.uint32).reshape(B, -1))
+        assert np.array_equal(d.tokens.download(np.uint32), np.concatenate([toks, np.repeat(toks[-1], B - T)]))
+    else:
+        outs.append(d.tokens.download(np.uint32).reshape(B, 1))
+    assert np.all(np.isfinite(outs[1].view(np.float32)))
+    for out in outs:
+        assert np.array_equal(out[n:], np.repeat(out[n:n + 1], B - n, axis=0))
+    assert np.array_equal(d.seq_lens.download(np.uint32), 8 + np.minimum(np.arange(B), T - 1))
+
+
+@pytest.mark.parametrize("words,src,first,count", [(1, 3, 4, 60), (255, 0, 1, 1), (257, 9, 0, 9), (1536, 15, 16, 48)])
+def test_repeat_row(ctx, words, src, first, count):
+    rows = max(src + 1, first + count) + 1
+    x = np.random.default_rng(words).integers(0, 2 ** 32, (rows, words), dtype=np.uint32)
+    d = ctx.from_numpy(x)
+    ctx.repeatRow(d, words, src, first, count)
+    x[first:first + count] = x[src]
+    assert np.array_equal(d.download(np.uint32).reshape(rows, words), x)
+    with pytest.raises(G4Error, match="repeatRow"):
+        ctx.repeatRow(d, words, first, first, count)
