@@ -58,7 +58,7 @@ BLOCK_BYTES = {"q4k": Q4K_BYTES, "q6k": Q6K_BYTES}
 # the layer matrices and their default formats (Q4_K, the down projection Q6_K)
 MATRICES = ("wq", "wk", "wv", "wo", "wgate", "wup", "wdown")
 # rows of a long prompt's pass through the layers (BatchDecoder.prefill): its
-# buffers take about 0.2 MB a row; past this the matmuls gain nothing
+# buffers take about 0.22 MB a row on the real layout and 160 MB for any
 WIDE_ROWS = 2048
 DEFAULT_TYPES = {"wq": "q4k", "wk": "q4k", "wv": "q4k", "wo": "q4k", "wgate": "q4k", "wup": "q4k", "wdown": "q6k"}
 
@@ -930,10 +930,12 @@ class BatchDecoder(_SyntheticModel):
                                   np.uint8)
         self.rope_cs = self._rope_tables(self.max_seq)
         # prompts longer than one chunk of B rows go through the layers this
-        # many rows at a time (0: B at a time)
+        # many rows at a time (0: B at a time); the buffers of such a pass come
+        # with the first prompt that takes one, for as many rows as it needs
         self.wide_rows = min(max(B, WIDE_ROWS // B * B), -(-self.max_seq // B) * B) if self._wide_prefill() else 0
-        if self.wide_rows:
-            self._build_wide()
+        self.wide, self.wide_cap = None, 0
+        # split-K partial sums of o and down: four chunks of a full pass, more of a short one
+        self.wide_parts = 4 * max(self.wide_rows, 512) * s.hidden
         ctx.fill_normal_f32(self.hidden, B * s.hidden, self._seed(), 0.0, 1.0)
         ctx.sync()
 
@@ -1217,18 +1219,25 @@ class BatchDecoder(_SyntheticModel):
                         and L.qt["wgate"] == L.qt["wup"] and "f16" not in (L.qt["wgate"], L.qt["wdown"])
                         for il, L in enumerate(self.layers)))
 
-    def _build_wide(self) -> None:
-        c, s, R, f32 = self.ctx, self.s, self.wide_rows, np.float32
-        H = s.hidden
-        ob = c.prefill_operand_bytes
-        w = self.wide = {
-            "hidden": c.empty(R * H, f32), "hidden2": c.empty(R * H, f32), "xops": c.empty(ob(H, R), np.uint8),
-            "q": c.empty(R * s.q_dim, f32), "k": c.empty(R * s.kv_dim, f32), "v": c.empty(R * s.kv_dim, f32),
-            "attn": c.empty(R * s.q_dim, f32), "aops": c.empty(ob(s.q_dim, R), np.uint8),
-            "fops": c.empty(ob(s.max_ffn, R), np.uint8)}
-        # split-K partial sums of o and down: four chunks of a full pass, more of a short one
-        self.wide_parts = 4 * max(R, 512) * H
-        w["parts"] = c.empty(self.wide_parts, f32)
+    def _wide_buffers(self, rows: int) -> None:
+        """Buffers of a pass over `rows` rows, kept for the prompts that follow; at least twice the rows (up to
+        wide_rows) where a longer prompt outgrows them, so that growing prompts replace them a few times only."""
+        if rows <= self.wide_cap:
+            return
+        R = min(max(rows, 2 * self.wide_cap), max(rows, self.wide_rows))
+        self.wide, self.wide_cap = None, 0  # (the old ones are given back first)
+        self.wide = self._build_wide(R)
+        self.wide_cap = R
+
+    def _build_wide(self, R: int) -> dict:
+        """The buffers by name, parts of one allocation: the first prompt waits for it (512 rows 0.8 ms;
+        twenty allocations 1.2 ms; 1900 rows 0.4 and 1.6)."""
+        c, s = self.ctx, self.s
+        H, LD = s.hidden, s.n_layers * s.ple_dim
+        ob, lo = c.prefill_operand_bytes, c.prefill_operand_lo_bytes
+        n = {"hidden": 4 * R * H, "hidden2": 4 * R * H, "xops": ob(H, R), "q": 4 * R * s.q_dim, "k": 4 * R * s.kv_dim,
+             "v": 4 * R * s.kv_dim, "attn": 4 * R * s.q_dim, "aops": ob(s.q_dim, R), "fops": ob(s.max_ffn, R),
+             "parts": 4 * self.wide_parts}
         need, ws = 0, 0
         for il, L in enumerate(self.layers):
             ws = max(ws, c.prefill_attn_workspace_bytes(c.paged_fused_params(
@@ -1236,32 +1245,37 @@ class BatchDecoder(_SyntheticModel):
                 0, s.eps, 1.0, 0)))
             Q, KV, I = s.q_dim_of(il), s.kv_dim_of(il), s.ffn_of(il)
             qkv = [("wq", Q)] + ([("wk", KV), ("wv", KV)] if s.is_producer(il) else [])
-            for ms, rows, n in [([m for m, _ in qkv], [r for _, r in qkv], H), (["wo"], [H], Q),
-                                (["wgate", "wup"], [I, I], H), (["wdown"], [H], I)]:
-                need = max([need] + [c.prefill_weight_bytes(L.qt[m], rows, n) for m in ms])
+            for ms, rows, width in [([m for m, _ in qkv], [r for _, r in qkv], H), (["wo"], [H], Q),
+                                    (["wgate", "wup"], [I, I], H), (["wdown"], [H], I)]:
+                need = max([need] + [c.prefill_weight_bytes(L.qt[m], rows, width) for m in ms])
         if s.ple_dim:
-            need = max(need, *(c.prefill_weight_bytes("f16", [rows], n) for rows, n in
-                               [(s.n_layers * s.ple_dim, H), (s.ple_dim, H), (H, s.ple_dim)]))
-        w["wops"] = c.empty(need, np.uint8)
-        w["attn_ws"] = c.empty(ws, np.uint8)
+            need = max(need, *(c.prefill_weight_bytes("f16", [rows], width) for rows, width in
+                               [(LD, H), (s.ple_dim, H), (H, s.ple_dim)]))
+        n.update(wops=need, attn_ws=ws)
         # f16 matrices take their vectors' third term too (f32's 24 bits, as in a step)
-        lo = c.prefill_operand_lo_bytes
         f16 = {m: any(L.qt[m] == "f16" for L in self.layers) for m in ("wq", "wk", "wv", "wo")}
         if s.ple_dim or f16["wq"] or f16["wk"] or f16["wv"]:
-            w["xops_lo"] = c.empty(lo(H, R), np.uint8)
+            n["xops_lo"] = lo(H, R)
         if f16["wo"]:
-            w["aops_lo"] = c.empty(lo(s.q_dim, R), np.uint8)
+            n["aops_lo"] = lo(s.q_dim, R)
         if s.ple_dim:
-            LD = s.n_layers * s.ple_dim
-            w["pops_lo"] = c.empty(lo(s.ple_dim, R), np.uint8)
-            w.update(hidden3=c.empty(R * H, f32), ple_projected=c.empty(R * LD, f32), ple_inputs=c.empty(R * LD, f32),
-                     ple_gate=c.empty(R * H, f32), pops=c.empty(ob(s.ple_dim, R), np.uint8), ple_out=c.empty(R * H, f32))
+            n.update(pops_lo=lo(s.ple_dim, R), hidden3=4 * R * H, ple_projected=4 * R * LD, ple_inputs=4 * R * LD,
+                     ple_gate=4 * R * H, pops=ob(s.ple_dim, R), ple_out=4 * R * H)
+        at = {}
+        total = 0
+        for name, size in n.items():
+            at[name] = total
+            total += -(-size // 256) * 256
+        w = {"all": c.alloc(total)}
+        w.update((name, Buffer(c, w["all"].ptr + at[name], n[name], owned=False)) for name in n)
+        return w
 
     def _prefill_wide(self, toks, start: int, pad: int, sample: str) -> None:
         """The prompt (its last token repeated `pad` times to whole chunks of
         B rows) up to wide_rows rows a pass, then the head over the last B."""
-        c, s, B, H, w = self.ctx, self.s, self.B, self.s.hidden, self.wide
         T = int(toks.size)
+        self._wide_buffers(min(self.wide_rows, T + pad))
+        c, s, B, H, w = self.ctx, self.s, self.B, self.s.hidden, self.wide
         ctok = np.concatenate([toks, np.repeat(toks[-1], pad)]).astype(np.uint32)
         clen = (np.concatenate([np.arange(T), np.repeat(T - 1, pad)]) + start + 1).astype(np.uint32)
         dtok, dlen = c.from_numpy(ctok), c.from_numpy(clen)

@@ -381,3 +381,29 @@ def test_repeat_row(ctx, words, src, first, count):
     assert np.array_equal(d.download(np.uint32).reshape(rows, words), x)
     with pytest.raises(G4Error, match="repeatRow"):
         ctx.repeatRow(d, words, first, first, count)
+
+
+def test_wide_buffers_come_with_the_first_long_prompt(ctx):
+    """A decoder whose prompts fit a chunk holds no buffers of a whole-prompt pass; a longer prompt brings them, a
+    longer one again replaces them, and what came before changes no result."""
+    B, s = 32, E2BShape.real(n_layers=3, n_unshared=2, global_layers=(1,), vocab=2048)
+
+    def decoder():
+        return BatchDecoder(ctx, [0] * B, s, seed=35, reserve=700, shared_pages=True, embed=True)
+
+    def prompt(d, T):
+        row = d.prefill(np.random.default_rng(T).integers(0, s.vocab, T).astype(np.uint32), 0)
+        return d.hidden.download(np.uint32), d.logits.download(np.uint32), d.tokens.download(np.uint32), row
+
+    d = decoder()
+    assert d.wide_rows == 704 and d.wide is None
+    prompt(d, 20)
+    prompt(d, 64)  # (two chunks of 32)
+    assert d.wide is None and d.wide_cap == 0
+    caps = []
+    for T in (70, 100, 333, 699, 70):
+        got = prompt(d, T)
+        caps.append(d.wide_cap)
+        for a, b in zip(got, prompt(decoder(), T)):
+            assert np.array_equal(a, b), T
+    assert caps == [96, 192, 384, 704, 704]
