@@ -858,12 +858,17 @@ void mm_launch_kg(g4_ctx* ctx, const MmArgs& a, uint32_t groups, bool unroll) {
 }
 
 // K groups per workgroup: the gate/up pair (one workgroup per CU, a whole K
-// each) takes two, but one where 64-vector operands let a CU hold two
-// single-group workgroups and the launch has more than one per CU (FFN 12288:
-// 384 workgroups, 38.2 -> 32.4 us: two groups' 140 KB leave one workgroup per
-// CU and the second half of the launch waits for the first); launches of about one workgroup per CU or fewer take
-// three where kc allows (a wave per SIMD leaves the latency of every MFMA
-// and operand read exposed; 12 waves share one CU's work three ways).
+// each) takes two, but one where copied 64-vector operands let a CU hold two
+// single-group workgroups and the launch has more than one per CU (two groups'
+// 140 KB leave one workgroup per CU and the second half of the launch waits for
+// the first). 64 vectors, weights from memory, two groups -> one: FFN 8448 x
+// 1536 32.2 -> 28.4 us, 12288 32.7 -> 29.3, 24576 52 -> 48.6; x 2048 43.6 ->
+// 35.0, 43.8 -> 38.1, 69.4 -> 65.7. Operands rebuilt from f32 keep two, where
+// the rebuilding, not the products, fills a workgroup's time: 12288 x 1536 62.1
+// against 77.3 with one, x 2048 84.2 against 104. Launches of about one
+// workgroup per CU or fewer take three where kc allows (a wave per SIMD leaves
+// the latency of every MFMA and operand read exposed; 12 waves share one CU's
+// work three ways).
 //
 // The unrolled walk holds a register set per block: it is taken by launches
 // of about one workgroup per CU or fewer (latency-bound), and with 64-vector
@@ -874,14 +879,16 @@ template <int QT, int BPR, int NTV, int MODE, int OPK>
 int mm_launch(g4_ctx* ctx, const MmArgs& a, uint32_t groups) {
   const uint32_t cus = (uint32_t)(ctx->num_cus > 0 ? ctx->num_cus : 256);
   // one tall Q6_K matrix (at least 16 tiles of 16 rows per CU: the LM head) and
-  // up to 32 vectors. 262144 x 1536 with the sampling launches: 8 vectors 133 ->
-  // 114 us, 32 176 -> 146. (Q4_K, whose blocks load in a third of the pieces:
-  // 97 -> 101 and 136 -> 132 us, so it keeps mmf_kernel.)
+  // up to 32 vectors. mmf_kernel -> the tall one, 8 and 32 vectors: 65536 x 1536
+  // 34.3 -> 29.7 and 45.6 -> 35.7 us, 262144 x 1536 114 -> 91.7 and 143 -> 112;
+  // 65536 x 2048 44.3 -> 29.1 and 62.8 -> 36.4, 262144 x 2048 152 -> 102 and 198
+  // -> 129. (Q4_K, whose blocks load in a third of the pieces, 262144 x 1536 with
+  // the sampling launches: 97 -> 101 and 136 -> 132, so it keeps mmf_kernel.)
   if constexpr (QT == 1 && MODE == 0 && OPK == 1 && NTV <= 2 && (BPR == 6 || BPR == 8))
     if (a.n == 1 && a.ksplit == 1 && groups >= 4 * cus)
       return g4_internal_tall_q6k(ctx, a.s[0].W, a.s[0].Y, a.s[0].M, a.K, a.ops, a.B, a.cap);
   const bool few = groups * a.ksplit <= cus;
-  if (MODE == 1 && a.kc % 2 == 0 && (NTV <= 2 || few)) {
+  if (MODE == 1 && a.kc % 2 == 0 && (NTV <= 2 || OPK == 0 || few)) {
     if constexpr (MODE == 1) mm_launch_kg<QT, BPR, NTV, MODE, OPK, 2>(ctx, a, groups, few);
   } else if (NTV <= 2 && few && a.kc % 3 == 0 && (a.kc == 3 || a.kc == 6)) {
     if constexpr (NTV <= 2) mm_launch_kg<QT, BPR, NTV, MODE, OPK, 3>(ctx, a, groups, true);

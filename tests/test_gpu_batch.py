@@ -147,7 +147,34 @@ def _decode_sub_operands(raw: np.ndarray, M: int, B: int) -> np.ndarray:
     return val.transpose(1, 4, 0, 2, 3, 5).reshape(16 * ntv, M)
 
 
-@pytest.mark.parametrize("B,M", [(5, 6144), (32, 6144), (64, 6144), (16, 12288)])
+@pytest.mark.parametrize("B,M,N", [(33, 12288, 1536), (64, 12288, 1536), (64, 8448, 2048)])
+@pytest.mark.parametrize("prebuilt", [False, True])
+def test_gate_up_more_workgroups_than_cus(ctx, B, M, N, prebuilt):
+    """gelu(gate) * up at 33-64 vectors where the launch has more workgroups than the chip CUs (one K group per
+    workgroup over copied operands, two over rebuilt ones), against float64 on rows at the ends and between."""
+    Wg, Wu = O.gen_q4k(115, M * N // 256), O.gen_q4k(116, M * N // 256)
+    X = O.gen_normal_f32(117, B * N, 0.0, 0.02).reshape(B, N)
+    xn, out = ctx.empty(B * N, np.float32), ctx.from_numpy(np.full(B * M, np.nan, np.float32))
+    ops = ctx.empty(ctx.batch_operand_bytes(N, B), np.uint8)
+    ctx.batchPrep(ctx.from_numpy(X), 1, None, None, None, None, xn, N, B, ops=ops)
+    ctx.gateUpGeluBatch(xn, ctx.from_numpy(Wg), ctx.from_numpy(Wu), out, M, N, B, ops=ops if prebuilt else None)
+    got = out.download(np.float32).reshape(B, M)
+    assert np.all(np.isfinite(got))
+    rows = np.unique(np.concatenate([np.arange(32), np.arange(M - 32, M),
+                                     np.random.default_rng(1).integers(0, M, 300)]))
+
+    def product(W):
+        w = O.np_dequant_q4k(W.reshape(M, -1)[rows].reshape(-1)).astype(np.float64).reshape(len(rows), N)
+        return X.astype(np.float64) @ w.T
+
+    a, u = product(Wg), product(Wu)
+    t = np.clip(0.7978845608028654 * a * (1 + 0.044715 * a * a), -15, 15)
+    want = 0.5 * a * (1 + np.tanh(t)) * u
+    for b in range(B):
+        assert_close(got[b, rows], want[b].astype(np.float32), what=f"vector {b}")
+
+
+@pytest.mark.parametrize("B,M", [(5, 6144), (32, 6144), (64, 6144), (16, 12288), (33, 12288), (64, 12288)])
 def test_ffn_handoff_operands(ctx, B, M):
     """The gate/up launch's product as sub-block-scaled operand blocks: the
     f32 product equals the plain launch's, the blocks hold it to 2^-19 of the
