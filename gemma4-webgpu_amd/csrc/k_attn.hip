@@ -1375,28 +1375,43 @@ int merge(g4_ctx* ctx, const AttnArgs& a, float* out, const SplitPlan& sp, uint3
 // 1 KV head x 256: 9.0 against 11.8 us at 512 positions, 11.2 against
 // 13.9 at 4096, 20.7 against 21.5 at 32768); in the decode step the fused
 // form (mqf_kernel) keeps the matrix cores.
-// Head dim 512 takes it for windows past 512 positions: below, the VALU form's
-// 32-position workgroups, several to a CU, are done sooner (ten layers, 15
-// sequences to 268 positions 714 against 722-739 us; 40 to 900: 1172 against
-// 1133, 64 to 4096: 1405 against 1330).
-bool mq_fits(uint32_t G, uint32_t hd, uint32_t num_seqs, uint32_t eff) {
-  return G == 8 && (hd == 256 || (hd == 512 && eff > 512)) && num_seqs <= 64;
+// Head dim 512 takes it for windows of at least 1024 positions in launches of
+// at least 64 positions per CU. Below either, the VALU form's 32-position
+// workgroups, several to a CU, are done before one of these (a CU holds one at
+// a time: 15 us and 4 us a step). us per call, VALU and this, sequences of 0.5 to 1
+// times the window (VALU first): 1-8 x 1024 15-18 and 19-20, 2 x 4096 18 and 22,
+// 8 x 640 17 and 20, 32 x 640 26 and 35; 32 x 1024 31 and 26, 8 x 2048 33 and
+// 22, 4 x 4096 26 and 26, 16 x 2048 54 and 25, 64 x 4096 247 and 129.
+bool mq_fits(const g4_ctx* ctx, uint32_t G, uint32_t hd, uint32_t num_seqs, uint32_t nkh, uint32_t eff) {
+  if (G != 8 || num_seqs > 64) return false;
+  const uint64_t cus = ctx->num_cus > 0 ? (uint64_t)ctx->num_cus : 256;
+  return hd == 256 || (hd == 512 && eff >= 1024 && (uint64_t)num_seqs * nkh * eff >= 64 * cus);
 }
 
 // Steps per workgroup from the largest window, sized for about four
 // workgroups per CU when every sequence is that long. At head dim 512 a CU
-// holds one workgroup at a time: sized for two where that is a step or two
-// (the live half of the windows then fits the chip once), four beyond, so
-// that the last round is short (64 sequences to 4096 positions, ten layers:
-// two, six and eight cost 41, 18 and 19 us more).
+// holds one workgroup at a time, and a round costs 11 us and 4 a step: one
+// round where three steps do that (32 x 1024 positions 37 us in two rounds of
+// one step, 25 in one of two; 8 x 4096 47 and 26; windows half as long 21 and
+// 24, 32 and 24), two where that is up to four (16 x 8192 106 us in four rounds
+// of two steps, 64 in two of four; 32 x 4096 84 and 63), four beyond, so that
+// the last round is short (64 sequences to 4096 positions, ten layers: two, six
+// and eight cost 41, 18 and 19 us more).
 template <int HD>
 int mq_decode(g4_ctx* ctx, const char* fn, const AttnArgs& base, uint32_t num_seqs, float* out, size_t ws_len,
               uint8_t* ops = nullptr) {
   const uint32_t eff = eff_len(base.cap, base.window);
   const uint64_t cus = ctx->num_cus > 0 ? (uint64_t)ctx->num_cus : 256;
   const uint64_t want = ((uint64_t)num_seqs * eff + 64 * 4 * cus - 1) / (64 * 4 * cus);
-  const uint64_t two = ((uint64_t)num_seqs * eff + 64 * 2 * cus - 1) / (64 * 2 * cus);
-  const uint32_t nstep = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(HD == 512 && two <= 2 ? two : want, 1), 16);
+  uint32_t nstep = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(want, 1), 16);
+  if constexpr (HD == 512) {
+    const uint64_t items = (uint64_t)num_seqs * base.nkh;
+    const uint64_t two = (items * eff + 64 * 2 * cus - 1) / (64 * 2 * cus);
+    uint32_t one = 1;
+    while (one <= 3 && items * ceil_div(eff, MQ_STEP * one) > cus) ++one;
+    if (one <= 3) nstep = one;
+    else if (two <= 4) nstep = (uint32_t)two;
+  }
   const uint32_t chunk = MQ_STEP * nstep;
   const uint32_t max_chunks = ceil_div(eff == 0 ? 1 : eff, chunk);
   const size_t need = ws_bytes(num_seqs, base.nkh, max_chunks, MQ_G, HD);
@@ -1860,7 +1875,8 @@ int g4_pagedAttnDecodeOps(g4_ctx* ctx, const float* q, const uint16_t* k_pool, c
   int rc = paged_setup(__func__, k_pool, v_pool, page_table, seq_lens, p, workspace, workspace_bytes, a, sp);
   if (rc) return rc;
   a.q = q;
-  if (mq_fits(p.num_q_heads / p.num_kv_heads, p.head_dim, p.num_seqs, eff_len(p.max_seq_len, p.sliding_window)))
+  if (mq_fits(ctx, p.num_q_heads / p.num_kv_heads, p.head_dim, p.num_seqs, p.num_kv_heads,
+              eff_len(p.max_seq_len, p.sliding_window)))
     return p.head_dim == 256 ? mq_decode<256>(ctx, __func__, a, p.num_seqs, output, workspace_bytes, (uint8_t*)ops)
                              : mq_decode<512>(ctx, __func__, a, p.num_seqs, output, workspace_bytes, (uint8_t*)ops);
   rc = launch_attn<true, false>(ctx, a, p.num_q_heads / p.num_kv_heads, p.head_dim, sp.cp,

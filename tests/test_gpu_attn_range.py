@@ -70,8 +70,8 @@ KINDS = ["sink", "large", "tiny", "left out"]
 
 @pytest.mark.parametrize("kind", KINDS)
 def test_paged_512(ctx, kind):
-    hd, B = 512, 3
-    lens = [L, 800, 705]
+    hd, B = 512, 16  # (fewer positions in all take the VALU form)
+    lens = [L, 800, 705, 900] * 4
     q, k, v = _inputs(kind, hd, B)
     per = -(-L // PAGE)
     order = np.random.default_rng(2).permutation(B * per).astype(np.int32).reshape(B, per)
