@@ -34,8 +34,6 @@
 //    matmul that follows, so that its workgroups copy them instead of each
 //    building them again (the LM head's 4096 workgroups read the same
 //    activations).
-#include <utility>
-
 #include "mm_operand.hpp"
 
 namespace {
@@ -400,14 +398,6 @@ struct OpSrc {
 
 using g4d::gelu_tanh;  // shaders/gelu_mul.wgsl:10-16
 
-__device__ __forceinline__ float epilogue(float y, float cap) {
-  if (cap > 0.f) {
-    const float t = fminf(fmaxf(y / cap, -15.0f), 15.0f);
-    return tanhf(t) * cap;
-  }
-  return y;
-}
-
 // Products of one super-block: the weights of this lane's 16-row tile in wr,
 // the block's operands in LDS at lds; acc[t] gains the tile's sums for
 // vectors 16t .. 16t + 15.
@@ -623,15 +613,6 @@ __device__ __forceinline__ void mm_epilogue(const MmArgs& a, f4 (&acc)[NTV], uin
         if (row + i < M) dst[i] = epilogue(acc[t][i], cap);
     }
   }
-}
-
-template <typename F, int... J>
-__device__ __forceinline__ void static_for_seq(F&& f, std::integer_sequence<int, J...>) {
-  (f(std::integral_constant<int, J>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_seq(f, std::make_integer_sequence<int, N>{});
 }
 
 // MODE 0: a row group is 64 rows of one segment. MODE 1 (gate/up): segments

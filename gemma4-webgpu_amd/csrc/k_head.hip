@@ -14,8 +14,6 @@
 // multiplied: one barrier per tile. A tile costs a wave 250 VALU instructions
 // (40 us of 262144 x 1536); the chain from barrier to barrier bounds it, above
 // the 64 us of its bytes.
-#include <utility>
-
 #include "mm_operand.hpp"
 
 namespace {
@@ -31,20 +29,6 @@ struct TallArgs {
   const uint8_t* ops;  // [NSB][Ops::bytes(NTV)]
 };
 
-__device__ __forceinline__ float epilogue(float y, float cap) {
-  if (cap > 0.f) return tanhf(fminf(fmaxf(y / cap, -15.0f), 15.0f)) * cap;
-  return y;
-}
-
-template <typename F, int... J>
-__device__ __forceinline__ void static_for_seq(F&& f, std::integer_sequence<int, J...>) {
-  (f(std::integral_constant<int, J>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_seq(f, std::make_integer_sequence<int, N>{});
-}
-
 template <int NSB, int NTV>
 struct Mlh {
   static constexpr uint32_t RB = NSB * Blk<1>::BYTES, TB = 16 * RB;  // bytes of a row, of a tile
@@ -59,21 +43,15 @@ struct Mlh {
 // 16 bytes per lane from src to LDS at dst + 16 lane, non-temporal. Written as
 // the instruction itself because the compiler, which knows the builtin's LDS
 // write, waits for every such load before any pair of LDS reads it merges
-// (read2 loses the object they belong to); the waits are wait_vmcnt and the
-// barrier below. (m0 takes the LDS address, with one wait state after its
-// write; the compiler keeps nothing in it.)
-__device__ __forceinline__ void to_lds(const void* src, uint8_t* dst) {
+// (read2 loses the object they belong to); the waits are the caller's
+// wait_vmcnt and lds_barrier. (m0 takes the LDS address, with one wait state
+// after its write. It is a reserved register, which the compiler sets at each
+// use of its own and never keeps a value in, so a clobber entry says nothing;
+// nothing else in this file's code uses it.)
+__device__ __forceinline__ void to_lds_unwaited(const void* src, uint8_t* dst) {
   const uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)dst);
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(src), "s"(at) : "memory");
 }
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt field");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-// (waits for no load in flight, unlike __syncthreads's fence)
-__device__ __forceinline__ void ring_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // A lane's row of a tile in LDS (blk: its block; sh: the block's offset within
 // its dword, uniform over the wave) as matrix-core weight registers.
 __device__ __forceinline__ WRegs<1> lds_weights(const uint8_t* blk, int q, uint32_t sh) {
@@ -122,7 +100,7 @@ __global__ __launch_bounds__(64 * NSB, NTV == 1 ? 3 : 2) void mlh_kernel(TallArg
 #pragma unroll
     for (int k = 0; k < P::PW; ++k) {
       const uint32_t pc = min((uint32_t)(w + k * NSB), (uint32_t)P::NP - 1u);
-      to_lds(src + min(pc * 1024u + l * 16u, P::TB - 16u), buf + pc * 1024u);
+      to_lds_unwaited(src + min(pc * 1024u + l * 16u, P::TB - 16u), buf + pc * 1024u);
     }
   };
   static_for<D - 1>([&](auto ic) { stage(decltype(ic)::value, ring[decltype(ic)::value]); });
@@ -166,7 +144,7 @@ __global__ __launch_bounds__(64 * NSB, NTV == 1 ? 3 : 2) void mlh_kernel(TallArg
       // tile i was requested D - 1 turns ago; D - 2 later tiles may be in flight
       // (a store among them makes the wait stricter)
       wait_vmcnt<P::PW*(D - 2)>();
-      ring_barrier();  // the tile is in LDS, the last one's partial sums are; its slot is free
+      lds_barrier();  // the tile is in LDS, the last one's partial sums are; its slot is free
       stage(i + D - 1, ring[(I + D - 1) % D]);
       __builtin_amdgcn_sched_barrier(0);
       if (i > 0) reduce(i - 1);
@@ -195,7 +173,7 @@ __global__ __launch_bounds__(64 * NSB, NTV == 1 ? 3 : 2) void mlh_kernel(TallArg
       }
     });
   wait_vmcnt<0>();  // no load into this workgroup's LDS outlives it
-  ring_barrier();
+  lds_barrier();
   reduce(n - 1);
 }
 

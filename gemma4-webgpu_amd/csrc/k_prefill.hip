@@ -137,13 +137,6 @@ constexpr uint32_t WAUX_LDS = 2048;  // a wave's row tiles' Aux values, likewise
 __device__ __forceinline__ void to_lds(const void* src, uint8_t* dst) {  // 16 bytes per lane, dst + 16 lane
   __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
 }
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-// Barrier after which LDS written before it (global -> LDS loads: by waves
-// that waited for them) is readable; waits for no load in flight.
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // MODE 0: row group g is row tiles 4 RT g .. +4 RT - 1 of the segments in
 // order, RT consecutive tiles per wave. MODE 1 (gate/up, RT 4): segments 0

@@ -1,8 +1,10 @@
 // mm_operand.hpp — Q4_K / Q6_K weight tiles as matrix-core A operands, shared
-// by the batched matmul (k_batch.hip) and the prefill matmul (k_prefill.hip):
-// the loads of one 16-row tile and super-block and their conversion to f16
+// by the batched matmuls (k_batch.hip, k_head.hip) and the prefill matmul
+// (k_prefill.hip): the loads of one 16-row tile and super-block and their conversion to f16
 // sc * q values in the v_mfma_f32_16x16x32_f16 operand order.
 #pragma once
+#include <utility>
+
 #include "g4_internal.hpp"
 
 namespace g4mm {
@@ -17,6 +19,36 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));  // native vector: s
 __device__ __forceinline__ uint32_t pack_h2(_Float16 a, _Float16 b) {
   h2 v = {a, b};
   return __builtin_bit_cast(uint32_t, v);
+}
+
+// f(0), f(1), ... f(N - 1), each index a compile-time constant.
+template <typename F, int... J>
+__device__ __forceinline__ void static_for_seq(F&& f, std::integer_sequence<int, J...>) {
+  (f(std::integral_constant<int, J>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_seq(f, std::make_integer_sequence<int, N>{});
+}
+
+// Waits until at most N of the wave's memory loads are in flight.
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+  static_assert(N >= 0 && N < 64, "vmcnt field");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+// Barrier after which LDS written before it (global -> LDS loads: by waves
+// that waited for them) is readable; waits for no load in flight, unlike
+// __syncthreads's fence.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// A logit's softcap (shaders/logit_softcap.wgsl), none for cap 0.
+__device__ __forceinline__ float epilogue(float y, float cap) {
+  if (cap > 0.f) {
+    const float t = fminf(fmaxf(y / cap, -15.0f), 15.0f);
+    return tanhf(t) * cap;
+  }
+  return y;
 }
 
 template <int QT>
