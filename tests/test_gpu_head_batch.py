@@ -1,6 +1,6 @@
 """GPU parity of the tall Q6_K matmul (the LM head over up to 32 vectors): rows
 at both ends and a sample of the others against a float64 product of the same
-dequantized weights, with whole and short last tiles of 16 rows, both widths,
+dequantized weights, every output finite and the same from call to call, with whole and short last tiles of 16 rows, both widths,
 vector counts on both sides of a 16-vector tile, and the softcap. The weight
 operand rounds sc * (q - 32) once to f16 (2^-12 at most, 1.4e-4 root mean
 square): 3e-4, of the products. Behind the softcap that holds while its slope
@@ -30,11 +30,19 @@ def test_tall_q6k_matmul(ctx, M, N, B, cap):
         X[B // 2] *= 30.0
     ops, xn, y = ctx.alloc(ctx.batch_operand_bytes(N, B)), ctx.zeros(B * N, np.float32), ctx.zeros(B * M, np.float32)
     ctx.batchPrep(ctx.from_numpy(X), 1, None, None, None, None, xn, N, B, ops=ops)
-    for _ in range(2):  # (a second call over the same buffers gives the same)
-        assert ctx.matmulSegmentsBatchPartial("q6k", xn, [ctx.from_numpy(b)], [y], [M], N, B, 1, ops=ops,
-                                              softcap=cap) == 1
-    got = y.download(np.float32).reshape(B, M)
+    at = 4 if M % 4 else 0  # (weights are 4-byte aligned)
+    buf = ctx.alloc(b.nbytes + at).upload(b, at)
+    w = buf.offset(at)
+
+    def call():
+        y.upload(np.full(B * M, np.nan, np.float32))
+        assert ctx.matmulSegmentsBatchPartial("q6k", xn, [w], [y], [M], N, B, 1, ops=ops, softcap=cap) == 1
+        return y.download(np.float32).reshape(B, M)
+
+    got = call()
     assert np.all(np.isfinite(got))
+    for _ in range(2):  # the sums' order is fixed: every output again, bit for bit
+        assert np.array_equal(call().view(np.uint32), got.view(np.uint32))
     rows = np.unique(np.concatenate([np.arange(40), np.arange(M - 40, M),
                                      np.random.default_rng(1).integers(0, M, 200)]))
     w = O.np_dequant_q6k(b.reshape(M, -1)[rows].reshape(-1)).astype(np.float64).reshape(len(rows), N)

@@ -17,7 +17,9 @@ prompt in chunks of 16 (the last one short), from position 0 and after 600
 cached positions (past the 512 window), on a local + global layer pair and
 on Gemma-4-E2B's layer kinds (head dim 512 globals, layers reading a
 producer's cache); and a 100-token prompt in the benchmark's 64-row chunks
-(one whole chunk, then a short one)."""
+(one whole chunk, then a short one). The probe keeps a prompt in chunks; each
+prompt then runs again without it, all rows in one pass, and its last token is
+held to the same oracle."""
 import numpy as np
 import pytest
 
@@ -99,4 +101,9 @@ def test_prefill_matches_sequential_forwards(ctx, kind, start, B, T):
                 assert_close(g, want, what=f"{nm} row {start + t} layer {il}")
                 worst = max(worst, O.rel_l2(g, want))
     print(f"[prefill] {kind} start {start}: worst K/V row rel-L2 {worst:.2e}", flush=True)
+    # the same prompt without the probe: one pass of all its rows
+    d.fill_kv(seed=32)
+    assert d.wide_rows >= T and d.prefill(toks, start) == last and d.wide is not None
+    assert_close(d.hidden.download(np.float32).reshape(B, s.hidden)[last], x, what="one pass: last token hidden")
+    assert_close(d.logits.download(np.float32).reshape(B, s.vocab)[last], lg, what="one pass: last token logits")
     del d

@@ -271,6 +271,45 @@ def test_wide_prefill_equals_chunks(ctx, layout, B, T, start):
             assert_close(a, b, what="cache")
 
 
+MIXES = {
+    "q6k": lambda il, m: "q6k",
+    "q4k": lambda il, m: "q4k",
+    "mixed": lambda il, m: {"wq": "q4k", "wk": "q6k", "wv": "q4k", "wo": "q6k", "wdown": "q4k"}.get(m, "q6k"),
+    "f16 q/k/v/o": lambda il, m: "f16" if m in ("wq", "wk", "wv", "wo") else "q4k" if m != "wdown" else "q6k",
+    "f16 v, o of layer 1": lambda il, m: "f16" if m == "wv" or (m == "wo" and il) else "q4k",
+}
+
+
+@pytest.mark.parametrize("mix,shape,B,T", [
+    ("q6k", {}, 64, 70), ("q4k", {}, 64, 129), ("mixed", {}, 16, 50), ("f16 q/k/v/o", {}, 64, 100),
+    ("f16 v, o of layer 1", {"real": True}, 64, 90), ("mixed", {"hidden": 2048}, 64, 140),
+    ("mixed", {"hidden": 2048, "real": True}, 32, 70),
+    ("q4k", {"n_layers": 1, "global_layers": ()}, 64, 2100),  # past the rows of one pass
+])
+def test_wide_prefill_formats_and_widths(ctx, mix, shape, B, T):
+    """A prompt in whole passes against its chunks, where the layers' formats differ, at the other hidden width, and
+    past the rows of one pass: its last token's residual row and logits, and the K/V rows."""
+    kw = dict(shape)
+    make = E2BShape.real if kw.pop("real", False) else E2BShape
+    s = make(**{"n_layers": 2, "global_layers": (1,), "vocab": 2048, **kw})
+    d = BatchDecoder(ctx, [0] * B, s, seed=37, reserve=T + 2 * B, shared_pages=True, embed=True, wtypes=MIXES[mix])
+    assert d.wide_rows >= B
+    toks = np.random.default_rng(4).integers(0, s.vocab, T).astype(np.uint32)
+
+    def go(**kw):
+        d.fill_kv(seed=38)
+        row = d.prefill(toks, 0, **kw)
+        return [row, d.hidden.download(np.float32).reshape(B, -1)[row],
+                d.logits.download(np.float32).reshape(B, -1)[row]] + [
+                    p.download(np.uint16).view(np.float16).astype(np.float32) for L in d.layers
+                    for p in (L.k_cache, L.v_cache)]
+
+    want, got = go(probe=lambda *a: None), go()
+    assert d.wide is not None and got[0] == want[0]
+    for a, b in zip(got[1:], want[1:]):
+        assert_close(a, b, what=f"{mix}, {T} tokens")
+
+
 def _attn_case(ctx, hd, T, start, window, n_kv=1, short_ws=False):
     """Rows at start .. start + T - 1 of one scattered page list against the oracle's paged attention."""
     page, nq = 16, 8 * n_kv
