@@ -9,9 +9,10 @@
 //  * unpack_kernel decodes a launch's matrices once into matrix-core operand
 //    order in a scratch buffer (f16 sc * q, the values k_batch.hip's waves
 //    form in registers; the f16 row d's and the Q4_K mins beside them). It
-//    costs one write and one read of 2 B per weight: 4-5 % of a 1900-token
-//    pass; decoding in the matmul instead would repeat per 64 tokens and take
-//    about as many VALU cycles as the products take matrix-core cycles.
+//    costs one write and one read of 2 B per weight: 7 % of a 1900-token
+//    pass, 13 % of a 512-token one; decoding in the matmul instead would
+//    repeat per 64 tokens and take about as many VALU cycles as the products
+//    take matrix-core cycles.
 //  * pf_gemm_kernel: a workgroup (4 waves) owns 64 RT rows (RT 16-row tiles
 //    per wave) x 64 vectors. The weight operands go from memory (L2) straight
 //    into registers, 1 KB contiguous per wave load; the activation operands

@@ -58,7 +58,9 @@ BLOCK_BYTES = {"q4k": Q4K_BYTES, "q6k": Q6K_BYTES}
 # the layer matrices and their default formats (Q4_K, the down projection Q6_K)
 MATRICES = ("wq", "wk", "wv", "wo", "wgate", "wup", "wdown")
 # rows of a long prompt's pass through the layers (BatchDecoder.prefill): its
-# buffers take about 0.22 MB a row on the real layout and 160 MB for any
+# buffers take about 0.22 MB a row on the real layout and 160 MB for any. More
+# rows still gain, for that memory: 4000 tokens over 20 layers 49.0 ms at 512
+# rows (0.22 GB), 34.7 at 1024, 28.1 at 2048 (0.55 GB), 23.4 at 4096 (1.0 GB)
 WIDE_ROWS = 2048
 DEFAULT_TYPES = {"wq": "q4k", "wk": "q4k", "wv": "q4k", "wo": "q4k", "wgate": "q4k", "wup": "q4k", "wdown": "q6k"}
 
