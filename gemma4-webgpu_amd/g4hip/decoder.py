@@ -1161,7 +1161,8 @@ class BatchDecoder(_SyntheticModel):
         full forward per prompt token instead (src/engine.ts:1923-1938) and
         samples from the last one (src/engine.ts:2014-2017); as there, only
         the last chunk runs the LM head. A prompt of more than two chunks
-        (of more than one past 32 rows) takes the layers up to `wide_rows` rows at a time instead, through the
+        (one past 32 rows each, three below 16 without per-layer embeddings)
+        takes the layers up to `wide_rows` rows at a time instead, through the
         prefill matmuls (each weight read and unpacked once per pass), and
         leaves the same rows as its last chunk would. A short last
         chunk repeats its last token and position in the spare rows
@@ -1183,8 +1184,11 @@ class BatchDecoder(_SyntheticModel):
         # (two chunks of at most 32 rows are as fast as one pass: 20 tokens by
         # 16 rows over ten layers 1.22 against 1.49 ms, 40 by 32 1.36 against
         # 1.53; three, or two of 64, are slower: 40 by 16 1.77 against 1.52, 70
-        # by 64 1.73 against 1.51)
-        if nch > (1 if B > 32 else 2) and self.wide_rows and probe is None:
+        # by 64 1.73 against 1.51. Of fewer than 16 rows, without per-layer
+        # embeddings, so are three: five uniform layers 11 by 5 0.91 against
+        # 0.95, 16 by 5 1.17 against 0.94; with them, ten layers 2.48 against 2.26)
+        few = 1 if B > 32 else 2 if B >= 16 or self.s.ple_dim else 3
+        if nch > few and self.wide_rows and probe is None:
             self._prefill_wide(toks, start, pad, sample)
             return n - 1
         # every chunk's tokens and lengths (before the step appends each row)

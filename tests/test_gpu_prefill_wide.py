@@ -235,7 +235,9 @@ def test_prefill_ple_gated(ctx, T, parts):
     ("uniform", 64, 300, 600),   # past the window
     ("real", 64, 131, 37),
     ("real", 7, 23, 0),          # odd chunks
-    ("uniform", 1, 3, 5),
+    ("uniform", 1, 3, 5),        # (three chunks of few rows stay chunks)
+    ("uniform", 1, 4, 5),
+    ("uniform", 5, 16, 40),
     ("uniform", 64, 9, 0),       # one chunk: 16 and 32 of its rows, and all
     ("real", 64, 27, 700),
     ("uniform", 64, 33, 0),
